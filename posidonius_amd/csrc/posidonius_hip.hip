@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "whfast_step.hpp"
+#include "whfast_fixed.hpp"
 #include "adjoint_kernels.hpp"
 
 #ifndef POS_WAVES_PER_EU
@@ -136,7 +137,7 @@ __device__ inline void load_lane(const DevEnsemble &E, WaveLds &lds, Lane &B, in
     for (int q = 0; q < 3; ++q) {
         sp[q] = E.spin[q * nb + b];
         lds.s[q][lane] = sp[q];
-        lds.ag[q][lane] = E.acc[q * nb + b];
+        lds.acc(q, lane) = E.acc[q * nb + b];
     }
     if (lane < NX) lds.xb[lane][WAVE] = 0.;   // the exchange area's zero column
     if (lane == 0) lds.m[WAVE] = 0.;
@@ -146,7 +147,7 @@ __device__ inline void load_lane(const DevEnsemble &E, WaveLds &lds, Lane &B, in
     __syncthreads();
 }
 
-__device__ inline void store_lane(const DevEnsemble &E, const WaveLds &lds, const Lane &B) {
+__device__ inline void store_lane(const DevEnsemble &E, WaveLds &lds, const Lane &B) {
     if (!B.valid()) return;
     // The indices pass through an empty asm so that the field addresses are
     // formed here again rather than kept from load_lane across the step loop
@@ -163,7 +164,7 @@ __device__ inline void store_lane(const DevEnsemble &E, const WaveLds &lds, cons
         E.spin[q * nb + b] = lds.s[q][lane];
         E.err_v[q * nb + b] = B.ev[q];
         E.err_L[q * nb + b] = B.eL[q];
-        E.acc[q * nb + b] = lds.ag[q][lane];
+        E.acc[q * nb + b] = lds.acc(q, lane);
     }
     E.radius[b] = lds.R[lane];
     E.inertia[b] = lds.I[lane];
@@ -204,9 +205,7 @@ void whfast_steps_kernel(DevEnsemble E, int n_steps, int wave_begin, int wave_en
     }
 }
 
-// The same K steps over waves [wave_begin, wave_end) of variant V (the
-// adjoint admits the generic Kidder variant and the fixed-effect-set one),
-// also writing the step tape of the adjoint (one row per step plus the final
+// The same K steps over waves [wave_begin, wave_end) of variant V, also writing the step tape of the adjoint (one row per step plus the final
 // state).
 template <int V>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(POS_WAVES_PER_EU)))
@@ -223,6 +222,27 @@ void whfast_record_kernel(DevEnsemble E, int n_steps, TapeRef T, int wave_begin,
             iterate<true, V>(E, lds, B, T, step);
         }
         store_lane(E, lds, B);
+        __syncthreads();
+    }
+}
+
+// K steps of waves [wave_begin, wave_end) of a fixed-effect-set variant by
+// teams of M wavefronts (whfast_fixed.hpp); with REC also the step tape.
+template <int M, bool REC, int V>
+__global__ __launch_bounds__(64 * M) __attribute__((amdgpu_waves_per_eu(POS_WAVES_PER_EU)))
+void whfast_fixed_kernel(DevEnsemble E, int n_steps, TapeRef T, int wave_begin, int wave_end) {
+    constexpr bool JACOBI = (V & VAR_JACOBI) != 0;
+    __shared__ FixedLds<M, JACOBI> lds;
+    // uniform over a wavefront, so that each one runs its own role's code
+    const int role = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    for (int wave = wave_begin + blockIdx.x; wave < wave_end; wave += gridDim.x) {
+        if (M == 1 || role == 0) fixed_run<M, 0, REC, JACOBI>(E, lds, wave, n_steps, T);
+        else if constexpr (M == 2) fixed_run<M, 1, REC, JACOBI>(E, lds, wave, n_steps, T);
+        else if constexpr (M == 4) {
+            if (role == 1) fixed_run<M, 1, REC, JACOBI>(E, lds, wave, n_steps, T);
+            else if (role == 2) fixed_run<M, 2, REC, JACOBI>(E, lds, wave, n_steps, T);
+            else fixed_run<M, 3, REC, JACOBI>(E, lds, wave, n_steps, T);
+        }
         __syncthreads();
     }
 }
@@ -280,7 +300,7 @@ __global__ __launch_bounds__(64) void gravity_kernel(DevEnsemble E, double *out_
     const int nb = E.n_bodies;
     if (B.valid()) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) out_acc[q * nb + B.body] = lds.ag[q][B.lane];
+        for (int q = 0; q < 3; ++q) out_acc[q * nb + B.body] = lds.acc(q, B.lane);
         if (B.k == 0) out_status[B.sys] = B.status;
     }
 }
@@ -294,8 +314,7 @@ __global__ __launch_bounds__(64) void effects_kernel(DevEnsemble E, double *out_
     Lane B;
     load_lane<V>(E, lds, B, wave);
     double a[3], dL[3];
-    PairGeo unused;
-    additional_effects<V>(E, lds, B, false, a, dL, unused);
+    additional_effects<V>(E, lds, B, false, a, dL);
     const int nb = E.n_bodies;
     if (B.valid()) {
 #pragma unroll
@@ -361,7 +380,7 @@ template <class T> struct DBuf {
 }  // namespace
 
 struct pos_ens {
-    int device = 0;
+    int device = 0, n_cus = 0;
     hipStream_t stream = nullptr;
     pos_options opts{};
     int n_systems = 0, n_bodies = 0;
@@ -864,6 +883,26 @@ template <int V> void launch_steps_variant(pos_ens *h, int grid, int n_steps, in
     hipLaunchKernelGGL(whfast_steps_kernel<V>, dim3(grid), dim3(64), 0, h->stream, h->E, n_steps, w0, w1);
 }
 
+// Wavefronts per team for a launch of `waves` wave-table entries.  A team of
+// four fits a CU twice at once (256 registers a lane), a team of two four
+// times, a single wavefront eight times; each is used as long as all its teams
+// run at once.  Per step of star + 2 planets systems on 256 CUs, teams of
+// 1 / 2 / 4: 23.4 / 16.2 / 15.1 us at 250 entries, 26.0 / 21.0 / 18.9 at 500,
+// 25.9 / 21.5 / 30.1 at 600, 27.0 / 24.1 / 36.0 at 1,000 and
+// 35.4 / 34.6 / 45.4, then 37.4 / 42.6 / 52.4 at 1,150 and 1,500.
+int team_size(const pos_ens *h, int waves) {
+    return waves <= 2 * h->n_cus ? 4 : waves <= 4 * h->n_cus ? 2 : 1;
+}
+
+template <bool REC, int V>
+void launch_fixed(pos_ens *h, const DevEnsemble &E, int grid, int n_steps, const TapeRef &T, int w0, int w1) {
+    switch (team_size(h, w1 - w0)) {
+        case 4: hipLaunchKernelGGL((whfast_fixed_kernel<4, REC, V>), dim3(grid), dim3(256), 0, h->stream, E, n_steps, T, w0, w1); break;
+        case 2: hipLaunchKernelGGL((whfast_fixed_kernel<2, REC, V>), dim3(grid), dim3(128), 0, h->stream, E, n_steps, T, w0, w1); break;
+        default: hipLaunchKernelGGL((whfast_fixed_kernel<1, REC, V>), dim3(grid), dim3(64), 0, h->stream, E, n_steps, T, w0, w1); break;
+    }
+}
+
 // One launch per kernel variant present; the persistent grid size caps each.
 // Returns the number of launches through *launches (optional).
 int launch_steps(pos_ens *h, int n_steps, int *launches = nullptr) {
@@ -880,8 +919,8 @@ int launch_steps(pos_ens *h, int n_steps, int *launches = nullptr) {
             case 4: launch_steps_variant<4>(h, grid, n_steps, w0, w1); break;
             case 5: launch_steps_variant<5>(h, grid, n_steps, w0, w1); break;
             case 6: launch_steps_variant<6>(h, grid, n_steps, w0, w1); break;
-            case 8: launch_steps_variant<8>(h, grid, n_steps, w0, w1); break;
-            case 24: launch_steps_variant<24>(h, grid, n_steps, w0, w1); break;
+            case 8: launch_fixed<false, 8>(h, h->E, grid, n_steps, TapeRef{nullptr, 0}, w0, w1); break;
+            case 24: launch_fixed<false, 24>(h, h->E, grid, n_steps, TapeRef{nullptr, 0}, w0, w1); break;
             default: return fail(POS_E_INVALID, "internal error: unknown kernel variant");
         }
         HIP_TRY(hipGetLastError());
@@ -981,6 +1020,10 @@ int32_t pos_create(const pos_ensemble_desc *d, const pos_options *opts, pos_ens 
 
     pos_ens *h = new pos_ens();
     h->device = o.device;
+    if (hipDeviceGetAttribute(&h->n_cus, hipDeviceAttributeMultiprocessorCount, o.device) != hipSuccess) {
+        delete h;
+        return fail(POS_E_HIP, "hipDeviceGetAttribute failed");
+    }
     if (hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking) != hipSuccess) {
         delete h;
         return fail(POS_E_HIP, "hipStreamCreate failed");
@@ -1837,11 +1880,9 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
             if (v == GRV_KIDDER)
                 hipLaunchKernelGGL(whfast_record_kernel<GRV_KIDDER>, grid, dim3(64), 0, h->stream, Er, seg_len(s), tape, w0, w1);
             else if (v == (GRV_KIDDER | VAR_FAST))
-                hipLaunchKernelGGL(whfast_record_kernel<GRV_KIDDER | VAR_FAST>, grid, dim3(64), 0, h->stream, Er, seg_len(s), tape,
-                                   w0, w1);
+                launch_fixed<true, GRV_KIDDER | VAR_FAST>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
             else if (v == (GRV_KIDDER | VAR_FAST | VAR_JACOBI))
-                hipLaunchKernelGGL(whfast_record_kernel<GRV_KIDDER | VAR_FAST | VAR_JACOBI>, grid, dim3(64), 0, h->stream, Er,
-                                   seg_len(s), tape, w0, w1);
+                launch_fixed<true, GRV_KIDDER | VAR_FAST | VAR_JACOBI>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
             else
                 return fail(POS_E_INVALID, "internal error: kernel variant without an adjoint");
             HIP_TRY(hipGetLastError());

@@ -28,6 +28,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "../../include/posidonius_hip.h"
 #include "crmath.hpp"
@@ -164,6 +165,12 @@ struct WaveLds {
     // the slots they skip.  The odd row stride also spreads the folds' reads
     // of one column in several rows over the LDS banks.
     double xb[NX][WAVE + 1];
+
+    static constexpr int COM_ROW = 6;      // rows of the centre-of-mass sums of inertial_to_alternative
+    static constexpr int HIST_V_ROW = 3;   // rows write_history_record exchanges velocities in (positions: 0-2)
+    __device__ __forceinline__ double &acc(int q, int lane) { return ag[q][lane]; }
+    __device__ __forceinline__ double sigma_of(const DevEnsemble &, int lane, int) const { return sigma[lane]; }
+    __device__ __forceinline__ double k2_of(const DevEnsemble &, int lane, int) const { return k2[lane]; }
 };
 
 // Every kernel that uses the exchange area runs one wavefront per workgroup
@@ -227,7 +234,8 @@ __device__ inline LaneGroup lane_group(const DevEnsemble &E, int wave, int lane)
 }
 
 // G m of the body in LDS slot l (the reference's mass_g = mass * K2)
-__device__ __forceinline__ double mg_of(const WaveLds &lds, int l) { return lds.m[l] * K2; }
+template <class Lds>
+__device__ __forceinline__ double mg_of(const Lds &lds, int l) { return lds.m[l] * K2; }
 
 // ---- per-lane registers -----------------------------------------------------
 enum : uint32_t {
@@ -383,7 +391,8 @@ enum {   // orbiting body -> host contributions
     C_COUNT = 24
 };
 
-__device__ __forceinline__ void put3(WaveLds &lds, int slot, int lane, double x, double y, double z) {
+template <class Lds>
+__device__ __forceinline__ void put3(Lds &lds, int slot, int lane, double x, double y, double z) {
     lds.xb[slot][lane] = x; lds.xb[slot + 1][lane] = y; lds.xb[slot + 2][lane] = z;
 }
 
@@ -403,8 +412,8 @@ __device__ __forceinline__ void put3(WaveLds &lds, int slot, int lane, double x,
 // flight cost registers.
 constexpr int FOLD_BATCH = 4;
 constexpr int REACTION_ROWS = 3;
-template <int R, bool SKIP_HOST, class Load>
-__device__ __forceinline__ void fold_rows(const Lane &B, double (&acc)[R], Load load) {
+template <int R, bool SKIP_HOST, class Body, class Load>
+__device__ __forceinline__ void fold_rows(const Body &B, double (&acc)[R], Load load) {
     for (int j0 = 0; j0 < B.n; j0 += FOLD_BATCH) {
         double t[R][FOLD_BATCH];
 #pragma unroll
@@ -502,7 +511,7 @@ __device__ __forceinline__ int chained_body(const Lane &B, int c) { return c == 
 __device__ inline void gr_newtonian(WaveLds &lds, Lane &B, double an[3]) {
     const int lane = B.lane, hl = B.hl();
 #pragma unroll
-    for (int q = 0; q < 3; ++q) an[q] = lds.ag[q][lane];
+    for (int q = 0; q < 3; ++q) an[q] = lds.acc(q, lane);
     // the ignored pairs: the first body after the host in chained order
     // (Jacobi) or every body (heliocentric splittings)
     const int np = B.coord == POS_COORD_JACOBI ? 1 : B.n - 1;
@@ -802,103 +811,15 @@ __device__ inline void disk_force(const DevEnsemble &E, const WaveLds &lds, cons
     F[2] = factor_migration * pv[2] + factor_eccentricity * sp * px[2] + factor_inclination * pv[2];
 }
 
-// Terms of an orbiting body's pair with its host that depend only on the
-// positions, masses, radii and fixed dissipation parameters.  Within one
-// implicit-midpoint solve the positions do not move, and in the fixed-effect-
-// set kernel (no evolution, no evolving dissipation) the radii and factors do
-// not change either, so these are evaluated once per solve instead of once
-// per iteration.  Each is the same rounded value the in-loop expression gives
-// (same operations in the same order), and a quotient by a hoisted divisor
-// uses its correctly rounded reciprocal (divr), which is exact.
-struct PairGeo {
-    double px[3];            // heliocentric position
-    Rcp Rd;                  // distance and its reciprocal
-    Rcp Rp8;                 // distance^8 and its reciprocal
-    double d5;               // distance^5
-    double os, op;           // tidal orthogonal components (constant_time_lag.rs:206-264)
-    double od, pd, id;       // os / d, op / d, 1 / d
-    double conservative;     // conservative radial tidal component (266-307)
-    double term1, term2;     // the two dissipative radial terms without their velocity factor
-    double m3d5, c15;        // -3 / d^5 and 15 / d^7 (oblate_spheroid.rs:51-60)
-    double mgc, mg_d;        // -(G m_h + G m) / (d^2 c^2) and (G m_h + G m) / d
-    double c1pn, o1pn;       // 1PN: 2 (2 + f) mg / d and (mg / (d^2 c^2)) 2 (2 - f)
-    double c2pn;             // 2PN: 3/4 (12 + 29 f) (mg^2 / d^2)
-    double n3[3];            // unit vector of the separation
-    // carried from one evaluation to the next: the scalar products of the
-    // separation with the host's and the body's spins of the previous
-    // evaluation (tides/common.rs:143-170, rotational_flattening/common.rs:93-120)
-    double rs_star, rs_planet;
-};
-
-// The pair geometry of this lane's body (orbiting lanes; zeros elsewhere),
-// with every lane's position exchanged through rows 0-2, and the scalar
-// products with the spins currently in LDS (those of the last evaluation).
-__device__ inline void pair_geometry(WaveLds &lds, const Lane &B, PairGeo &g) {
-    const int lane = B.lane;
-    const int hl = B.hl();
-    if (B.valid()) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
-    wsync();
-    double d = 1.;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) g.px[q] = 0.;
-    g.rs_star = 0.;
-    g.rs_planet = 0.;
-    if (B.orbiting()) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) g.px[q] = B.x[q] - lds.xb[q][hl];
-        d = sqrt(p2(g.px[0]) + p2(g.px[1]) + p2(g.px[2]));
-        g.rs_star = g.px[0] * lds.s[0][hl] + g.px[1] * lds.s[1][hl] + g.px[2] * lds.s[2][hl];
-        g.rs_planet = g.px[0] * lds.s[0][lane] + g.px[1] * lds.s[1][lane] + g.px[2] * lds.s[2][lane];
-    }
-    wsync();
-    const double m = B.m, hm = lds.m[hl];
-    const double hR = lds.R[hl], R = lds.R[lane];
-    g.Rd = rcp(d);
-    const double d7 = p7(d);
-    const Rcp Rd7 = rcp(d7);
-    g.d5 = p5(d);
-    g.Rp8 = rcp(p8(d));
-    const double sigma_host = lds.sigma[hl], sigma_pair = lds.sigma[lane];
-    g.os = divr(4.5 * p2(m) * p10(hR) * sigma_host, Rd7);
-    g.op = divr(4.5 * p2(hm) * p10(R) * sigma_pair, Rd7);
-    const double hm2 = hm * hm;
-    const double pm2 = m * m;
-    g.conservative = divr(-3.0 * K2, Rd7) * (pm2 * p5(hR) * lds.k2[hl] + hm2 * p5(R) * lds.k2[lane]);
-    g.term1 = pm2 * p10(hR) * sigma_host;
-    g.term2 = hm2 * p10(R) * sigma_pair;
-    g.od = divr(g.os, g.Rd);
-    g.pd = divr(g.op, g.Rd);
-    g.id = divr(1.0, g.Rd);
-    g.m3d5 = -3. / g.d5;
-    g.c15 = divr(15., Rd7);
-    const double hmg = mg_of(lds, hl), pmg = mg_of(lds, lane);
-    const double f = lds.kf[lane];
-    const double mg = hmg + pmg;
-    const double distance_2 = p2(d);
-    const Rcp Rdc = rcp(distance_2 * SPEED_OF_LIGHT_2);
-    g.mgc = divr(-mg, Rdc);
-    g.mg_d = divr(mg, g.Rd);
-    g.c1pn = divr(2.0 * (2.0 + f) * mg, g.Rd);
-    g.o1pn = divr(mg, Rdc) * 2.0 * (2.0 - f);
-    g.c2pn = 3.0 / 4.0 * (12.0 + 29.0 * f) * (p2(mg) / distance_2);
-#pragma unroll
-    for (int q = 0; q < 3; ++q) g.n3[q] = divr(g.px[q], g.Rd);
-}
-
 // Accelerations and spin derivatives of every body of the group at the current
 // (averaged) state.  Outputs are accumulated in the reference's order:
 // a_add = ((0 + tides) + flattening) + GR and
 // dL/dt = ((tides + flattening) + GR) + wind (universe.rs:540-614).
-// With H (the fixed-effect-set kernel inside an implicit-midpoint solve) the
-// pair terms come from geo, which pair_geometry filled at the start of the
-// solve, and the spins' scalar products are carried in geo from one
-// evaluation to the next; without H geo is not read.
-template <int V, bool H = false>
+template <int V>
 __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, Lane &B, bool evolution,
-                                          double a_add[3], double dLdt[3], PairGeo &geo) {
+                                          double a_add[3], double dLdt[3]) {
     constexpr int GRV = V & 3;
     constexpr bool EXT = (V & VAR_EXT) != 0;
-    static_assert(!H || ((V & VAR_FAST) != 0 && !EXT), "hoisted pair terms need fixed radii and factors");
     const LaneTests<V> LT(B);
     const int lane = B.lane;
     const int hl = B.hl();
@@ -906,51 +827,35 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
     // ---- inertial -> heliocentric (universe.rs:318-351); the host's
     //      heliocentric velocity is zero at this point ----
     if (B.valid()) {
-        if (!H) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
+        lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2];
         lds.xb[3][lane] = B.v[0]; lds.xb[4][lane] = B.v[1]; lds.xb[5][lane] = B.v[2];
     }
-    // With H the old spins are not read from LDS (their scalar products are
-    // carried), so the new spins are published in the same exchange as the
-    // velocities.
-    if (H) own_spin(lds, B);
     wsync();
     double px[3] = {0., 0., 0.}, pv[3] = {0., 0., 0.};
     double d = 1., nv2 = 0., nv = 1.;
     double rs_star = 0., rs_planet = 0.;
-    if (H) {
-#pragma unroll
-        for (int q = 0; q < 3; ++q) px[q] = geo.px[q];
-        d = geo.Rd.b;
-    }
     if (orbiting) {
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
-            if (!H) px[q] = B.x[q] - lds.xb[q][hl];
+            px[q] = B.x[q] - lds.xb[q][hl];
             pv[q] = B.v[q] - lds.xb[3 + q][hl];
         }
-        if (!H) d = sqrt(p2(px[0]) + p2(px[1]) + p2(px[2]));
+        d = sqrt(p2(px[0]) + p2(px[1]) + p2(px[2]));
         nv2 = p2(pv[0]) + p2(pv[1]) + p2(pv[2]);
         nv = sqrt(nv2);
         // Universe::initialize runs before the spins are refreshed
         // (universe.rs:429-430), so the scalar products of tides/common.rs:143-170
         // and rotational_flattening/common.rs:93-120 use the spins of the
         // previous evaluation.
-        if (H) {
-            rs_star = geo.rs_star;
-            rs_planet = geo.rs_planet;
-        } else {
-            rs_star = px[0] * lds.s[0][hl] + px[1] * lds.s[1][hl] + px[2] * lds.s[2][hl];
-            rs_planet = px[0] * lds.s[0][lane] + px[1] * lds.s[1][lane] + px[2] * lds.s[2][lane];
-        }
+        rs_star = px[0] * lds.s[0][hl] + px[1] * lds.s[1][hl] + px[2] * lds.s[2][hl];
+        rs_planet = px[0] * lds.s[0][lane] + px[1] * lds.s[1][lane] + px[2] * lds.s[2][lane];
     }
-    const Rcp Rd = H ? geo.Rd : rcp(d);
+    const Rcp Rd = rcp(d);
     const double vr = orbiting ? divr(px[0] * pv[0] + px[1] * pv[1] + px[2] * pv[2], Rd) : 0.;
-    if (!H) {
-        wsync();
-        // ---- evolution and spin = L / I (universe.rs:305-316) ----
-        if (evolution && (B.flags & F_EVOLUTION)) evolve_body(E, lds, B, B.t);
-        own_spin(lds, B);
-    }
+    wsync();
+    // ---- evolution and spin = L / I (universe.rs:305-316) ----
+    if (evolution && (B.flags & F_EVOLUTION)) evolve_body(E, lds, B, B.t);
+    own_spin(lds, B);
     double dk[3] = {0., 0., 0.};   // disk acceleration of this body
     double host_lag = 0.;
     if (EXT) {
@@ -968,7 +873,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
             lds.xb[3][lane] = B.is_host() ? E.lag[B.body] : ((B.flags & F_DISK_ROLE) ? 1. : 0.);
         }
     }
-    if (!H) wsync();
+    wsync();
     if (EXT) {
         if (B.valid() && B.is_host() && (B.flags & F_DISK)) {   // disk.rs:259-265, bodies in index order
             double sum[3] = {0., 0., 0.};
@@ -994,9 +899,9 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
         const double s[3] = {lds.s[0][lane], lds.s[1][lane], lds.s[2][lane]};
         const double hs2 = p2(hs[0]) + p2(hs[1]) + p2(hs[2]), s2 = p2(s[0]) + p2(s[1]) + p2(s[2]);
         const double hR = lds.R[hl], R = lds.R[lane];
-        const double d7 = H ? 0. : p7(d);
-        const Rcp Rd7 = H ? Rcp{0., 0.} : rcp(d7);
-        const double d5 = H ? geo.d5 : p5(d);
+        const double d7 = p7(d);
+        const Rcp Rd7 = rcp(d7);
+        const double d5 = p5(d);
         // ---- the dissipation factors of this host-body pair: the bodies' own
         //      scaled factors, or for evolving-dissipation models the pair
         //      values of a dynamical tide this orbit excites
@@ -1031,10 +936,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
         }
         // ---- tides: orthogonal components (constant_time_lag.rs:206-264) ----
         double os = 0., op = 0.;
-        if (H) {
-            os = geo.os;
-            op = geo.op;
-        } else if (LT.tides_role) {
+        if (LT.tides_role) {
             os = divr(4.5 * p2(m) * p10(hR) * sigma_host, Rd7);
             op = divr(4.5 * p2(hm) * p10(R) * sigma_pair, Rd7);
         }
@@ -1055,17 +957,16 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
             // radial component (constant_time_lag.rs:266-307)
             const double hm2 = hm * hm;
             const double pm2 = m * m;
-            const double conservative = H ? geo.conservative
-                                          : divr(-3.0 * K2, Rd7) * (pm2 * p5(hR) * lds.k2[hl] + hm2 * p5(R) * lds.k2[lane]);
-            const double factor1 = H ? divr(-13.5 * vr, geo.Rp8) : -13.5 * vr / p8(d);
-            const double term1 = H ? geo.term1 : pm2 * p10(hR) * sigma_host;
-            const double term2 = H ? geo.term2 : hm2 * p10(R) * sigma_pair;
+            const double conservative = divr(-3.0 * K2, Rd7) * (pm2 * p5(hR) * lds.k2[hl] + hm2 * p5(R) * lds.k2[lane]);
+            const double factor1 = -13.5 * vr / p8(d);
+            const double term1 = pm2 * p10(hR) * sigma_host;
+            const double term2 = hm2 * p10(R) * sigma_pair;
             const double diss_pm = factor1 * term2;
             const double dissipative = diss_pm + factor1 * term1;
             const double radial = conservative + dissipative;
             // force (constant_time_lag.rs:309-332)
             const double factor3 = radial + divr((os + op) * vr, Rd);
-            const double od = H ? geo.od : divr(os, Rd), pd = H ? geo.pd : divr(op, Rd);
+            const double od = divr(os, Rd), pd = divr(op, Rd);
             const double F0 = divr(factor3 * px[0], Rd) + od * (hs[1] * px[2] - hs[2] * px[1] - pv[0])
                             + pd * (s[1] * px[2] - s[2] * px[1] - pv[0]);
             const double F1 = divr(factor3 * px[1], Rd) + od * (hs[2] * px[0] - hs[0] * px[2] - pv[1])
@@ -1084,8 +985,8 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
         if (LT.rf && !LT.rf_role) put3(lds, C_RF, lane, 0., 0., 0.);
         if (LT.rf_role) {
             // radial component (oblate_spheroid.rs:51-60) and force (83-97)
-            const double radial = (H ? geo.m3d5 : -3. / d5) * (fp + fs)
-                + (H ? geo.c15 : divr(15., Rd7)) * (fs * rs_star * rs_star / hs2 + fp * rs_planet * rs_planet / s2);
+            const double radial = -3. / d5 * (fp + fs)
+                + divr(15., Rd7) * (fs * rs_star * rs_star / hs2 + fp * rs_planet * rs_planet / s2);
             const double F0 = radial * px[0] + ofp * s[0] + ofs * hs[0];
             const double F1 = radial * px[1] + ofp * s[1] + ofs * hs[1];
             const double F2 = radial * px[2] + ofp * s[2] + ofs * hs[2];
@@ -1112,7 +1013,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
                 const double cx = px[1] * pv[2] - px[2] * pv[1];
                 const double cy = px[2] * pv[0] - px[0] * pv[2];
                 const double cz = px[0] * pv[1] - px[1] * pv[0];
-                const double id = H ? geo.id : divr(1.0, Rd);
+                const double id = divr(1.0, Rd);
                 tdL[0] = -1.0 * (op * (d * s[0] - divr(rs_planet * px[0], Rd) - id * cx));
                 tdL[1] = -1.0 * (op * (d * s[1] - divr(rs_planet * px[1], Rd) - id * cy));
                 tdL[2] = -1.0 * (op * (d * s[2] - divr(rs_planet * px[2], Rd) - id * cz));
@@ -1147,17 +1048,17 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
             const double hmg = mg_of(lds, hl), pmg = mg_of(lds, lane);
             const double f = lds.kf[lane];
             const double mg = hmg + pmg;
-            const double distance_2 = H ? 0. : p2(d);
-            const Rcp Rdc = H ? Rcp{0., 0.} : rcp(distance_2 * SPEED_OF_LIGHT_2);
-            const double mgc = H ? geo.mgc : divr(-mg, Rdc);          // -mg / (d^2 c^2)
-            const double mg_d = H ? geo.mg_d : divr(mg, Rd);
+            const double distance_2 = p2(d);
+            const Rcp Rdc = rcp(distance_2 * SPEED_OF_LIGHT_2);
+            const double mgc = divr(-mg, Rdc);          // -mg / (d^2 c^2)
+            const double mg_d = divr(mg, Rd);
             const double mOverM = divr(m, Rhm);
             const Rcp Rnv = rcp(nv);
             double gr[3];
             {   // 1PN
                 const double radial_velocity_2 = p2(vr);
-                const double radial = mgc * ((1.0 + 3.0 * f) * nv2 - (H ? geo.c1pn : divr(2.0 * (2.0 + f) * mg, Rd)) - 1.5 * f * radial_velocity_2);
-                const double orthogonal = (H ? geo.o1pn : divr(mg, Rdc) * 2.0 * (2.0 - f)) * vr * nv;
+                const double radial = mgc * ((1.0 + 3.0 * f) * nv2 - divr(2.0 * (2.0 + f) * mg, Rd) - 1.5 * f * radial_velocity_2);
+                const double orthogonal = divr(mg, Rdc) * 2.0 * (2.0 - f) * vr * nv;
 #pragma unroll
                 for (int q = 0; q < 3; ++q) gr[q] = divr(radial * px[q], Rd) + divr(orthogonal * pv[q], Rnv);
                 put3(lds, C_G1, lane, mOverM * gr[0], mOverM * gr[1], mOverM * gr[2]);
@@ -1168,7 +1069,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
                 const double vr4 = p2(vr2);
                 const double f2 = p2(f);
                 const double radial = mgc
-                    * ((H ? geo.c2pn : 3.0 / 4.0 * (12.0 + 29.0 * f) * (p2(mg) / distance_2))
+                    * (3.0 / 4.0 * (12.0 + 29.0 * f) * (p2(mg) / distance_2)
                        + f * (3.0 - 4.0 * f) * nv4
                        + 15.0 / 8.0 * f * (1.0 - 3.0 * f) * vr4
                        - 3.0 / 2.0 * f * (3.0 - 4.0 * f) * vr2 * nv2
@@ -1193,8 +1094,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
                 const Rcp RM{M, lds.inv_M[lane]};
                 const double mass_factor = divr(hm - m, RM);
                 const double Lp[3] = {I * s[0], I * s[1], I * s[2]};
-                const double n3[3] = {H ? geo.n3[0] : divr(px[0], Rd), H ? geo.n3[1] : divr(px[1], Rd),
-                                      H ? geo.n3[2] : divr(px[2], Rd)};
+                const double n3[3] = {divr(px[0], Rd), divr(px[1], Rd), divr(px[2], Rd)};
                 const double factor_a = G / SPEED_OF_LIGHT_2;
                 double a[3];
                 {
@@ -1235,10 +1135,6 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
         } else {
 #pragma unroll
             for (int q = 0; q < 3; ++q) dLdt[q] = dLdt[q] + 0.;
-        }
-        if (H) {   // for the next evaluation, whose spins are refreshed before it reads them
-            geo.rs_star = px[0] * hs[0] + px[1] * hs[1] + px[2] * hs[2];
-            geo.rs_planet = px[0] * s[0] + px[1] * s[1] + px[2] * s[2];
         }
     }
     wsync();
@@ -1319,13 +1215,10 @@ __device__ inline void integrate_velocity_dependent_forces(const DevEnsemble &E,
     double v_orig[3], L_orig[3], dv[3] = {0., 0., 0.}, dL[3] = {0., 0., 0.};
 #pragma unroll
     for (int q = 0; q < 3; ++q) { v_orig[q] = B.v[q]; L_orig[q] = B.L[q]; }
-    constexpr bool H = (V & VAR_FAST) != 0;   // fixed radii and factors: hoist the pair terms
-    PairGeo geo;
-    if (H) pair_geometry(lds, B, geo);
     bool converged = false;
     for (int it = 0; it < MIDPOINT_MAX_ITER; ++it) {
         double a_add[3], dLdt[3];
-        additional_effects<V, H>(E, lds, B, evolution && it == 0, a_add, dLdt, geo);
+        additional_effects<V>(E, lds, B, evolution && it == 0, a_add, dLdt);
         double pdv = 0., pdL = 0.;   // |change of the final state|^2 of this body
         double fv2 = 0., fL2 = 0.;   // |final state|^2 of this body
 #pragma unroll
@@ -1525,7 +1418,8 @@ __device__ inline void kepler_individual_step(Lane &B, double mass_g, double dt)
 
 // Jacobi prefix sums up to body k (whfast.rs:574-576, 642-651): the
 // cumulative G-mass and mass of the host and the bodies before k, k included.
-__device__ inline void jacobi_prefix(const WaveLds &lds, const Lane &B, double *mu, double *eta, int *rank) {
+template <class Lds>
+__device__ inline void jacobi_prefix(const Lds &lds, const Lane &B, double *mu, double *eta, int *rank) {
     const int hl = B.hl();
     double m_g = mg_of(lds, hl), e = lds.m[hl];
     int r = 0;
@@ -1539,7 +1433,8 @@ __device__ inline void jacobi_prefix(const WaveLds &lds, const Lane &B, double *
     *mu = m_g; *eta = e; *rank = r;
 }
 
-__device__ inline void kepler_steps(const WaveLds &lds, Lane &B, double dt) {
+template <class Lds>
+__device__ inline void kepler_steps(const Lds &lds, Lane &B, double dt) {
     if (B.orbiting()) {
         double mu;
         if (B.coord == POS_COORD_JACOBI) {
@@ -1562,7 +1457,8 @@ __device__ inline void kepler_steps(const WaveLds &lds, Lane &B, double dt) {
 // ===========================================================================
 // Coordinate transforms, jump and interaction (whfast.rs:495-625, 881-1155)
 // ===========================================================================
-__device__ inline void inertial_to_alternative(WaveLds &lds, Lane &B) {
+template <class Lds>
+__device__ inline void inertial_to_alternative(Lds &lds, Lane &B) {
     const int lane = B.lane;
     if (B.valid()) {
         lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2];
@@ -1607,19 +1503,20 @@ __device__ inline void inertial_to_alternative(WaveLds &lds, Lane &B) {
         // whfast.rs:973-1023: centre of mass, host first then the others in
         // order; the seven ordered sums (x, v weighted by the masses, and the
         // masses themselves as 1 * m from row 13) are spread over the group's
-        // lanes and left in rows 6-12 of column gbase
+        // lanes and left in rows COM_ROW.. of column gbase
         if (B.valid()) lds.xb[13][lane] = 1.;
         wsync();
         for (int q = B.k; B.valid() && q < 7; q += B.n) {
             const int rq = q < 6 ? q : 13;
             double acc[1] = {0. + lds.xb[rq][hl] * lds.m[hl]};
             fold_rows<1, true>(B, acc, [&](int, int l) { return lds.xb[rq][l] * lds.m[l]; });
-            lds.xb[6 + q][B.gbase] = acc[0];
+            lds.xb[Lds::COM_ROW + q][B.gbase] = acc[0];
         }
         wsync();
-        const double cx[3] = {lds.xb[6][B.gbase], lds.xb[7][B.gbase], lds.xb[8][B.gbase]};
-        const double cv[3] = {lds.xb[9][B.gbase], lds.xb[10][B.gbase], lds.xb[11][B.gbase]};
-        const double cm = lds.xb[12][B.gbase];
+        constexpr int R = Lds::COM_ROW;
+        const double cx[3] = {lds.xb[R][B.gbase], lds.xb[R + 1][B.gbase], lds.xb[R + 2][B.gbase]};
+        const double cv[3] = {lds.xb[R + 3][B.gbase], lds.xb[R + 4][B.gbase], lds.xb[R + 5][B.gbase]};
+        const double cm = lds.xb[R + 6][B.gbase];
         B.com_m = cm;
         const Rcp Rcm = rcp(cm);
 #pragma unroll
@@ -1641,7 +1538,8 @@ __device__ inline void inertial_to_alternative(WaveLds &lds, Lane &B) {
     wsync();
 }
 
-__device__ inline void jump_step(WaveLds &lds, Lane &B, double dt) {
+template <class Lds>
+__device__ inline void jump_step(Lds &lds, Lane &B, double dt) {
     if (B.coord == POS_COORD_JACOBI) return;
     const int lane = B.lane;
     if (B.orbiting()) {
@@ -1679,7 +1577,8 @@ __device__ inline void jump_step(WaveLds &lds, Lane &B, double dt) {
     }
 }
 
-__device__ inline void interaction_step(WaveLds &lds, Lane &B, double dt) {
+template <class Lds>
+__device__ inline void interaction_step(Lds &lds, Lane &B, double dt) {
     const int lane = B.lane;
     const int hl = B.hl();
     if (B.coord == POS_COORD_JACOBI) {
@@ -1688,7 +1587,7 @@ __device__ inline void interaction_step(WaveLds &lds, Lane &B, double dt) {
         double eta = lds.m[hl];
         double s[3], aj_own[3] = {0., 0., 0.};
 #pragma unroll
-        for (int q = 0; q < 3; ++q) s[q] = eta * lds.ag[q][hl];
+        for (int q = 0; q < 3; ++q) s[q] = eta * lds.acc(q, hl);
         for (int j = 0; j < B.n; ++j) {
             if (j == B.host) continue;
             const int l = B.gbase + j;
@@ -1698,7 +1597,7 @@ __device__ inline void interaction_step(WaveLds &lds, Lane &B, double dt) {
             const double pme = eta * ei;
             double aj[3];
 #pragma unroll
-            for (int q = 0; q < 3; ++q) aj[q] = lds.ag[q][l] - s[q] * ei;
+            for (int q = 0; q < 3; ++q) aj[q] = lds.acc(q, l) - s[q] * ei;
             if (j == B.k) {
 #pragma unroll
                 for (int q = 0; q < 3; ++q) aj_own[q] = aj[q];
@@ -1726,18 +1625,19 @@ __device__ inline void interaction_step(WaveLds &lds, Lane &B, double dt) {
     if (B.orbiting()) {
         if (B.coord == POS_COORD_DEMOCRATIC_HELIOCENTRIC) {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + dt * lds.ag[q][lane];
+            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + dt * lds.acc(q, lane);
         } else {
             const double hm = lds.m[hl];
             const double factor = hm + B.m;
             const Rcp Rhm{hm, lds.inv_m[hl]};
 #pragma unroll
-            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + divr(dt * factor * lds.ag[q][lane], Rhm);
+            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + divr(dt * factor * lds.acc(q, lane), Rhm);
         }
     }
 }
 
-__device__ inline void alternative_to_inertial(WaveLds &lds, Lane &B) {
+template <class Lds>
+__device__ inline void alternative_to_inertial(Lds &lds, Lane &B) {
     const int lane = B.lane;
     if (B.orbiting()) {
         lds.xb[0][lane] = B.ax[0]; lds.xb[1][lane] = B.ax[1]; lds.xb[2][lane] = B.ax[2];
@@ -1826,7 +1726,8 @@ __device__ inline void alternative_to_inertial(WaveLds &lds, Lane &B) {
 // ===========================================================================
 // Newtonian gravity (universe.rs:198-303)
 // ===========================================================================
-__device__ inline void gravity(const DevEnsemble &E, WaveLds &lds, Lane &B) {
+template <class Lds>
+__device__ inline void gravity(const DevEnsemble &E, Lds &lds, Lane &B) {
     const int lane = B.lane;
     if (B.valid()) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
     wsync();
@@ -1861,7 +1762,7 @@ __device__ inline void gravity(const DevEnsemble &E, WaveLds &lds, Lane &B) {
             acc[1] = acc[1] + prefact * dy;
             acc[2] = acc[2] + prefact * dz;
         }
-        lds.ag[0][lane] = acc[0]; lds.ag[1][lane] = acc[1]; lds.ag[2][lane] = acc[2];
+        lds.acc(0, lane) = acc[0]; lds.acc(1, lane) = acc[1]; lds.acc(2, lane) = acc[2];
     }
     wsync();
 }
@@ -1872,7 +1773,8 @@ __device__ inline void gravity(const DevEnsemble &E, WaveLds &lds, Lane &B) {
 // active lane of the wavefront holds a status or count other than the one
 // its group agreed on last (a wavefront-wide vote), every lane already holds
 // the group's OR and maximum, and the exchange is skipped.
-__device__ inline void merge_status(WaveLds &lds, Lane &B) {
+template <class Lds>
+__device__ inline void merge_status(Lds &lds, Lane &B) {
     if (!__any(B.status != B.seen_status || B.tw != B.seen_tw)) return;
     lds.xb[0][B.lane] = __builtin_bit_cast(double, (unsigned long long)B.status);
     lds.xb[1][B.lane] = (double)B.tw;
@@ -1897,12 +1799,13 @@ __device__ inline void merge_status(WaveLds &lds, Lane &B) {
 // state: the reference evaluates it from the tidal internals of the last
 // effects evaluation of the previous step, half a step earlier.
 // ===========================================================================
-template <bool EXT>
-__device__ inline void write_history_record(const DevEnsemble &E, WaveLds &lds, Lane &B) {
+template <bool EXT, class Lds>
+__device__ inline void write_history_record(const DevEnsemble &E, Lds &lds, Lane &B) {
+    constexpr int VR = Lds::HIST_V_ROW;
     const int lane = B.lane;
     if (B.valid()) {
         lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2];
-        lds.xb[3][lane] = B.v[0]; lds.xb[4][lane] = B.v[1]; lds.xb[5][lane] = B.v[2];
+        lds.xb[VR][lane] = B.v[0]; lds.xb[VR + 1][lane] = B.v[1]; lds.xb[VR + 2][lane] = B.v[2];
     }
     wsync();
     double dedt = 0.;   // a body the tidal loops skip keeps its initial 0 (tides/common.rs:263-281)
@@ -1910,12 +1813,12 @@ __device__ inline void write_history_record(const DevEnsemble &E, WaveLds &lds, 
         const int hl = B.hl();
         double r[3], u[3];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) { r[q] = B.x[q] - lds.xb[q][hl]; u[q] = B.v[q] - lds.xb[3 + q][hl]; }
+        for (int q = 0; q < 3; ++q) { r[q] = B.x[q] - lds.xb[q][hl]; u[q] = B.v[q] - lds.xb[VR + q][hl]; }
         const double d = sqrt(p2(r[0]) + p2(r[1]) + p2(r[2]));
         const double vr = (r[0] * u[0] + r[1] * u[1] + r[2] * u[2]) / d;
         const double hm = lds.m[hl];
         const double R = lds.R[lane];
-        double sigma = lds.sigma[lane];   // or its pair-dependent map entry
+        double sigma = lds.sigma_of(E, lane, B.body);   // or its pair-dependent map entry
         if (EXT && (B.flags & F_DYN) && E.pair_ph[B.body] == E.pair_ph[B.body]) sigma = E.pair_ph[B.body];
         const double op = 4.5 * p2(hm) * p10(R) * sigma / p7(d);
         const double diss_pm = -13.5 * vr / p8(d) * (p2(hm) * p10(R) * sigma);
@@ -1950,7 +1853,7 @@ __device__ inline void write_history_record(const DevEnsemble &E, WaveLds &lds, 
         }
         rec[HF_RADIUS * nb] = lds.R[lane];
         rec[HF_RG2 * nb] = E.rg2[B.body];
-        rec[HF_LOVE * nb] = lds.k2[lane];
+        rec[HF_LOVE * nb] = lds.k2_of(E, lane, B.body);
         rec[HF_DEDT * nb] = dedt;
         rec[HF_LAG * nb] = EXT ? E.lag[B.body] : 0.;
         rec[HF_MIGRATION * nb] = EXT ? E.disk_migration[B.body] : 0.;
