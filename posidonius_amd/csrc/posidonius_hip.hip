@@ -137,7 +137,7 @@ __device__ inline void load_lane(const DevEnsemble &E, WaveLds &lds, Lane &B, in
     for (int q = 0; q < 3; ++q) {
         sp[q] = E.spin[q * nb + b];
         lds.s[q][lane] = sp[q];
-        lds.acc(q, lane) = E.acc[q * nb + b];
+        lds.ag[q][lane] = E.acc[q * nb + b];
     }
     if (lane < NX) lds.xb[lane][WAVE] = 0.;   // the exchange area's zero column
     if (lane == 0) lds.m[WAVE] = 0.;
@@ -147,7 +147,7 @@ __device__ inline void load_lane(const DevEnsemble &E, WaveLds &lds, Lane &B, in
     __syncthreads();
 }
 
-__device__ inline void store_lane(const DevEnsemble &E, WaveLds &lds, const Lane &B) {
+__device__ inline void store_lane(const DevEnsemble &E, const WaveLds &lds, const Lane &B) {
     if (!B.valid()) return;
     // The indices pass through an empty asm so that the field addresses are
     // formed here again rather than kept from load_lane across the step loop
@@ -164,7 +164,7 @@ __device__ inline void store_lane(const DevEnsemble &E, WaveLds &lds, const Lane
         E.spin[q * nb + b] = lds.s[q][lane];
         E.err_v[q * nb + b] = B.ev[q];
         E.err_L[q * nb + b] = B.eL[q];
-        E.acc[q * nb + b] = lds.acc(q, lane);
+        E.acc[q * nb + b] = lds.ag[q][lane];
     }
     E.radius[b] = lds.R[lane];
     E.inertia[b] = lds.I[lane];
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(64) void gravity_kernel(DevEnsemble E, double *out_
     const int nb = E.n_bodies;
     if (B.valid()) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) out_acc[q * nb + B.body] = lds.acc(q, B.lane);
+        for (int q = 0; q < 3; ++q) out_acc[q * nb + B.body] = lds.ag[q][B.lane];
         if (B.k == 0) out_status[B.sys] = B.status;
     }
 }

@@ -166,9 +166,9 @@ struct WaveLds {
     // of one column in several rows over the LDS banks.
     double xb[NX][WAVE + 1];
 
-    static constexpr int COM_ROW = 6;      // rows of the centre-of-mass sums of inertial_to_alternative
-    static constexpr int HIST_V_ROW = 3;   // rows write_history_record exchanges velocities in (positions: 0-2)
-    __device__ __forceinline__ double &acc(int q, int lane) { return ag[q][lane]; }
+    // rows write_history_record exchanges positions and velocities in
+    static constexpr __device__ int hist_x_row(int q) { return q; }
+    static constexpr __device__ int hist_v_row(int q) { return 3 + q; }
     __device__ __forceinline__ double sigma_of(const DevEnsemble &, int lane, int) const { return sigma[lane]; }
     __device__ __forceinline__ double k2_of(const DevEnsemble &, int lane, int) const { return k2[lane]; }
 };
@@ -412,8 +412,8 @@ __device__ __forceinline__ void put3(Lds &lds, int slot, int lane, double x, dou
 // flight cost registers.
 constexpr int FOLD_BATCH = 4;
 constexpr int REACTION_ROWS = 3;
-template <int R, bool SKIP_HOST, class Body, class Load>
-__device__ __forceinline__ void fold_rows(const Body &B, double (&acc)[R], Load load) {
+template <int R, bool SKIP_HOST, class Load>
+__device__ __forceinline__ void fold_rows(const Lane &B, double (&acc)[R], Load load) {
     for (int j0 = 0; j0 < B.n; j0 += FOLD_BATCH) {
         double t[R][FOLD_BATCH];
 #pragma unroll
@@ -511,7 +511,7 @@ __device__ __forceinline__ int chained_body(const Lane &B, int c) { return c == 
 __device__ inline void gr_newtonian(WaveLds &lds, Lane &B, double an[3]) {
     const int lane = B.lane, hl = B.hl();
 #pragma unroll
-    for (int q = 0; q < 3; ++q) an[q] = lds.acc(q, lane);
+    for (int q = 0; q < 3; ++q) an[q] = lds.ag[q][lane];
     // the ignored pairs: the first body after the host in chained order
     // (Jacobi) or every body (heliocentric splittings)
     const int np = B.coord == POS_COORD_JACOBI ? 1 : B.n - 1;
@@ -1320,22 +1320,31 @@ __device__ inline void kepler_individual_step(Lane &B, double mass_g, double dt)
     const double eta0 = x0[0] * v0[0] + x0[1] * v0[1] + x0[2] * v0[2];
     const double zeta0 = mass_g - beta * r0;
     double x, gs[4];
-    double invperiod = 0.;
-    double x_per_period;
     const bool elliptic = beta > 0.;
-    if (elliptic) {
+    // The orbital frequency and the anomaly per period enter two rare
+    // decisions (a step longer than an orbit; a first correction of more than
+    // 1% of a period) and the bisection.  Their square root and quotients are
+    // formed only when a product of the squares, off by some ulps at most,
+    // cannot exclude the decision with 1% to spare.
+    auto orbit = [&](double &invperiod, double &x_per_period) {
         const double sqrt_beta = sqrt(beta);
         invperiod = sqrt_beta * beta / (2. * PI * mass_g);
         x_per_period = (2. * PI) / sqrt_beta;
-        if (fabs(dt) * invperiod > 1. && B.tw == 0) {
-            B.status |= POS_STATUS_TIMESTEP_WARNING;
-            B.tw += 1;
+    };
+    if (elliptic) {
+        const double mu2 = 2. * PI * mass_g;
+        if (!(dt * dt * beta * beta * beta <= 0.98 * (mu2 * mu2))) {
+            double invperiod, x_per_period;
+            orbit(invperiod, x_per_period);
+            if (fabs(dt) * invperiod > 1. && B.tw == 0) {
+                B.status |= POS_STATUS_TIMESTEP_WARNING;
+                B.tw += 1;
+            }
         }
         const double dtr0i = dt * r0i;
         x = dtr0i * (1. - dtr0i * eta0 * 0.5 * r0i);
     } else {
         x = 0.;
-        x_per_period = __builtin_nan("");
     }
     int converged = 0;
     double old_x = x;
@@ -1343,7 +1352,14 @@ __device__ inline void kepler_individual_step(Lane &B, double mass_g, double dt)
     double e = eta0 * gs[1] + zeta0 * gs[2];
     double ri = 1. / (r0 + e);
     x = ri * (x * e - eta0 * gs[2] - zeta0 * gs[3] + dt);
-    if (!__builtin_isnan(x_per_period) && fabs(x - old_x) > 0.01 * x_per_period) {
+    bool laguerre = false;
+    constexpr double LIMIT2 = 0.98 * (0.01 * 2. * PI) * (0.01 * 2. * PI);
+    if (elliptic && !((x - old_x) * (x - old_x) * beta <= LIMIT2)) {
+        double invperiod, x_per_period;
+        orbit(invperiod, x_per_period);
+        laguerre = !__builtin_isnan(x_per_period) && fabs(x - old_x) > 0.01 * x_per_period;
+    }
+    if (laguerre) {
         // Laguerre-Conway (rare: only when the step is a sizeable part of an orbit)
         x = beta * dt / mass_g;
         double prev_x[NMAX_QUART + 1];
@@ -1379,6 +1395,8 @@ __device__ inline void kepler_individual_step(Lane &B, double mass_g, double dt)
         B.status |= POS_STATUS_KEPLER_BISECTION;
         double x_min, x_max;
         if (elliptic) {
+            double invperiod, x_per_period;
+            orbit(invperiod, x_per_period);
             x_min = x_per_period * floor(dt * invperiod);
             x_max = x_min + x_per_period;
         } else {
@@ -1418,8 +1436,7 @@ __device__ inline void kepler_individual_step(Lane &B, double mass_g, double dt)
 
 // Jacobi prefix sums up to body k (whfast.rs:574-576, 642-651): the
 // cumulative G-mass and mass of the host and the bodies before k, k included.
-template <class Lds>
-__device__ inline void jacobi_prefix(const Lds &lds, const Lane &B, double *mu, double *eta, int *rank) {
+__device__ inline void jacobi_prefix(const WaveLds &lds, const Lane &B, double *mu, double *eta, int *rank) {
     const int hl = B.hl();
     double m_g = mg_of(lds, hl), e = lds.m[hl];
     int r = 0;
@@ -1433,8 +1450,7 @@ __device__ inline void jacobi_prefix(const Lds &lds, const Lane &B, double *mu, 
     *mu = m_g; *eta = e; *rank = r;
 }
 
-template <class Lds>
-__device__ inline void kepler_steps(const Lds &lds, Lane &B, double dt) {
+__device__ inline void kepler_steps(const WaveLds &lds, Lane &B, double dt) {
     if (B.orbiting()) {
         double mu;
         if (B.coord == POS_COORD_JACOBI) {
@@ -1457,8 +1473,7 @@ __device__ inline void kepler_steps(const Lds &lds, Lane &B, double dt) {
 // ===========================================================================
 // Coordinate transforms, jump and interaction (whfast.rs:495-625, 881-1155)
 // ===========================================================================
-template <class Lds>
-__device__ inline void inertial_to_alternative(Lds &lds, Lane &B) {
+__device__ inline void inertial_to_alternative(WaveLds &lds, Lane &B) {
     const int lane = B.lane;
     if (B.valid()) {
         lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2];
@@ -1503,20 +1518,19 @@ __device__ inline void inertial_to_alternative(Lds &lds, Lane &B) {
         // whfast.rs:973-1023: centre of mass, host first then the others in
         // order; the seven ordered sums (x, v weighted by the masses, and the
         // masses themselves as 1 * m from row 13) are spread over the group's
-        // lanes and left in rows COM_ROW.. of column gbase
+        // lanes and left in rows 6-12 of column gbase
         if (B.valid()) lds.xb[13][lane] = 1.;
         wsync();
         for (int q = B.k; B.valid() && q < 7; q += B.n) {
             const int rq = q < 6 ? q : 13;
             double acc[1] = {0. + lds.xb[rq][hl] * lds.m[hl]};
             fold_rows<1, true>(B, acc, [&](int, int l) { return lds.xb[rq][l] * lds.m[l]; });
-            lds.xb[Lds::COM_ROW + q][B.gbase] = acc[0];
+            lds.xb[6 + q][B.gbase] = acc[0];
         }
         wsync();
-        constexpr int R = Lds::COM_ROW;
-        const double cx[3] = {lds.xb[R][B.gbase], lds.xb[R + 1][B.gbase], lds.xb[R + 2][B.gbase]};
-        const double cv[3] = {lds.xb[R + 3][B.gbase], lds.xb[R + 4][B.gbase], lds.xb[R + 5][B.gbase]};
-        const double cm = lds.xb[R + 6][B.gbase];
+        const double cx[3] = {lds.xb[6][B.gbase], lds.xb[7][B.gbase], lds.xb[8][B.gbase]};
+        const double cv[3] = {lds.xb[9][B.gbase], lds.xb[10][B.gbase], lds.xb[11][B.gbase]};
+        const double cm = lds.xb[12][B.gbase];
         B.com_m = cm;
         const Rcp Rcm = rcp(cm);
 #pragma unroll
@@ -1538,8 +1552,7 @@ __device__ inline void inertial_to_alternative(Lds &lds, Lane &B) {
     wsync();
 }
 
-template <class Lds>
-__device__ inline void jump_step(Lds &lds, Lane &B, double dt) {
+__device__ inline void jump_step(WaveLds &lds, Lane &B, double dt) {
     if (B.coord == POS_COORD_JACOBI) return;
     const int lane = B.lane;
     if (B.orbiting()) {
@@ -1577,8 +1590,7 @@ __device__ inline void jump_step(Lds &lds, Lane &B, double dt) {
     }
 }
 
-template <class Lds>
-__device__ inline void interaction_step(Lds &lds, Lane &B, double dt) {
+__device__ inline void interaction_step(WaveLds &lds, Lane &B, double dt) {
     const int lane = B.lane;
     const int hl = B.hl();
     if (B.coord == POS_COORD_JACOBI) {
@@ -1587,7 +1599,7 @@ __device__ inline void interaction_step(Lds &lds, Lane &B, double dt) {
         double eta = lds.m[hl];
         double s[3], aj_own[3] = {0., 0., 0.};
 #pragma unroll
-        for (int q = 0; q < 3; ++q) s[q] = eta * lds.acc(q, hl);
+        for (int q = 0; q < 3; ++q) s[q] = eta * lds.ag[q][hl];
         for (int j = 0; j < B.n; ++j) {
             if (j == B.host) continue;
             const int l = B.gbase + j;
@@ -1597,7 +1609,7 @@ __device__ inline void interaction_step(Lds &lds, Lane &B, double dt) {
             const double pme = eta * ei;
             double aj[3];
 #pragma unroll
-            for (int q = 0; q < 3; ++q) aj[q] = lds.acc(q, l) - s[q] * ei;
+            for (int q = 0; q < 3; ++q) aj[q] = lds.ag[q][l] - s[q] * ei;
             if (j == B.k) {
 #pragma unroll
                 for (int q = 0; q < 3; ++q) aj_own[q] = aj[q];
@@ -1625,19 +1637,18 @@ __device__ inline void interaction_step(Lds &lds, Lane &B, double dt) {
     if (B.orbiting()) {
         if (B.coord == POS_COORD_DEMOCRATIC_HELIOCENTRIC) {
 #pragma unroll
-            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + dt * lds.acc(q, lane);
+            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + dt * lds.ag[q][lane];
         } else {
             const double hm = lds.m[hl];
             const double factor = hm + B.m;
             const Rcp Rhm{hm, lds.inv_m[hl]};
 #pragma unroll
-            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + divr(dt * factor * lds.acc(q, lane), Rhm);
+            for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + divr(dt * factor * lds.ag[q][lane], Rhm);
         }
     }
 }
 
-template <class Lds>
-__device__ inline void alternative_to_inertial(Lds &lds, Lane &B) {
+__device__ inline void alternative_to_inertial(WaveLds &lds, Lane &B) {
     const int lane = B.lane;
     if (B.orbiting()) {
         lds.xb[0][lane] = B.ax[0]; lds.xb[1][lane] = B.ax[1]; lds.xb[2][lane] = B.ax[2];
@@ -1726,8 +1737,7 @@ __device__ inline void alternative_to_inertial(Lds &lds, Lane &B) {
 // ===========================================================================
 // Newtonian gravity (universe.rs:198-303)
 // ===========================================================================
-template <class Lds>
-__device__ inline void gravity(const DevEnsemble &E, Lds &lds, Lane &B) {
+__device__ inline void gravity(const DevEnsemble &E, WaveLds &lds, Lane &B) {
     const int lane = B.lane;
     if (B.valid()) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
     wsync();
@@ -1762,7 +1772,7 @@ __device__ inline void gravity(const DevEnsemble &E, Lds &lds, Lane &B) {
             acc[1] = acc[1] + prefact * dy;
             acc[2] = acc[2] + prefact * dz;
         }
-        lds.acc(0, lane) = acc[0]; lds.acc(1, lane) = acc[1]; lds.acc(2, lane) = acc[2];
+        lds.ag[0][lane] = acc[0]; lds.ag[1][lane] = acc[1]; lds.ag[2][lane] = acc[2];
     }
     wsync();
 }
@@ -1801,11 +1811,10 @@ __device__ inline void merge_status(Lds &lds, Lane &B) {
 // ===========================================================================
 template <bool EXT, class Lds>
 __device__ inline void write_history_record(const DevEnsemble &E, Lds &lds, Lane &B) {
-    constexpr int VR = Lds::HIST_V_ROW;
     const int lane = B.lane;
     if (B.valid()) {
-        lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2];
-        lds.xb[VR][lane] = B.v[0]; lds.xb[VR + 1][lane] = B.v[1]; lds.xb[VR + 2][lane] = B.v[2];
+#pragma unroll
+        for (int q = 0; q < 3; ++q) { lds.xb[Lds::hist_x_row(q)][lane] = B.x[q]; lds.xb[Lds::hist_v_row(q)][lane] = B.v[q]; }
     }
     wsync();
     double dedt = 0.;   // a body the tidal loops skip keeps its initial 0 (tides/common.rs:263-281)
@@ -1813,7 +1822,7 @@ __device__ inline void write_history_record(const DevEnsemble &E, Lds &lds, Lane
         const int hl = B.hl();
         double r[3], u[3];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) { r[q] = B.x[q] - lds.xb[q][hl]; u[q] = B.v[q] - lds.xb[VR + q][hl]; }
+        for (int q = 0; q < 3; ++q) { r[q] = B.x[q] - lds.xb[Lds::hist_x_row(q)][hl]; u[q] = B.v[q] - lds.xb[Lds::hist_v_row(q)][hl]; }
         const double d = sqrt(p2(r[0]) + p2(r[1]) + p2(r[2]));
         const double vr = (r[0] * u[0] + r[1] * u[1] + r[2] * u[2]) / d;
         const double hm = lds.m[hl];
