@@ -130,16 +130,16 @@ class Ensemble:
         system, record, body); clears the device buffer."""
         cap = getattr(self, "_hist_cap", 0)
         n_max = cap * self.n_bodies
-        buf = (abi.HistoryRecord * max(n_max, 1))()
-        n = C.c_int64()
-        abi.check(self._lib.pos_history_drain(self._h, buf, n_max, C.byref(n)))
         dt = np.dtype([("system", np.int32), ("body", np.int32), ("time", np.float64), ("time_step", np.float64),
                        ("position", np.float64, 3), ("spin", np.float64, 3), ("velocity", np.float64, 3),
                        ("mass", np.float64), ("radius", np.float64), ("radius_of_gyration_2", np.float64),
                        ("love_number", np.float64), ("scaled_dissipation_factor", np.float64),
                        ("lag_angle", np.float64), ("denergy_dt", np.float64), ("migration_timescale", np.float64)])
         assert dt.itemsize == C.sizeof(abi.HistoryRecord)
-        return np.frombuffer(bytes(buf)[:n.value * dt.itemsize], dtype=dt).copy()
+        buf = np.empty(max(n_max, 1), dtype=dt)    # pages that stay unwritten are never touched
+        n = C.c_int64()
+        abi.check(self._lib.pos_history_drain(self._h, buf.ctypes.data_as(C.POINTER(abi.HistoryRecord)), n_max, C.byref(n)))
+        return buf[:n.value] if 2 * n.value >= n_max else buf[:n.value].copy()
 
     # -- discrete adjoint -----------------------------------------------------
     def adjoint_record(self, n_steps: int, segment_steps: int = 0):
