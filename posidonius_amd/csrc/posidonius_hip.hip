@@ -236,12 +236,12 @@ void whfast_fixed_kernel(DevEnsemble E, int n_steps, TapeRef T, int wave_begin, 
     // uniform over a wavefront, so that each one runs its own role's code
     const int role = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     for (int wave = wave_begin + blockIdx.x; wave < wave_end; wave += gridDim.x) {
-        if (M == 1 || role == 0) fixed_run<M, 0, REC, JACOBI>(E, lds, wave, n_steps, T);
-        else if constexpr (M == 2) fixed_run<M, 1, REC, JACOBI>(E, lds, wave, n_steps, T);
+        if (M == 1 || role == 0) fixed_run<M, 0, REC, V>(E, lds, wave, n_steps, T);
+        else if constexpr (M == 2) fixed_run<M, 1, REC, V>(E, lds, wave, n_steps, T);
         else if constexpr (M == 4) {
-            if (role == 1) fixed_run<M, 1, REC, JACOBI>(E, lds, wave, n_steps, T);
-            else if (role == 2) fixed_run<M, 2, REC, JACOBI>(E, lds, wave, n_steps, T);
-            else fixed_run<M, 3, REC, JACOBI>(E, lds, wave, n_steps, T);
+            if (role == 1) fixed_run<M, 1, REC, V>(E, lds, wave, n_steps, T);
+            else if (role == 2) fixed_run<M, 2, REC, V>(E, lds, wave, n_steps, T);
+            else fixed_run<M, 3, REC, V>(E, lds, wave, n_steps, T);
         }
         __syncthreads();
     }
@@ -314,7 +314,8 @@ __global__ __launch_bounds__(64) void effects_kernel(DevEnsemble E, double *out_
     Lane B;
     load_lane<V>(E, lds, B, wave);
     double a[3], dL[3];
-    additional_effects<V>(E, lds, B, false, a, dL);
+    SolveCache sc;
+    additional_effects<V>(E, lds, B, false, a, dL, sc, true);
     const int nb = E.n_bodies;
     if (B.valid()) {
 #pragma unroll
@@ -837,6 +838,7 @@ int system_variant(const pos_ensemble_desc *d, int s, int host) {
     if (v == GRV_KIDDER && effects == FAST_EFFECTS && implementation == POS_GR_KIDDER1995 && every_body_orbits(d, s, host)) {
         if (d->coordinates[s] == POS_COORD_DEMOCRATIC_HELIOCENTRIC) v |= VAR_FAST;
         if (d->coordinates[s] == POS_COORD_JACOBI) v |= VAR_FAST | VAR_JACOBI;
+        if (d->coordinates[s] == POS_COORD_WHDS) v |= VAR_FAST | VAR_WHDS;
     }
     return v;
 }
@@ -1075,6 +1077,7 @@ int launch_steps(pos_ens *h, int n_steps, int *launches = nullptr) {
             case 6: launch_steps_variant<6>(h, grid, n_steps, w0, w1); break;
             case 8: launch_fixed<false, 8>(h, h->E, grid, n_steps, TapeRef{nullptr, 0}, w0, w1); break;
             case 24: launch_fixed<false, 24>(h, h->E, grid, n_steps, TapeRef{nullptr, 0}, w0, w1); break;
+            case 40: launch_fixed<false, 40>(h, h->E, grid, n_steps, TapeRef{nullptr, 0}, w0, w1); break;
             default: return fail(POS_E_INVALID, "internal error: unknown kernel variant");
         }
         HIP_TRY(hipGetLastError());
@@ -1135,7 +1138,8 @@ int launch_effects(pos_ens *h, double *d_a, double *d_l) {
             case 4: hipLaunchKernelGGL(effects_kernel<4>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
             case 5: hipLaunchKernelGGL(effects_kernel<5>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
             case 6: hipLaunchKernelGGL(effects_kernel<6>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
-            case 8: hipLaunchKernelGGL(effects_kernel<8>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
+            case 8: case 40:   // the effects do not depend on the coordinates
+                hipLaunchKernelGGL(effects_kernel<8>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
             case 24: hipLaunchKernelGGL(effects_kernel<24>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
             default: return fail(POS_E_INVALID, "internal error: unknown kernel variant");
         }
@@ -1999,7 +2003,7 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
         if (s + 2 < A.n_seg) HIP_TRY(hipStreamWaitEvent(h->stream, A.swept_ev[buf], 0));
         int r = adjoint_copy_state(h, A.ckpt + (size_t)s * A.state_bytes, false);
         if (r) return r;
-        for (int v = 0; v < N_VARIANTS; ++v) {   // pos_adjoint_record admits variants 0, 8 and 24 only
+        for (int v = 0; v < N_VARIANTS; ++v) {   // pos_adjoint_record admits variants 0, 8, 24 and 40 only
             const int w0 = h->variant_waves[v][0], w1 = h->variant_waves[v][1];
             if (w1 <= w0) continue;
             const dim3 grid(std::min(h->grid, w1 - w0));
@@ -2012,6 +2016,8 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
                 launch_fixed<true, GRV_KIDDER | VAR_FAST>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
             else if (v == (GRV_KIDDER | VAR_FAST | VAR_JACOBI))
                 launch_fixed<true, GRV_KIDDER | VAR_FAST | VAR_JACOBI>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
+            else if (v == (GRV_KIDDER | VAR_FAST | VAR_WHDS))
+                launch_fixed<true, GRV_KIDDER | VAR_FAST | VAR_WHDS>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
             else
                 return fail(POS_E_INVALID, "internal error: kernel variant without an adjoint");
             HIP_TRY(hipGetLastError());

@@ -1,6 +1,5 @@
 // whfast_fixed.hpp -- the step of the fixed effect set (VAR_FAST): systems with
-// exactly tides + flattening + Kidder GR with spins, in democratic
-// heliocentric or Jacobi coordinates, run by teams of one, two or four
+// exactly tides + flattening + Kidder GR with spins, in any coordinates, run by teams of one, two or four
 // wavefronts.
 //
 // Most of a step is the evaluation of those effects inside the two
@@ -836,16 +835,19 @@ __device__ __forceinline__ void fixed_gravity(const DevEnsemble &E, Lds &lds, Fi
     }
 }
 
-// Democratic heliocentric drift (whfast.rs:495-625, 973-1155).  Each body
+// Democratic heliocentric and WHDS drift (whfast.rs:495-625, 973-1155).  Each body
 // forms its own term of every sum (a quotient by a mass included) before the
 // terms are exchanged, so a sum is only its additions.
-template <bool DIRECT, bool REC, class Lds>
+template <bool DIRECT, bool REC, bool WHDS, class Lds>
 __device__ __forceinline__ void drift_heliocentric(const DevEnsemble &E, Lds &lds, FixedLane &B, double acc[3], const TapeRef &T,
                                                    int row) {
     const int lane = B.lane, hl = B.hl();
     const double half_dt = 0.5 * B.dt;
     const Rcp Rm0{lds.m[hl], lds.of_system(B, K_INV_HM)};
     const Rcp Rmt{lds.of_system(B, K_TOTAL), lds.of_system(B, K_INV_TOTAL)};
+    // WHDS: the mass of the pair with the host, the velocities' factor (whfast.rs:973-1023)
+    const Rcp Rpair = rcp(WHDS ? Rm0.b + B.m : 1.);
+    const double factor = WHDS ? divr(Rpair.b, Rm0) : 1.;
     // centre of mass, the host first
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
@@ -865,11 +867,12 @@ __device__ __forceinline__ void drift_heliocentric(const DevEnsemble &E, Lds &ld
             B.comv[q] = divr(com[1][q], Rmt);
             B.ax[q] = B.x[q] - lds.xb[6 + q][hl];
             B.av[q] = B.v[q] - B.comv[q];
+            if constexpr (WHDS) B.av[q] = B.av[q] * factor;
         }
         wsync();
     }
     auto drift = [&](int field) {
-        if (B.orb) kepler_individual_step(B, mg_of(lds, hl), half_dt);
+        if (B.orb) kepler_individual_step(B, WHDS ? mg_of(lds, hl) + mg_of(lds, lane) : mg_of(lds, hl), half_dt);
 #pragma unroll
         for (int q = 0; q < 3; ++q) B.comx[q] = B.comx[q] + half_dt * B.comv[q];
         if (REC) *T.at(row, field, B.body) = B.orb ? B.kx : 0.;
@@ -878,12 +881,15 @@ __device__ __forceinline__ void drift_heliocentric(const DevEnsemble &E, Lds &ld
         const double zero[1][3] = {{0., 0., 0.}};
         double p[1][3];
 #pragma unroll
-        for (int q = 0; q < 3; ++q) lds.xb[q][lane] = B.m * B.av[q];
+        for (int q = 0; q < 3; ++q) lds.xb[q][lane] = WHDS ? divr(B.m * B.av[q], Rpair) : B.m * B.av[q];
         wsync();
         group_sums<1, false, DIRECT>(lds, B, zero, p);
         wsync();
 #pragma unroll
-        for (int q = 0; q < 3; ++q) B.ax[q] = B.ax[q] + divr(half_dt * p[0][q], Rm0);
+        for (int q = 0; q < 3; ++q) {
+            if constexpr (WHDS) B.ax[q] = B.ax[q] + half_dt * (p[0][q] - divr(B.m * B.av[q], Rpair));
+            else B.ax[q] = B.ax[q] + divr(half_dt * p[0][q], Rm0);
+        }
     };
     drift(TP_XK1);
     jump();
@@ -905,7 +911,7 @@ __device__ __forceinline__ void drift_heliocentric(const DevEnsemble &E, Lds &ld
     fixed_gravity<false, DIRECT ? 4 : 2>(E, lds, B, acc);
     wsync();
 #pragma unroll
-    for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + B.dt * acc[q];
+    for (int q = 0; q < 3; ++q) B.av[q] = B.av[q] + (WHDS ? divr(B.dt * Rpair.b * acc[q], Rm0) : B.dt * acc[q]);
     jump();
     drift(TP_XK2);
     {
@@ -914,15 +920,16 @@ __device__ __forceinline__ void drift_heliocentric(const DevEnsemble &E, Lds &ld
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             lds.xb[q][lane] = divr(B.ax[q] * B.m, Rmt);
-            lds.xb[3 + q][lane] = B.av[q] * lds.konst(B, K_M_OVER_HM);
+            lds.xb[3 + q][lane] = B.av[q] * (WHDS ? divr(B.m, Rpair) : lds.konst(B, K_M_OVER_HM));
         }
         wsync();
         group_sums<2, true, DIRECT>(lds, B, init, h);
         wsync();
+        const Rcp Rfactor = rcp(factor);
 #pragma unroll
         for (int q = 0; q < 3; ++q) {
             B.x[q] = B.host_lane ? h[0][q] : B.ax[q] + h[0][q];
-            B.v[q] = B.host_lane ? h[1][q] : B.av[q] + B.comv[q];
+            B.v[q] = B.host_lane ? h[1][q] : (WHDS ? divr(B.av[q], Rfactor) : B.av[q]) + B.comv[q];
         }
     }
 }
@@ -1054,9 +1061,10 @@ __device__ __forceinline__ void drift_jacobi(const DevEnsemble &E, Lds &lds, Fix
 // The lane's body and its constants; wave 0 fills the shared constants and the
 // published positions and velocities, the owner of the spins the spins of the
 // last evaluation.  Ends without a barrier.
-template <int M, int ROLE, bool JACOBI>
-__device__ __forceinline__ void fixed_load(const DevEnsemble &E, FixedLds<M, JACOBI> &lds, FixedLane &B, int wave) {
+template <int M, int ROLE, int V>
+__device__ __forceinline__ void fixed_load(const DevEnsemble &E, FixedLds<M, (V & VAR_JACOBI) != 0> &lds, FixedLane &B, int wave) {
     using W = Role<M, ROLE>;
+    constexpr bool JACOBI = (V & VAR_JACOBI) != 0;
     const int lane = threadIdx.x & (WAVE - 1);
     const LaneGroup lg = lane_group(E, wave, lane);
     const int s = lg.sys;
@@ -1077,7 +1085,7 @@ __device__ __forceinline__ void fixed_load(const DevEnsemble &E, FixedLds<M, JAC
     while (__any(B.n > B.nmax)) ++B.nmax;
     B.pairs = __any(B.n == 2);
     B.hosts_first = !__any(valid && B.hidx != 0);
-    B.coord = JACOBI ? POS_COORD_JACOBI : POS_COORD_DEMOCRATIC_HELIOCENTRIC;
+    B.coord = JACOBI ? POS_COORD_JACOBI : (V & VAR_WHDS) ? POS_COORD_WHDS : POS_COORD_DEMOCRATIC_HELIOCENTRIC;
     B.flags = (valid ? F_VALID : 0u) | (B.host_lane ? F_HOST : 0u) | F_TIDES | F_RF | F_GR | F_SPIN |
               (B.orb ? (F_TIDES_ROLE | F_RF_ROLE | F_GR_ROLE) : 0u);
     const int b = B.body, nb = E.n_bodies;
@@ -1239,13 +1247,14 @@ __device__ __forceinline__ void fixed_store(const DevEnsemble &E, const Lds &lds
 
 // The steps of one launch for the systems of wave `wave`, wavefront ROLE of the
 // team.  With REC each step also writes its tape row.
-template <int M, int ROLE, bool REC, bool JACOBI>
-__device__ __forceinline__ void fixed_run(const DevEnsemble &E, FixedLds<M, JACOBI> &lds, int wave, int n_steps, const TapeRef &T) {
+template <int M, int ROLE, bool REC, int V>
+__device__ __forceinline__ void fixed_run(const DevEnsemble &E, FixedLds<M, (V & VAR_JACOBI) != 0> &lds, int wave, int n_steps, const TapeRef &T) {
     using W = Role<M, ROLE>;
+    constexpr bool JACOBI = (V & VAR_JACOBI) != 0;
     constexpr uint32_t STOPPED = POS_STATUS_COMPLETED | POS_STATUS_FATAL;
     FixedLane B;
     FixedGeo g{};
-    fixed_load<M, ROLE, JACOBI>(E, lds, B, wave);
+    fixed_load<M, ROLE, V>(E, lds, B, wave);
     const int lane = B.lane;
     bool act = false, snap = false;
     double s_last[3];
@@ -1348,7 +1357,7 @@ __device__ __forceinline__ void fixed_run(const DevEnsemble &E, FixedLds<M, JACO
                     double acc[3];
                     wsync();
                     if constexpr (JACOBI) drift_jacobi<(M > 1), REC>(E, lds, B, acc, T, step);
-                    else drift_heliocentric<(M > 1), REC>(E, lds, B, acc, T, step);
+                    else drift_heliocentric<(M > 1), REC, (V & VAR_WHDS) != 0>(E, lds, B, acc, T, step);
                     // the state's gravitational acceleration, stored here rather than held through the second kick
                     const int nb = E.n_bodies;
 #pragma unroll

@@ -463,18 +463,19 @@ __device__ __forceinline__ void host_reaction_sums(WaveLds &lds, const Lane &B) 
 enum GrVariant { GRV_KIDDER = 0, GRV_ANDERSON = 1, GRV_NEWHALL = 2 };
 // Kernel variant: the GR variant plus VAR_EXT for systems with the disk effect
 // or an evolving-dissipation host (the extended effects pass).  The device
-// copy of a system's effect mask carries its variant in bits 16-18.
+// copy of a system's effect mask carries its variant in bits 16-21.
 constexpr int VAR_EXT = 4;
 // VAR_FAST: every system of the launch has exactly tides + flattening + Kidder
 // GR (spins integrated), no wind, disk or evolution, democratic heliocentric
-// coordinates (with VAR_JACOBI: Jacobi coordinates); the flags and the
+// coordinates (with VAR_JACOBI or VAR_WHDS: those); the flags and the
 // coordinate type are then compile-time constants and the per-system branches
 // fold away (same arithmetic).
 constexpr int VAR_FAST = 8;
 constexpr int VAR_JACOBI = 16;   // only with VAR_FAST
-constexpr int N_VARIANTS = 32;
+constexpr int VAR_WHDS = 32;     // only with VAR_FAST
+constexpr int N_VARIANTS = 64;
 constexpr uint32_t EFF_VAR_SHIFT = 16;
-__host__ __device__ __forceinline__ int eff_variant(uint32_t eff) { return (int)((eff >> EFF_VAR_SHIFT) & 31u); }
+__host__ __device__ __forceinline__ int eff_variant(uint32_t eff) { return (int)((eff >> EFF_VAR_SHIFT) & 63u); }
 __host__ __device__ __forceinline__ int eff_gr_variant(uint32_t eff) { return eff_variant(eff) & 3; }
 
 // The effect and role tests of a lane for kernel variant V.  Under VAR_FAST
@@ -502,6 +503,19 @@ struct LaneTests {
 // index): position of body k, and body at position c.
 __device__ __forceinline__ int chained_pos(const Lane &B, int k) { return k == B.host ? 0 : (k < B.host ? k + 1 : k); }
 __device__ __forceinline__ int chained_body(const Lane &B, int c) { return c == 0 ? B.host : (c - 1 < B.host ? c - 1 : c); }
+
+// What the effects evaluations of one implicit-midpoint solve share because the
+// positions, masses and time do not change inside it: formed by the first
+// evaluation, read by the others (each is the value the expression would give
+// again).  A kernel variant keeps what its effects use.
+struct SolveCache {
+    double an[3];           // Newtonian acceleration of gr_newtonian
+    double a1, a2;          // Newhall: this body's mass sums
+    double nc[3];           // Newhall: the acceleration terms of the first fixed-point pass
+    double viscosity, surface_density;   // disk at this body
+};
+
+constexpr Rcp RC2{SPEED_OF_LIGHT_2, 1. / SPEED_OF_LIGHT_2};
 
 // general_relativity.rs:641-681: the accelerations of the last gravity
 // evaluation plus the host pair terms the splitting ignored; the separation
@@ -540,12 +554,12 @@ __device__ inline void gr_newtonian(WaveLds &lds, Lane &B, double an[3]) {
 }
 
 // Anderson et al. 1975 through Jacobi coordinates (general_relativity.rs:461-639)
-__device__ inline void gr_anderson1975(WaveLds &lds, Lane &B, double g[3]) {
+__device__ inline void gr_anderson1975(WaveLds &lds, Lane &B, double g[3], SolveCache &sc, bool first) {
     const int lane = B.lane, hl = B.hl();
     if (B.valid()) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
     wsync();
-    double an[3];
-    gr_newtonian(lds, B, an);
+    if (first) gr_newtonian(lds, B, sc.an);
+    const double *an = sc.an;
     if (B.valid()) {
 #pragma unroll
         for (int q = 0; q < 3; ++q) { lds.xb[3 + q][lane] = B.v[q]; lds.xb[6 + q][lane] = an[q]; }
@@ -589,21 +603,23 @@ __device__ inline void gr_anderson1975(WaveLds &lds, Lane &B, double g[3]) {
         double vi[3] = {jv[0], jv[1], jv[2]};
         double vi2 = p2(jv[0]) + p2(jv[1]) + p2(jv[2]);
         const double ri = sqrt(p2(jx[0]) + p2(jx[1]) + p2(jx[2]));
-        double fa = (0.5 * vi2 + 3. * mu / ri) / SPEED_OF_LIGHT_2;
+        const double potential = 3. * mu / ri;
+        double fa = divr(0.5 * vi2 + potential, RC2);
         for (int it = 0; it < 10; ++it) {
             const double o0 = vi[0], o1 = vi[1], o2 = vi[2];
-            vi[0] = jv[0] / (1. - fa); vi[1] = jv[1] / (1. - fa); vi[2] = jv[2] / (1. - fa);
+            const Rcp R1 = rcp(1. - fa);
+            vi[0] = divr(jv[0], R1); vi[1] = divr(jv[1], R1); vi[2] = divr(jv[2], R1);
             vi2 = vi[0] * vi[0] + vi[1] * vi[1] + vi[2] * vi[2];
-            fa = (0.5 * vi2 + 3. * mu / ri) / SPEED_OF_LIGHT_2;
+            fa = divr(0.5 * vi2 + potential, RC2);
             const double dvx = vi[0] - o0, dvy = vi[1] - o1, dvz = vi[2] - o2;
             if ((dvx * dvx + dvy * dvy + dvz * dvz) / vi2 < DBL_EPS_2) break;
         }
         const double ri3 = ri * ri * ri;
-        const double fb = (mu / ri - 1.5 * vi2) * mu / ri3 / SPEED_OF_LIGHT_2;
+        const double fb = divr((mu / ri - 1.5 * vi2) * mu / ri3, RC2);
         const double rdr = jx[0] * jv[0] + jx[1] * jv[1] + jx[2] * jv[2];
         const double vd0 = ja[0] + fb * jx[0], vd1 = ja[1] + fb * jx[1], vd2 = ja[2] + fb * jx[2];
         const double vdv = vi[0] * vd0 + vi[1] * vd1 + vi[2] * vd2;
-        const double fd = (vdv - 3. * mu / ri3 * rdr) / SPEED_OF_LIGHT_2;
+        const double fd = divr(vdv - 3. * mu / ri3 * rdr, RC2);
 #pragma unroll
         for (int q = 0; q < 3; ++q) ja[q] = fb * (1. - fa) * jx[q] - fa * ja[q] - fd * vi[q];
         lds.xb[9][lane] = ja[0]; lds.xb[10][lane] = ja[1]; lds.xb[11][lane] = ja[2];
@@ -636,119 +652,139 @@ __device__ inline void gr_anderson1975(WaveLds &lds, Lane &B, double g[3]) {
     wsync();
 }
 
-// Newhall et al. 1983, every pair (general_relativity.rs:683-895)
-__device__ inline void gr_newhall1983(WaveLds &lds, Lane &B, double g[3]) {
+// Newhall et al. 1983, every pair (general_relativity.rs:683-895).  Most of the
+// pair terms depend on the positions alone: the sums a1 and a2 and, the first
+// pass of the fixed point starting from zero, its acceleration terms.  They are
+// formed by the first evaluation of a solve; an evaluation then costs the
+// velocity terms, one square root and two reciprocals a pair (430 against 110
+// instructions; quotients by a shared or constant divisor go through divr).
+__device__ inline void gr_newhall1983(WaveLds &lds, Lane &B, double g[3], SolveCache &sc, bool first) {
     const int lane = B.lane;
     const int n = B.n;
     if (B.valid()) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
     wsync();
-    double an[3];
-    gr_newtonian(lds, B, an);
+    if (first) gr_newtonian(lds, B, sc.an);
     if (B.valid()) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) { lds.xb[3 + q][lane] = B.v[q]; lds.xb[6 + q][lane] = an[q]; }
+        for (int q = 0; q < 3; ++q) { lds.xb[3 + q][lane] = B.v[q]; lds.xb[6 + q][lane] = sc.an[q]; }
     }
-    const double c2 = SPEED_OF_LIGHT_2;
-    // distance to the body at chained position c (0 for itself)
-    auto dist = [&](int c) {
-        const int l = B.gbase + chained_body(B, c);
-        const double dx = B.x[0] - lds.xb[0][l], dy = B.x[1] - lds.xb[1][l], dz = B.x[2] - lds.xb[2][l];
-        return sqrt(p2(dx) + p2(dy) + p2(dz));
-    };
+    constexpr double c2 = SPEED_OF_LIGHT_2;
+    constexpr Rcp R2C2{2. * c2, 1. / (2. * c2)};
     const int me = chained_pos(B, B.k);
-    wsync();
-    // a2 depends only on the second body j: sum_l G m_l / (c^2 r_lj), which
-    // body j evaluates from its own distances (|x_l - x_j| = |x_j - x_l|)
-    double a1 = 0., a2own = 0.;
-    if (B.valid()) {
+    auto separation = [&](int l, double d[3]) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) d[q] = B.x[q] - lds.xb[q][l];
+        return sqrt(p2(d[0]) + p2(d[1]) + p2(d[2]));
+    };
+    // the acceleration terms of one fixed-point pass; rows 10-12 hold the
+    // previous iterate of every body (with START it is zero everywhere)
+    auto acceleration_terms = [&](double nc[3], auto start) {
+        nc[0] = nc[1] = nc[2] = 0.;
         for (int c = 0; c < n; ++c) {
             if (c == me) continue;
-            const double mk = lds.m[B.gbase + chained_body(B, c)];
-            const double r = dist(c);
-            a1 = a1 + (4. / c2) * G * mk / r;
-            a2own = a2own + (1. / c2) * G * mk / r;
+            const int l = B.gbase + chained_body(B, c);
+            double d[3], s[3];
+            const double rij = separation(l, d);
+            const double rij2 = p2(rij);
+            const Rcp R1 = rcp(rij), R3 = rcp(rij2 * rij);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) s[q] = lds.xb[6 + q][l] + (start ? 0. : lds.xb[10 + q][l]);
+            const double proj = d[0] * s[0] + d[1] * s[1] + d[2] * s[2];
+            const double gm = G * lds.m[l];
+#pragma unroll
+            for (int q = 0; q < 3; ++q)
+                nc[q] = nc[q] + divr(divr(gm * d[q], R3) * proj, R2C2) + divr((7. / (2. * c2)) * G * lds.m[l] * s[q], R1);
         }
-        lds.xb[9][lane] = a2own;
+    };
+    wsync();
+    if (first && B.valid()) {
+        // a2 depends only on the second body j: sum_l G m_l / (c^2 r_lj), which
+        // body j evaluates from its own distances (|x_l - x_j| = |x_j - x_l|)
+        sc.a1 = sc.a2 = 0.;
+        for (int c = 0; c < n; ++c) {
+            if (c == me) continue;
+            const int l = B.gbase + chained_body(B, c);
+            const double mk = lds.m[l];
+            double d[3];
+            const Rcp R1 = rcp(separation(l, d));
+            sc.a1 = sc.a1 + divr((4. / c2) * G * mk, R1);
+            sc.a2 = sc.a2 + divr((1. / c2) * G * mk, R1);
+        }
+        acceleration_terms(sc.nc, std::true_type{});
     }
+    if (B.valid()) lds.xb[9][lane] = sc.a2;
     wsync();
     double ac[3] = {0., 0., 0.};
     if (B.valid()) {
         const double vi2 = p2(B.v[0]) + p2(B.v[1]) + p2(B.v[2]);
+        const double a3 = divr(-vi2, RC2);
         for (int c = 0; c < n; ++c) {
             if (c == me) continue;
             const int l = B.gbase + chained_body(B, c);
-            const double dx = B.x[0] - lds.xb[0][l], dy = B.x[1] - lds.xb[1][l], dz = B.x[2] - lds.xb[2][l];
-            const double rij = sqrt(p2(dx) + p2(dy) + p2(dz));
+            double d[3];
+            const double rij = separation(l, d);
             const double rij2 = p2(rij);
-            const double rij3 = rij2 * rij;
+            const Rcp R3 = rcp(rij2 * rij);
             const double vj0 = lds.xb[3][l], vj1 = lds.xb[4][l], vj2c = lds.xb[5][l];
             const double a2 = lds.xb[9][l];
-            const double a3 = -vi2 / c2;
             const double vj2 = p2(vj0) + p2(vj1) + p2(vj2c);
-            const double a4 = -2. * vj2 / c2;
+            const double a4 = divr(-2. * vj2, RC2);
             const double a5 = (4. / c2) * (B.v[0] * vj0 + B.v[1] * vj1 + B.v[2] * vj2c);
-            const double a60 = dx * vj0 + dy * vj1 + dz * vj2c;
+            const double a60 = d[0] * vj0 + d[1] * vj1 + d[2] * vj2c;
             const double a6 = (3. / (2. * c2)) * p2(a60) / rij2;
-            const double f1 = a1 + a2 + a3 + a4 + a5 + a6;
+            const double f1 = sc.a1 + a2 + a3 + a4 + a5 + a6;
             const double gm = G * lds.m[l];
-            ac[0] = ac[0] + gm * dx * f1 / rij3;
-            ac[1] = ac[1] + gm * dy * f1 / rij3;
-            ac[2] = ac[2] + gm * dz * f1 / rij3;
-            const double dvx = B.v[0] - vj0, dvy = B.v[1] - vj1, dvz = B.v[2] - vj2c;
-            const double f2 = dx * (4. * B.v[0] - 3. * vj0) + dy * (4. * B.v[1] - 3. * vj1) + dz * (4. * B.v[2] - 3. * vj2c);
-            ac[0] = ac[0] + gm * f2 * dvx / rij3 / c2;
-            ac[1] = ac[1] + gm * f2 * dvy / rij3 / c2;
-            ac[2] = ac[2] + gm * f2 * dvz / rij3 / c2;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) ac[q] = ac[q] + divr(gm * d[q] * f1, R3);
+            const double dv[3] = {B.v[0] - vj0, B.v[1] - vj1, B.v[2] - vj2c};
+            const double f2 = d[0] * (4. * B.v[0] - 3. * vj0) + d[1] * (4. * B.v[1] - 3. * vj1) + d[2] * (4. * B.v[2] - 3. * vj2c);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) ac[q] = ac[q] + divr(divr(gm * f2 * dv[q], R3), RC2);
         }
     }
-    // fixed point: rows 10-12 hold the previous iterate of every body, rows
-    // 13-15 the new one.  A group stops iterating when its own test passes
-    // (every lane of the group evaluates it identically); the wavefront
-    // leaves the loop once every group has.
+    // The fixed point's convergence test of the reference only looks at
+    // components below dev_limit (the deviations persist across bodies and are
+    // only updated for those): without one in the wavefront the first pass is
+    // the result.
+    constexpr double dev_limit = 1.0e-30;
     double anew[3] = {0., 0., 0.};
-    bool done = !B.valid();
-    for (int k = 0; k < 10; ++k) {
-        if (B.valid()) { lds.xb[10][lane] = anew[0]; lds.xb[11][lane] = anew[1]; lds.xb[12][lane] = anew[2]; }
-        wsync();
-        double nc[3] = {0., 0., 0.};
-        if (!done) {
-            for (int c = 0; c < n; ++c) {
-                if (c == me) continue;
-                const int l = B.gbase + chained_body(B, c);
-                const double dx = B.x[0] - lds.xb[0][l], dy = B.x[1] - lds.xb[1][l], dz = B.x[2] - lds.xb[2][l];
-                const double rij = sqrt(p2(dx) + p2(dy) + p2(dz));
-                const double rij2 = p2(rij);
-                const double rij3 = rij2 * rij;
-                const double s0 = lds.xb[6][l] + lds.xb[10][l], s1 = lds.xb[7][l] + lds.xb[11][l], s2 = lds.xb[8][l] + lds.xb[12][l];
-                const double proj = dx * s0 + dy * s1 + dz * s2;
-                const double gm = G * lds.m[l];
-                nc[0] = nc[0] + (gm * dx / rij3) * proj / (2. * c2) + (7. / (2. * c2)) * G * lds.m[l] * s0 / rij;
-                nc[1] = nc[1] + (gm * dy / rij3) * proj / (2. * c2) + (7. / (2. * c2)) * G * lds.m[l] * s1 / rij;
-                nc[2] = nc[2] + (gm * dz / rij3) * proj / (2. * c2) + (7. / (2. * c2)) * G * lds.m[l] * s2 / rij;
+    if (B.valid()) { anew[0] = ac[0] + sc.nc[0]; anew[1] = ac[1] + sc.nc[1]; anew[2] = ac[2] + sc.nc[2]; }
+    const bool tiny = fabs(anew[0]) < dev_limit || fabs(anew[1]) < dev_limit || fabs(anew[2]) < dev_limit;
+    if (__any(B.valid() && tiny)) {
+        // rows 10-12 hold the previous iterate of every body, rows 13-15 the
+        // new one.  A group stops iterating when its own test passes (every
+        // lane of the group evaluates it identically); the wavefront leaves
+        // the loop once every group has.
+        anew[0] = anew[1] = anew[2] = 0.;
+        bool done = !B.valid();
+        for (int k = 0; k < 10; ++k) {
+            if (B.valid()) { lds.xb[10][lane] = anew[0]; lds.xb[11][lane] = anew[1]; lds.xb[12][lane] = anew[2]; }
+            wsync();
+            if (!done) {
+                double nc[3];
+                acceleration_terms(nc, std::false_type{});
+                anew[0] = ac[0] + nc[0]; anew[1] = ac[1] + nc[1]; anew[2] = ac[2] + nc[2];
             }
+            if (B.valid()) { lds.xb[13][lane] = anew[0]; lds.xb[14][lane] = anew[1]; lds.xb[15][lane] = anew[2]; }
+            wsync();
+            double maxdev = 0., ddx = 0., ddy = 0., ddz = 0.;
+            for (int c = 0; !done && c < n; ++c) {
+                const int l = B.gbase + chained_body(B, c);
+                const double nx = lds.xb[13][l], ny = lds.xb[14][l], nz = lds.xb[15][l];
+                if (fabs(nx) < dev_limit) ddx = fabs(nx - lds.xb[10][l]) / nx;
+                if (fabs(ny) < dev_limit) ddy = fabs(ny - lds.xb[11][l]) / ny;
+                if (fabs(nz) < dev_limit) ddz = fabs(nz - lds.xb[12][l]) / nz;
+                if (ddx > maxdev) maxdev = ddx;
+                if (ddy > maxdev) maxdev = ddy;
+                if (ddz > maxdev) maxdev = ddz;
+            }
+            if (maxdev < dev_limit) done = true;
+            wsync();
+            if (__all(done)) break;
         }
-        if (!done) { anew[0] = ac[0] + nc[0]; anew[1] = ac[1] + nc[1]; anew[2] = ac[2] + nc[2]; }
-        if (B.valid()) { lds.xb[13][lane] = anew[0]; lds.xb[14][lane] = anew[1]; lds.xb[15][lane] = anew[2]; }
-        wsync();
-        // convergence test of the reference, in its order (the deviations
-        // persist across bodies and are only updated for tiny components)
-        const double dev_limit = 1.0e-30;
-        double maxdev = 0., ddx = 0., ddy = 0., ddz = 0.;
-        for (int c = 0; !done && c < n; ++c) {
-            const int l = B.gbase + chained_body(B, c);
-            const double nx = lds.xb[13][l], ny = lds.xb[14][l], nz = lds.xb[15][l];
-            if (fabs(nx) < dev_limit) ddx = fabs(nx - lds.xb[10][l]) / nx;
-            if (fabs(ny) < dev_limit) ddy = fabs(ny - lds.xb[11][l]) / ny;
-            if (fabs(nz) < dev_limit) ddz = fabs(nz - lds.xb[12][l]) / nz;
-            if (ddx > maxdev) maxdev = ddx;
-            if (ddy > maxdev) maxdev = ddy;
-            if (ddz > maxdev) maxdev = ddz;
-        }
-        if (maxdev < dev_limit) done = true;
-        wsync();
-        if (__all(done)) break;
     }
     g[0] = anew[0]; g[1] = anew[1]; g[2] = anew[2];
+    wsync();
 }
 
 // tools.rs:251-285 (Mercury's perihelion distance and eccentricity)
@@ -782,21 +818,24 @@ __device__ inline bool excited_pair_factor(double mean_motion, double norm_spin,
 // Disk force on an orbiting body (disk.rs:155-268, Alibert et al. 2013) from
 // its heliocentric position and velocity; stores its migration timescale.
 __device__ inline void disk_force(const DevEnsemble &E, const WaveLds &lds, const Lane &B, const double px[3],
-                                  const double pv[3], double d, double nv2, double F[3]) {
+                                  const double pv[3], double d, double nv2, double F[3], SolveCache &sc, bool first) {
     const double *dp = E.disk_props + 6 * B.sys;   // inner, outer, lifetime, alpha, sigma0, mu
     const int hl = B.hl();
     const double hm = lds.m[hl], hmg = mg_of(lds, hl), m = B.m, mg = mg_of(lds, B.lane);
     const double sma = (mg + hmg) * d / (2.0 * (mg + hmg) - d * nv2);
-    // gas radial velocity from the alpha viscosity (disk.rs:206-226)
-    const double keplerian_frequency = sqrt(hmg / (d * (d * d)));
-    const double temperature = 280.0 * poscr::cr_rsqrt(d) * hm;
-    const double speed_of_sound_2 = BOLTZMANN_CONSTANT * temperature / (dp[5] * MASS_HYDROGEN_ATOM);
-    const double viscosity = dp[3] * speed_of_sound_2 / keplerian_frequency;
-    const double gas_radial_velocity = -3.0 * viscosity / (2.0 * sma);
-    // surface density (disk.rs:196-205)
-    const double initial = dp[4] * (1. / d) * poscr::cr_exp(-1.0 * d / dp[1]) * (1.0 - sqrt(dp[0] / d));
-    double surface_density = 0.0;
-    if (d > dp[0]) surface_density = initial * poscr::cr_exp(-B.t / dp[2]);
+    if (first) {   // what depends on the distance and the time alone
+        // alpha viscosity (disk.rs:206-226)
+        const double keplerian_frequency = sqrt(hmg / (d * (d * d)));
+        const double temperature = 280.0 * poscr::cr_rsqrt(d) * hm;
+        const double speed_of_sound_2 = BOLTZMANN_CONSTANT * temperature / (dp[5] * MASS_HYDROGEN_ATOM);
+        sc.viscosity = dp[3] * speed_of_sound_2 / keplerian_frequency;
+        // surface density (disk.rs:196-205)
+        const double initial = dp[4] * (1. / d) * poscr::cr_exp(-1.0 * d / dp[1]) * (1.0 - sqrt(dp[0] / d));
+        sc.surface_density = 0.0;
+        if (d > dp[0]) sc.surface_density = initial * poscr::cr_exp(-B.t / dp[2]);
+    }
+    const double gas_radial_velocity = -3.0 * sc.viscosity / (2.0 * sma);
+    const double surface_density = sc.surface_density;
     const double ratio = 2.0 * surface_density * p2(sma) / m;
     const double a_dot = gas_radial_velocity * ((ratio != ratio || ratio > 1.0) ? 1.0 : ratio);   // f64::min(1, .)
     const double timescale = -sma / a_dot;
@@ -812,12 +851,13 @@ __device__ inline void disk_force(const DevEnsemble &E, const WaveLds &lds, cons
 }
 
 // Accelerations and spin derivatives of every body of the group at the current
-// (averaged) state.  Outputs are accumulated in the reference's order:
+// (averaged) state; first: the first evaluation at these positions, which fills
+// the cache of the solve.  Outputs are accumulated in the reference's order:
 // a_add = ((0 + tides) + flattening) + GR and
 // dL/dt = ((tides + flattening) + GR) + wind (universe.rs:540-614).
 template <int V>
 __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, Lane &B, bool evolution,
-                                          double a_add[3], double dLdt[3]) {
+                                          double a_add[3], double dLdt[3], SolveCache &sc, bool first) {
     constexpr int GRV = V & 3;
     constexpr bool EXT = (V & VAR_EXT) != 0;
     const LaneTests<V> LT(B);
@@ -864,7 +904,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
         // body) and the host's lag angle (row 3 of its column) for the host
         double F[3] = {0., 0., 0.};
         if (orbiting && (B.flags & F_DISK) && (B.flags & F_DISK_ROLE)) {
-            disk_force(E, lds, B, px, pv, d, nv2, F);
+            disk_force(E, lds, B, px, pv, d, nv2, F, sc, first);
 #pragma unroll
             for (int q = 0; q < 3; ++q) dk[q] = B.inv_m * F[q];
         }
@@ -1182,8 +1222,8 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
     // ---- the other GR implementations: accelerations only, added last ----
     if (GRV != GRV_KIDDER) {   // uniform: such a launch holds only systems of this variant
         double g[3];
-        if (GRV == GRV_ANDERSON) gr_anderson1975(lds, B, g);
-        else gr_newhall1983(lds, B, g);
+        if (GRV == GRV_ANDERSON) gr_anderson1975(lds, B, g, sc, first);
+        else gr_newhall1983(lds, B, g, sc, first);
         if (B.valid() && LT.gr) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) a_add[q] = a_add[q] + g[q];
@@ -1216,9 +1256,10 @@ __device__ inline void integrate_velocity_dependent_forces(const DevEnsemble &E,
 #pragma unroll
     for (int q = 0; q < 3; ++q) { v_orig[q] = B.v[q]; L_orig[q] = B.L[q]; }
     bool converged = false;
+    SolveCache sc;
     for (int it = 0; it < MIDPOINT_MAX_ITER; ++it) {
         double a_add[3], dLdt[3];
-        additional_effects<V>(E, lds, B, evolution && it == 0, a_add, dLdt);
+        additional_effects<V>(E, lds, B, evolution && it == 0, a_add, dLdt, sc, it == 0);
         double pdv = 0., pdL = 0.;   // |change of the final state|^2 of this body
         double fv2 = 0., fL2 = 0.;   // |final state|^2 of this body
 #pragma unroll
