@@ -94,7 +94,8 @@ __device__ __forceinline__ V3 ld3(const double a[3]) { return V3{a[0], a[1], a[2
 __device__ __forceinline__ void st3(double a[3], V3 v) { a[0] = v.x; a[1] = v.y; a[2] = v.z; }
 
 // Sums over the bodies of the group (order is irrelevant for the adjoint).
-__device__ __forceinline__ V3 gsum3(const AdjLds &L, const AdjLane &A, int row, bool skip_host) {
+template <class Lds>
+__device__ __forceinline__ V3 gsum3(const Lds &L, const AdjLane &A, int row, bool skip_host) {
     V3 s{0., 0., 0.};
     for (int j = 0; j < A.n; ++j) {
         if (skip_host && j == A.host) continue;
@@ -103,7 +104,8 @@ __device__ __forceinline__ V3 gsum3(const AdjLds &L, const AdjLane &A, int row, 
     }
     return s;
 }
-__device__ __forceinline__ V3 gsum3m(const AdjLds &L, const AdjLane &A, int row, bool skip_host) {
+template <class Lds>
+__device__ __forceinline__ V3 gsum3m(const Lds &L, const AdjLane &A, int row, bool skip_host) {
     V3 s{0., 0., 0.};
     for (int j = 0; j < A.n; ++j) {
         if (skip_host && j == A.host) continue;
@@ -113,16 +115,27 @@ __device__ __forceinline__ V3 gsum3m(const AdjLds &L, const AdjLane &A, int row,
     }
     return s;
 }
-__device__ __forceinline__ void put3(AdjLds &L, int row, int lane, V3 v) {
+template <class Lds>
+__device__ __forceinline__ void put3(Lds &L, int row, int lane, V3 v) {
     L.xb[row][lane] = v.x; L.xb[row + 1][lane] = v.y; L.xb[row + 2][lane] = v.z;
 }
-__device__ __forceinline__ V3 get3(const AdjLds &L, int row, int lane) {
+template <class Lds>
+__device__ __forceinline__ V3 get3(const Lds &L, int row, int lane) {
     return V3{L.xb[row][lane], L.xb[row + 1][lane], L.xb[row + 2][lane]};
 }
 // Position of body j in the chain of the Jacobi recurrences (whfast.rs:889-933):
 // the host first, then the other bodies in index order.
 __device__ __forceinline__ int chain_of(const AdjLane &A, int j) {
     return j == A.host ? 0 : (j < A.host ? j + 1 : j);
+}
+
+// Transpose Jacobian with respect to its spin W of a body's own wind torque
+// (wind.rs:61-91), -k W f shape with f = wsat^2 once |W| reaches the
+// saturation and |W|^2 below it.
+__device__ __forceinline__ V3 wind_vjp(const AdjLane &A, V3 W, V3 mu_L) {
+    const double s2 = posadj::dot(W, W);
+    return sqrt(s2) >= A.wsat ? (-A.wk * A.wsat * A.wsat * A.wshape) * mu_L
+                              : (-A.wk * A.wshape) * (s2 * mu_L + (2. * posadj::dot(W, mu_L)) * W);
 }
 
 // One pass of the effects' vector-Jacobian product at the linearisation
@@ -173,14 +186,7 @@ __device__ inline void effects_vjp_pass(AdjLds &L, const AdjLane &A, const posad
         }
     }
     if (A.wind) {
-        // this body's own wind torque (wind.rs:61-91), -k W f shape with
-        // f = wsat^2 once |W| reaches the saturation and |W|^2 below it:
-        // its transpose Jacobian with respect to W, then W = L / I
-        const V3 W = in.Wp;
-        const double s2 = posadj::dot(W, W);
-        const V3 dW = sqrt(s2) >= A.wsat ? (-A.wk * A.wsat * A.wsat * A.wshape) * mu_L
-                                         : (-A.wk * A.wshape) * (s2 * mu_L + (2. * posadj::dot(W, mu_L)) * W);
-        gL = gL + (1. / A.I) * dW;
+        gL = gL + (1. / A.I) * wind_vjp(A, in.Wp, mu_L);
     }
     wsync();
 }
@@ -202,11 +208,16 @@ __device__ __forceinline__ bool settled(V3 a, V3 b) {
     return maxabs3(a - b) <= ADJ_FIXED_POINT_TOL * maxabs3(a);
 }
 
-// Adjoint of one implicit-midpoint kick (x fixed, y = (v, L), half step h):
-// on entry A.lv / A.lL are the cotangents of y1 and A.lx that of x; on exit
-// A.lv / A.lL are those of y0, A.lx has the kick's contribution added and the
-// parameter gradients are accumulated.
-__device__ inline void kick_adjoint(AdjLds &L, AdjLane &A, V3 x, V3 v0, V3 L0, V3 v1, V3 L1, double h) {
+// Linearisation point of a kick at positions x between (v0, L0) and (v1, L1):
+// the pair's constants, parameters and midpoint state of an orbiting body, and
+// every body's midpoint spin in in.Wp (which the wind torque uses).
+struct KickPoint {
+    posadj::PairConst C;
+    posadj::PairPar P;
+    posadj::PairIn in;
+};
+template <class Lds>
+__device__ inline KickPoint kick_point(Lds &L, const AdjLane &A, V3 x, V3 v0, V3 L0, V3 v1, V3 L1) {
     const int lane = A.lane;
     const V3 vm = 0.5 * (v0 + v1);
     const V3 Lm = A.spin ? 0.5 * (L0 + L1) : L0;
@@ -214,14 +225,27 @@ __device__ inline void kick_adjoint(AdjLds &L, AdjLane &A, V3 x, V3 v0, V3 L0, V
     if (A.valid) { put3(L, 0, lane, x); put3(L, 3, lane, vm); put3(L, 6, lane, W); }
     wsync();
     const int hl = A.hl();
-    const posadj::PairConst C{A.mh, A.m, L.R[hl], A.R, A.Ih, A.I, A.tides, A.flat, A.gr};
-    const posadj::PairPar P{L.sg[hl], A.sg, L.k2[hl], A.k2, L.kf[hl], A.kf};
-    posadj::PairIn in{V3{0., 0., 0.}, V3{0., 0., 0.}, V3{0., 0., 0.}, W};
+    KickPoint K{posadj::PairConst{A.mh, A.m, L.R[hl], A.R, A.Ih, A.I, A.tides, A.flat, A.gr},
+                posadj::PairPar{L.sg[hl], A.sg, L.k2[hl], A.k2, L.kf[hl], A.kf},
+                posadj::PairIn{V3{0., 0., 0.}, V3{0., 0., 0.}, V3{0., 0., 0.}, W}};
     if (A.orbiting()) {
-        in.r = x - get3(L, 0, hl);
-        in.u = vm - get3(L, 3, hl);
-        in.Wh = get3(L, 6, hl);
+        K.in.r = x - get3(L, 0, hl);
+        K.in.u = vm - get3(L, 3, hl);
+        K.in.Wh = get3(L, 6, hl);
     }
+    return K;
+}
+
+// Adjoint of one implicit-midpoint kick (x fixed, y = (v, L), half step h):
+// on entry A.lv / A.lL are the cotangents of y1 and A.lx that of x; on exit
+// A.lv / A.lL are those of y0, A.lx has the kick's contribution added and the
+// parameter gradients are accumulated.
+__device__ inline void kick_adjoint(AdjLds &L, AdjLane &A, V3 x, V3 v0, V3 L0, V3 v1, V3 L1, double h) {
+    const int lane = A.lane;
+    const KickPoint K = kick_point(L, A, x, v0, L0, v1, L1);
+    const posadj::PairConst &C = K.C;
+    const posadj::PairPar &P = K.P;
+    const posadj::PairIn &in = K.in;
     const V3 lam_v = ld3(A.lv), lam_L = ld3(A.lL);
     const V3 z{0., 0., 0.};
     V3 gx, gv, gL;
@@ -270,14 +294,105 @@ __device__ __forceinline__ V3 tape3(const TapeRef &T, int row, int field, int bo
 // start.  The host's moment of inertia is read back after the next wsync.
 // EVO: the launch holds systems with evolution tables (without them the
 // reads are compiled out).
-template <bool EVO>
-__device__ __forceinline__ void step_radii(const TapeRef &T, AdjLds &L, AdjLane &A, int row) {
+template <bool EVO, class Lds>
+__device__ __forceinline__ void step_radii(const TapeRef &T, Lds &L, AdjLane &A, int row) {
     if (!(EVO && A.valid && A.evolving)) return;
     A.R = *T.at(row, TP_R, A.body);
     A.I = *T.at(row, TP_I, A.body);
     L.R[A.lane] = A.R;
     L.I[A.lane] = A.I;
     if (A.wind) A.wshape = sqrt(A.R / R_SUN * 1. / A.m);
+}
+
+// One step's tape: the states at its ends and after its first kick, and the
+// universal anomalies of its drifts.
+struct StepTape {
+    V3 x0, v0, L0, v1, L1, x2, v2, L2;
+    double X1, X2;
+};
+__device__ __forceinline__ StepTape step_tape(const TapeRef &T, const AdjLane &A, int row) {
+    const V3 z{0., 0., 0.};
+    StepTape S{z, z, z, z, z, z, z, z, 0., 0.};
+    const int b = A.body;
+    if (A.valid) {
+        S.x0 = tape3(T, row, TP_X, b); S.v0 = tape3(T, row, TP_V, b); S.L0 = tape3(T, row, TP_L, b);
+        S.v1 = tape3(T, row, TP_V1, b); S.L1 = tape3(T, row, TP_L1, b);
+        S.X1 = *T.at(row, TP_XK1, b); S.X2 = *T.at(row, TP_XK2, b);
+        S.x2 = tape3(T, row + 1, TP_X, b); S.v2 = tape3(T, row + 1, TP_V, b); S.L2 = tape3(T, row + 1, TP_L, b);
+    }
+    return S;
+}
+
+// Linearisation points of a step's drifts and interaction: the two Kepler
+// drifts' initial states (Q, P) and Stiefel functions, the positions of the
+// interaction, and the velocities before the second kick.
+struct DriftPoint {
+    V3 Q0, P0, Q2, P1pp, xg, v2p;
+    double g1[6], g2[6];
+};
+
+// The drift and interaction of one step recomputed from the tape, in democratic
+// heliocentric coordinates or, with WHDS, in WHDS coordinates.
+template <bool EVO, bool WHDS, class Lds>
+__device__ inline DriftPoint drift_point(Lds &L, AdjLane &A, const StepTape &S) {
+    const int lane = A.lane;
+    const V3 z{0., 0., 0.};
+    const double h = 0.5 * A.dt, dt = A.dt;
+    const double mu = posadj::G_K2 * (WHDS ? A.mh + A.m : A.mh);
+    const bool orb = A.orbiting();
+    const int hl = A.hl();
+    DriftPoint D{z, z, z, z, z, z, {}, {}};
+    if (A.valid) { put3(L, 0, lane, S.x0); put3(L, 3, lane, S.v1); }
+    wsync();
+    if (EVO && A.evolving) A.Ih = L.I[hl];   // the host's moment of inertia of this step
+    const V3 Xc = (1. / A.M) * gsum3m(L, A, 0, false);
+    const V3 V = (1. / A.M) * gsum3m(L, A, 3, false);
+    D.Q0 = orb ? S.x0 - get3(L, 0, hl) : z;
+    D.P0 = orb ? (WHDS ? A.fv * (S.v1 - V) : S.v1 - V) : z;
+    wsync();
+    V3 Q1 = z, P1 = z;
+    if (orb) posadj::kepler_forward_g(mu, h, S.X1, D.Q0, D.P0, Q1, P1, D.g1);
+    const V3 Xc1 = Xc + h * V;
+    if (orb) put3(L, 0, lane, WHDS ? A.wj * P1 : P1);
+    wsync();
+    const V3 Q1p = !orb ? z
+                 : WHDS ? Q1 + h * (gsum3(L, A, 0, true) - A.wj * P1)
+                        : Q1 + (h / A.mh) * gsum3m(L, A, 0, true);
+    wsync();
+    if (orb) put3(L, 0, lane, Q1p);
+    wsync();
+    const V3 xh = Xc1 - (1. / A.M) * gsum3m(L, A, 0, true);
+    D.xg = orb ? Q1p + xh : xh;
+    wsync();
+    if (A.valid) put3(L, 0, lane, D.xg);
+    wsync();
+    V3 acc = z;
+    if (orb) {
+        for (int j = 0; j < A.n; ++j) {
+            if (j == A.host || j == A.k) continue;
+            const int l = A.gbase + j;
+            const V3 d = D.xg - get3(L, 0, l);
+            const double d2 = posadj::dot(d, d);
+            const double id = 1. / sqrt(d2);
+            acc += (-posadj::G_K2 * L.m[l] * id * id * id) * d;
+        }
+    }
+    D.P1pp = P1 + (WHDS ? dt * A.fv : dt) * acc;
+    wsync();
+    if (orb) put3(L, 0, lane, WHDS ? A.wj * D.P1pp : D.P1pp);
+    wsync();
+    D.Q2 = !orb ? z
+                : WHDS ? Q1p + h * (gsum3(L, A, 0, true) - A.wj * D.P1pp)
+                       : Q1p + (h / A.mh) * gsum3m(L, A, 0, true);
+    V3 Q3 = z, P3 = z;
+    if (orb) posadj::kepler_forward_g(mu, h, S.X2, D.Q2, D.P1pp, Q3, P3, D.g2);
+    wsync();
+    if (orb) put3(L, 0, lane, WHDS ? A.wj * P3 : P3);
+    wsync();
+    D.v2p = WHDS ? (orb ? (1. / A.fv) * P3 + V : V - gsum3(L, A, 0, true))
+                        : (orb ? P3 + V : V - (1. / A.mh) * gsum3m(L, A, 0, true));
+    wsync();
+    return D;
 }
 
 // Reverse of step `row` of the segment for democratic heliocentric
@@ -289,79 +404,18 @@ __device__ __forceinline__ void step_radii(const TapeRef &T, AdjLds &L, AdjLane 
 // state after the step on entry and before it on exit.
 template <bool EVO, bool WHDS>
 __device__ inline void adjoint_step(const AdjArgs &Ar, AdjLds &L, AdjLane &A, int row) {
-    const TapeRef &T = Ar.T;
     const int lane = A.lane;
-    const int b = A.body;
     const V3 z{0., 0., 0.};
-    V3 x0 = z, v0 = z, L0 = z, v1 = z, L1 = z, x2 = z, v2 = z, L2 = z;
-    double X1 = 0., X2 = 0.;
-    if (A.valid) {
-        x0 = tape3(T, row, TP_X, b); v0 = tape3(T, row, TP_V, b); L0 = tape3(T, row, TP_L, b);
-        v1 = tape3(T, row, TP_V1, b); L1 = tape3(T, row, TP_L1, b);
-        X1 = *T.at(row, TP_XK1, b); X2 = *T.at(row, TP_XK2, b);
-        x2 = tape3(T, row + 1, TP_X, b); v2 = tape3(T, row + 1, TP_V, b); L2 = tape3(T, row + 1, TP_L, b);
-    }
-    step_radii<EVO>(T, L, A, row);
+    const StepTape S = step_tape(Ar.T, A, row);
+    step_radii<EVO>(Ar.T, L, A, row);
     const double h = 0.5 * A.dt, dt = A.dt;
     const double mu = posadj::G_K2 * (WHDS ? A.mh + A.m : A.mh);
     const bool orb = A.orbiting();
     const int hl = A.hl();
+    const DriftPoint D = drift_point<EVO, WHDS>(L, A, S);
 
-    // ---------------- recompute the drift from (x0, v1) ----------------
-    if (A.valid) { put3(L, 0, lane, x0); put3(L, 3, lane, v1); }
-    wsync();
-    if (EVO && A.evolving) A.Ih = L.I[hl];   // the host's moment of inertia of this step
-    const V3 Xc = (1. / A.M) * gsum3m(L, A, 0, false);
-    const V3 V = (1. / A.M) * gsum3m(L, A, 3, false);
-    const V3 Q0 = orb ? x0 - get3(L, 0, hl) : z;
-    const V3 P0 = orb ? (WHDS ? A.fv * (v1 - V) : v1 - V) : z;
-    wsync();
-    V3 Q1 = z, P1 = z;
-    if (orb) posadj::kepler_forward_x(mu, h, X1, Q0, P0, Q1, P1);
-    const V3 Xc1 = Xc + h * V;
-    if (orb) put3(L, 0, lane, WHDS ? A.wj * P1 : P1);
-    wsync();
-    const V3 Q1p = !orb ? z
-                 : WHDS ? Q1 + h * (gsum3(L, A, 0, true) - A.wj * P1)
-                        : Q1 + (h / A.mh) * gsum3m(L, A, 0, true);
-    wsync();
-    if (orb) put3(L, 0, lane, Q1p);
-    wsync();
-    const V3 xh = Xc1 - (1. / A.M) * gsum3m(L, A, 0, true);
-    const V3 xg = orb ? Q1p + xh : xh;
-    wsync();
-    if (A.valid) put3(L, 0, lane, xg);
-    wsync();
-    V3 acc = z;
-    if (orb) {
-        for (int j = 0; j < A.n; ++j) {
-            if (j == A.host || j == A.k) continue;
-            const int l = A.gbase + j;
-            const V3 d = xg - get3(L, 0, l);
-            const double d2 = posadj::dot(d, d);
-            const double id = 1. / sqrt(d2);
-            acc += (-posadj::G_K2 * L.m[l] * id * id * id) * d;
-        }
-    }
-    const V3 P1pp = P1 + (WHDS ? dt * A.fv : dt) * acc;
-    wsync();
-    if (orb) put3(L, 0, lane, WHDS ? A.wj * P1pp : P1pp);
-    wsync();
-    const V3 Q2 = !orb ? z
-                : WHDS ? Q1p + h * (gsum3(L, A, 0, true) - A.wj * P1pp)
-                       : Q1p + (h / A.mh) * gsum3m(L, A, 0, true);
-    V3 Q3 = z, P3 = z;
-    if (orb) posadj::kepler_forward_x(mu, h, X2, Q2, P1pp, Q3, P3);
-    wsync();
-    if (orb) put3(L, 0, lane, WHDS ? A.wj * P3 : P3);
-    wsync();
-    const V3 v2p = WHDS ? (orb ? (1. / A.fv) * P3 + V : V - gsum3(L, A, 0, true))
-                        : (orb ? P3 + V : V - (1. / A.mh) * gsum3m(L, A, 0, true));
-    wsync();
-
-    // ---------------- reverse ----------------
     // second kick (at x2, between (v2', L1) and (v2, L2))
-    kick_adjoint(L, A, x2, v2p, L1, v2, L2, h);
+    kick_adjoint(L, A, S.x2, D.v2p, S.L1, S.v2, S.L2, h);
     // T^-1 of the second drift
     if (A.valid) { put3(L, 0, lane, ld3(A.lx)); put3(L, 3, lane, ld3(A.lv)); }
     wsync();
@@ -373,7 +427,7 @@ __device__ inline void adjoint_step(const AdjArgs &Ar, AdjLds &L, AdjLane &A, in
     wsync();
     // second Kepler drift and the centre-of-mass drift
     V3 Q2b = z, P1ppb = z;
-    if (orb) posadj::kepler_vjp(mu, h, X2, Q2, P1pp, Q3b, P3b, Q2b, P1ppb);
+    if (orb) posadj::kepler_vjp_g(mu, h, S.X2, D.Q2, D.P1pp, Q3b, P3b, Q2b, P1ppb, D.g2);
     V3 Xc1b = xh_tot;
     V3 Vb = Vb0 + h * xh_tot;
     // second jump
@@ -385,14 +439,14 @@ __device__ inline void adjoint_step(const AdjArgs &Ar, AdjLds &L, AdjLane &A, in
     // interaction and planet-planet gravity
     V3 P1b = P1ppb;
     const V3 ab = (WHDS ? dt * A.fv : dt) * P1ppb;
-    if (A.valid) { put3(L, 0, lane, orb ? ab : z); put3(L, 3, lane, xg); }
+    if (A.valid) { put3(L, 0, lane, orb ? ab : z); put3(L, 3, lane, D.xg); }
     wsync();
     V3 xgb = z;
     if (orb) {
         for (int j = 0; j < A.n; ++j) {
             if (j == A.host || j == A.k) continue;
             const int l = A.gbase + j;
-            const V3 d = xg - get3(L, 3, l);
+            const V3 d = D.xg - get3(L, 3, l);
             xgb += posadj::gravity_pair_vjp(L.m[l], d, ab) - posadj::gravity_pair_vjp(A.m, d, get3(L, 0, l));
         }
     }
@@ -411,7 +465,7 @@ __device__ inline void adjoint_step(const AdjArgs &Ar, AdjLds &L, AdjLane &A, in
     wsync();
     // first Kepler drift and the centre-of-mass drift
     V3 Q0b = z, P0b = z;
-    if (orb) posadj::kepler_vjp(mu, h, X1, Q0, P0, Q1pb, P1b, Q0b, P0b);
+    if (orb) posadj::kepler_vjp_g(mu, h, S.X1, D.Q0, D.P0, Q1pb, P1b, Q0b, P0b, D.g1);
     const V3 Xcb = Xc1b;
     Vb += h * Xc1b;
     // T of the first drift
@@ -426,12 +480,13 @@ __device__ inline void adjoint_step(const AdjArgs &Ar, AdjLds &L, AdjLane &A, in
     }
     wsync();
     // first kick (at x0, between (v0, L0) and (v1, L1))
-    kick_adjoint(L, A, x0, v0, L0, v1, L1, h);
+    kick_adjoint(L, A, S.x0, S.v0, S.L0, S.v1, S.L1, h);
 }
 
 // ---- sums over the chain of the Jacobi recurrences (rows of 3 values) ----
 // sum over the bodies before this one in the chain of m_j * row_j
-__device__ __forceinline__ V3 chain_before_m(const AdjLds &L, const AdjLane &A, int row) {
+template <class Lds>
+__device__ __forceinline__ V3 chain_before_m(const Lds &L, const AdjLane &A, int row) {
     V3 s{0., 0., 0.};
     for (int j = 0; j < A.n; ++j) {
         if (chain_of(A, j) >= A.chain) continue;
@@ -441,7 +496,8 @@ __device__ __forceinline__ V3 chain_before_m(const AdjLds &L, const AdjLane &A, 
     return s;
 }
 // sum over the bodies up to this one in the chain (itself included) of row_j
-__device__ __forceinline__ V3 chain_upto(const AdjLds &L, const AdjLane &A, int row) {
+template <class Lds>
+__device__ __forceinline__ V3 chain_upto(const Lds &L, const AdjLane &A, int row) {
     V3 s{0., 0., 0.};
     for (int j = 0; j < A.n; ++j) {
         if (chain_of(A, j) > A.chain) continue;
@@ -450,7 +506,8 @@ __device__ __forceinline__ V3 chain_upto(const AdjLds &L, const AdjLane &A, int 
     return s;
 }
 // sum over the non-host bodies from chain position c0 on of (m_j / eta_le_j) * row_j
-__device__ __forceinline__ V3 chain_from_w(const AdjLds &L, const AdjLane &A, int row, int c0) {
+template <class Lds>
+__device__ __forceinline__ V3 chain_from_w(const Lds &L, const AdjLane &A, int row, int c0) {
     V3 s{0., 0., 0.};
     for (int j = 0; j < A.n; ++j) {
         if (j == A.host || chain_of(A, j) < c0) continue;
@@ -460,7 +517,8 @@ __device__ __forceinline__ V3 chain_from_w(const AdjLds &L, const AdjLane &A, in
     return s;
 }
 // sum over the non-host bodies after this one in the chain of row_j / eta_lt_j
-__device__ __forceinline__ V3 chain_after_inv(const AdjLds &L, const AdjLane &A, int row) {
+template <class Lds>
+__device__ __forceinline__ V3 chain_after_inv(const Lds &L, const AdjLane &A, int row) {
     V3 s{0., 0., 0.};
     for (int j = 0; j < A.n; ++j) {
         if (j == A.host || chain_of(A, j) <= A.chain) continue;
@@ -468,6 +526,84 @@ __device__ __forceinline__ V3 chain_after_inv(const AdjLds &L, const AdjLane &A,
         s += (1. / (L.eta[l] - L.m[l])) * get3(L, row, l);
     }
     return s;
+}
+
+// The interaction's indirect term of the bodies after the first in the chain
+// (whfast.rs:955-962) adds r3 Q to the momentum of a body at Q; its transpose
+// Jacobian is r3 p - r5 (Q . p) Q.
+struct Indirect {
+    double r3, r5;
+};
+__device__ __forceinline__ Indirect indirect_term(const AdjLane &A, V3 Q) {
+    Indirect N{0., 0.};
+    if (A.orbiting() && A.chain > 1) {
+        const double r2 = posadj::dot(Q, Q) + 1e-12;
+        N.r3 = A.dt * posadj::G_K2 * A.eta_le * (1. / (r2 * sqrt(r2)));
+        N.r5 = 3. * N.r3 / r2;
+    }
+    return N;
+}
+
+// The drift and interaction of one step recomputed from the tape, in Jacobi
+// coordinates.
+template <bool EVO, class Lds>
+__device__ inline DriftPoint drift_point_jacobi(Lds &L, AdjLane &A, const StepTape &S) {
+    const int lane = A.lane;
+    const V3 z{0., 0., 0.};
+    const double h = 0.5 * A.dt, dt = A.dt;
+    const double mu = posadj::G_K2 * A.eta_le;
+    const bool orb = A.orbiting();
+    const int hl = A.hl();
+    const int first = A.host == 0 ? 1 : 0;   // index of the first body of the chain
+    DriftPoint D{z, z, z, z, z, z, {}, {}};
+    // to Jacobi coordinates from (S.x0, S.v1)
+    if (A.valid) { put3(L, 0, lane, S.x0); put3(L, 3, lane, S.v1); }
+    wsync();
+    if (EVO && A.evolving) A.Ih = L.I[hl];   // the host's moment of inertia of this step
+    const V3 com = (1. / A.M) * gsum3m(L, A, 0, false);
+    const V3 comv = (1. / A.M) * gsum3m(L, A, 3, false);
+    D.Q0 = orb ? S.x0 - (1. / A.eta_lt) * chain_before_m(L, A, 0) : z;
+    D.P0 = orb ? S.v1 - (1. / A.eta_lt) * chain_before_m(L, A, 3) : z;
+    wsync();
+    V3 Q1 = z, P1 = z;
+    if (orb) posadj::kepler_forward_g(mu, h, S.X1, D.Q0, D.P0, Q1, P1, D.g1);
+    const V3 com1 = com + h * comv;
+    // inertial positions of the interaction
+    if (A.valid) put3(L, 0, lane, Q1);
+    wsync();
+    D.xg = Q1 + com1 - chain_from_w(L, A, 0, orb ? A.chain : 1);
+    wsync();
+    // gravitational accelerations (the host / first-body pair left out)
+    if (A.valid) put3(L, 0, lane, D.xg);
+    wsync();
+    V3 acc = z;
+    if (A.valid) {
+        for (int j = 0; j < A.n; ++j) {
+            if (j == A.k) continue;
+            if ((A.k == A.host && j == first) || (j == A.host && A.k == first)) continue;
+            const int l = A.gbase + j;
+            const V3 d = D.xg - get3(L, 0, l);
+            const double d2 = posadj::dot(d, d);
+            const double id = 1. / sqrt(d2);
+            acc += (-posadj::G_K2 * L.m[l] * id * id * id) * d;
+        }
+    }
+    wsync();
+    if (A.valid) put3(L, 0, lane, acc);
+    wsync();
+    const V3 aj = orb ? acc - (1. / A.eta_lt) * chain_before_m(L, A, 0) : z;
+    wsync();
+    D.Q2 = Q1;
+    const Indirect N = indirect_term(A, Q1);
+    D.P1pp = orb ? P1 + dt * aj + N.r3 * Q1 : z;
+    V3 Q3 = z, P3 = z;
+    if (orb) posadj::kepler_forward_g(mu, h, S.X2, Q1, D.P1pp, Q3, P3, D.g2);
+    // velocities after the second drift in inertial coordinates
+    if (A.valid) put3(L, 0, lane, P3);
+    wsync();
+    D.v2p = P3 + comv - chain_from_w(L, A, 0, orb ? A.chain : 1);
+    wsync();
+    return D;
 }
 
 // Reverse of step `row` of the segment for a system in Jacobi coordinates
@@ -483,83 +619,18 @@ __device__ __forceinline__ V3 chain_after_inv(const AdjLds &L, const AdjLane &A,
 // and their vector-Jacobian products are the transposed sums.
 template <bool EVO>
 __device__ inline void adjoint_step_jacobi(const AdjArgs &Ar, AdjLds &L, AdjLane &A, int row) {
-    const TapeRef &T = Ar.T;
     const int lane = A.lane;
-    const int b = A.body;
     const V3 z{0., 0., 0.};
-    V3 x0 = z, v0 = z, L0 = z, v1 = z, L1 = z, x2 = z, v2 = z, L2 = z;
-    double X1 = 0., X2 = 0.;
-    if (A.valid) {
-        x0 = tape3(T, row, TP_X, b); v0 = tape3(T, row, TP_V, b); L0 = tape3(T, row, TP_L, b);
-        v1 = tape3(T, row, TP_V1, b); L1 = tape3(T, row, TP_L1, b);
-        X1 = *T.at(row, TP_XK1, b); X2 = *T.at(row, TP_XK2, b);
-        x2 = tape3(T, row + 1, TP_X, b); v2 = tape3(T, row + 1, TP_V, b); L2 = tape3(T, row + 1, TP_L, b);
-    }
-    step_radii<EVO>(T, L, A, row);
+    const StepTape S = step_tape(Ar.T, A, row);
+    step_radii<EVO>(Ar.T, L, A, row);
     const double h = 0.5 * A.dt, dt = A.dt;
     const double mu = posadj::G_K2 * A.eta_le;
     const bool orb = A.orbiting();
-    const int hl = A.hl();
-    const int rank = A.chain - 1;        // 0 for the first body of the chain
     const int first = A.host == 0 ? 1 : 0;   // index of the first body of the chain
+    const DriftPoint D = drift_point_jacobi<EVO>(L, A, S);
 
-    // ---------------- recompute the drifts and the interaction ----------------
-    // to Jacobi coordinates from (x0, v1)
-    if (A.valid) { put3(L, 0, lane, x0); put3(L, 3, lane, v1); }
-    wsync();
-    if (EVO && A.evolving) A.Ih = L.I[hl];   // the host's moment of inertia of this step
-    const V3 com = (1. / A.M) * gsum3m(L, A, 0, false);
-    const V3 comv = (1. / A.M) * gsum3m(L, A, 3, false);
-    const V3 Q0 = orb ? x0 - (1. / A.eta_lt) * chain_before_m(L, A, 0) : z;
-    const V3 P0 = orb ? v1 - (1. / A.eta_lt) * chain_before_m(L, A, 3) : z;
-    wsync();
-    V3 Q1 = z, P1 = z;
-    if (orb) posadj::kepler_forward_x(mu, h, X1, Q0, P0, Q1, P1);
-    const V3 com1 = com + h * comv;
-    // inertial positions of the interaction
-    if (A.valid) put3(L, 0, lane, Q1);
-    wsync();
-    const V3 xg = Q1 + com1 - chain_from_w(L, A, 0, orb ? A.chain : 1);
-    wsync();
-    // gravitational accelerations (the host / first-body pair left out)
-    if (A.valid) put3(L, 0, lane, xg);
-    wsync();
-    V3 acc = z;
-    if (A.valid) {
-        for (int j = 0; j < A.n; ++j) {
-            if (j == A.k) continue;
-            if ((A.k == A.host && j == first) || (j == A.host && A.k == first)) continue;
-            const int l = A.gbase + j;
-            const V3 d = xg - get3(L, 0, l);
-            const double d2 = posadj::dot(d, d);
-            const double id = 1. / sqrt(d2);
-            acc += (-posadj::G_K2 * L.m[l] * id * id * id) * d;
-        }
-    }
-    wsync();
-    if (A.valid) put3(L, 0, lane, acc);
-    wsync();
-    const V3 aj = orb ? acc - (1. / A.eta_lt) * chain_before_m(L, A, 0) : z;
-    wsync();
-    // the indirect term of the bodies after the first (whfast.rs:955-962)
-    double r2 = 1., r3i = 0.;
-    if (orb && rank > 0) {
-        r2 = posadj::dot(Q1, Q1) + 1e-12;
-        r3i = 1. / (r2 * sqrt(r2));
-    }
-    const double gk = dt * posadj::G_K2 * A.eta_le;
-    const V3 P1pp = orb ? P1 + dt * aj + (rank > 0 ? gk * r3i : 0.) * Q1 : z;
-    V3 Q3 = z, P3 = z;
-    if (orb) posadj::kepler_forward_x(mu, h, X2, Q1, P1pp, Q3, P3);
-    // velocities after the second drift in inertial coordinates
-    if (A.valid) put3(L, 0, lane, P3);
-    wsync();
-    const V3 v2p = P3 + comv - chain_from_w(L, A, 0, orb ? A.chain : 1);
-    wsync();
-
-    // ---------------- reverse ----------------
     // second kick (at x2, between (v2', L1) and (v2, L2))
-    kick_adjoint(L, A, x2, v2p, L1, v2, L2, h);
+    kick_adjoint(L, A, S.x2, D.v2p, S.L1, S.v2, S.L2, h);
     // back to inertial coordinates after the second drift
     if (A.valid) { put3(L, 0, lane, ld3(A.lx)); put3(L, 3, lane, ld3(A.lv)); }
     wsync();
@@ -570,16 +641,17 @@ __device__ inline void adjoint_step_jacobi(const AdjArgs &Ar, AdjLds &L, AdjLane
     wsync();
     // second Kepler drift
     V3 Q1b = z, P1ppb = z;
-    if (orb) posadj::kepler_vjp(mu, h, X2, Q1, P1pp, Q3b, P3b, Q1b, P1ppb);
+    if (orb) posadj::kepler_vjp_g(mu, h, S.X2, D.Q2, D.P1pp, Q3b, P3b, Q1b, P1ppb, D.g2);
     // interaction: the indirect term and the Jacobi accelerations
     const V3 P1b = P1ppb;
-    if (orb && rank > 0) Q1b += (gk * r3i) * P1ppb - (3. * gk * r3i / r2 * posadj::dot(Q1, P1ppb)) * Q1;
+    const Indirect N = indirect_term(A, D.Q2);
+    Q1b += N.r3 * P1ppb - (N.r5 * posadj::dot(D.Q2, P1ppb)) * D.Q2;
     if (A.valid) put3(L, 0, lane, orb ? dt * P1ppb : z);
     wsync();
     const V3 accb = (orb ? dt * P1ppb : z) - A.m * chain_after_inv(L, A, 0);
     wsync();
     // gravity
-    if (A.valid) { put3(L, 0, lane, accb); put3(L, 3, lane, xg); }
+    if (A.valid) { put3(L, 0, lane, accb); put3(L, 3, lane, D.xg); }
     wsync();
     V3 xgb = z;
     if (A.valid) {
@@ -587,7 +659,7 @@ __device__ inline void adjoint_step_jacobi(const AdjArgs &Ar, AdjLds &L, AdjLane
             if (j == A.k) continue;
             if ((A.k == A.host && j == first) || (j == A.host && A.k == first)) continue;
             const int l = A.gbase + j;
-            const V3 d = xg - get3(L, 3, l);
+            const V3 d = D.xg - get3(L, 3, l);
             xgb += posadj::gravity_pair_vjp(L.m[l], d, accb) - posadj::gravity_pair_vjp(A.m, d, get3(L, 0, l));
         }
     }
@@ -600,7 +672,7 @@ __device__ inline void adjoint_step_jacobi(const AdjArgs &Ar, AdjLds &L, AdjLane
     wsync();
     // first Kepler drift (com1 = com + h comv)
     V3 Q0b = z, P0b = z;
-    if (orb) posadj::kepler_vjp(mu, h, X1, Q0, P0, Q1b, P1b, Q0b, P0b);
+    if (orb) posadj::kepler_vjp_g(mu, h, S.X1, D.Q0, D.P0, Q1b, P1b, Q0b, P0b, D.g1);
     comvb += h * com1b;
     // to Jacobi coordinates from (x0, v1)
     if (A.valid) { put3(L, 0, lane, Q0b); put3(L, 3, lane, P0b); }
@@ -611,10 +683,11 @@ __device__ inline void adjoint_step_jacobi(const AdjArgs &Ar, AdjLds &L, AdjLane
     }
     wsync();
     // first kick (at x0, between (v0, L0) and (v1, L1))
-    kick_adjoint(L, A, x0, v0, L0, v1, L1, h);
+    kick_adjoint(L, A, S.x0, S.v0, S.L0, S.v1, S.L1, h);
 }
 
-__device__ inline void adjoint_load(const AdjArgs &Ar, AdjLds &L, AdjLane &A, int wave) {
+template <class Lds>
+__device__ inline void adjoint_load(const AdjArgs &Ar, Lds &L, AdjLane &A, int wave) {
     const DevEnsemble &E = Ar.E;
     const int lane = threadIdx.x;
     const LaneGroup lg = lane_group(E, wave, lane);

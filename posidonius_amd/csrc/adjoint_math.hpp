@@ -389,14 +389,22 @@ POS_HD void stiefel_g05(double beta, double X, double g[6]) {
     double c[6];
     if (fabs(z) < 1.) {
         // c_k(z) = sum_j (-z)^j / (k + 2j)! for k = 4, 5 (12 terms: the
-        // remainder is below 1/28! for |z| < 1), then c_k = 1/k! - z c_{k+2}
-        // downwards, which only multiplies by |z| < 1.
-        double t4 = 1. / 24., t5 = 1. / 120., s4 = 0., s5 = 0.;
-        for (int j = 0; j < 12; ++j) {
-            s4 += t4;
-            s5 += t5;
-            t4 *= -z / ((double)(5 + 2 * j) * (double)(6 + 2 * j));
-            t5 *= -z / ((double)(6 + 2 * j) * (double)(7 + 2 * j));
+        // remainder is below 1/28! for |z| < 1) by Horner's rule with the
+        // reciprocal factorials (dividing term by term cost 24 divisions in
+        // two chains), then c_k = 1/k! - z c_{k+2} downwards, which only
+        // multiplies by |z| < 1.
+        constexpr double F[24] = {   // 1 / k! for k = 4..27
+            1. / 24., 1. / 120., 1. / 720., 1. / 5040., 1. / 40320., 1. / 362880., 1. / 3628800., 1. / 39916800.,
+            1. / 479001600., 1. / 6227020800., 1. / 87178291200., 1. / 1307674368000., 1. / 20922789888000.,
+            1. / 355687428096000., 1. / 6402373705728000., 1. / 121645100408832000., 1. / 2432902008176640000.,
+            1. / 51090942171709440000., 1. / 1124000727777607680000., 1. / 25852016738884976640000.,
+            1. / 620448401733239439360000., 1. / 15511210043330985984000000., 1. / 403291461126605635584000000.,
+            1. / 10888869450418352160768000000.};
+        double s4 = F[22], s5 = F[23];
+#pragma unroll
+        for (int j = 20; j >= 0; j -= 2) {
+            s4 = F[j] - z * s4;
+            s5 = F[j + 1] - z * s5;
         }
         c[4] = s4;
         c[5] = s5;
@@ -430,19 +438,24 @@ POS_HD void stiefel_g05(double beta, double X, double g[6]) {
 
 // One drift of a body (position x0, velocity v0 relative to a centre of
 // gravitational parameter mu) over dt, for a given converged X.
-POS_HD void kepler_forward_x(double mu, double dt, double X, V3 x0, V3 v0, V3 &x1, V3 &v1) {
+// Returns the Stiefel functions in g.
+POS_HD void kepler_forward_g(double mu, double dt, double X, V3 x0, V3 v0, V3 &x1, V3 &v1, double g[6]) {
     const double r0 = sqrt(dot(x0, x0));
     const double v2 = dot(v0, v0);
     const double beta = 2. * mu / r0 - v2;
     const double eta0 = dot(x0, v0);
     const double zeta0 = mu - beta * r0;
-    double g[6];
     stiefel_g05(beta, X, g);
     const double r = r0 + eta0 * g[1] + zeta0 * g[2];
     const double f = -mu * g[2] / r0, gg = dt - mu * g[3];
     const double fd = -mu * g[1] / (r0 * r), gd = -mu * g[2] / r;
     x1 = x0 + f * x0 + gg * v0;
     v1 = v0 + fd * x0 + gd * v0;
+}
+
+POS_HD void kepler_forward_x(double mu, double dt, double X, V3 x0, V3 v0, V3 &x1, V3 &v1) {
+    double g[6];
+    kepler_forward_g(mu, dt, X, x0, v0, x1, v1, g);
 }
 
 // Residual of the universal Kepler equation, r0 X + eta0 G2 + zeta0 G3 - dt.
@@ -456,15 +469,15 @@ POS_HD double kepler_residual(double mu, double dt, double X, V3 x0, V3 v0) {
 
 // Vector-Jacobian product of the drift, X being the solution of the
 // universal Kepler equation (implicit differentiation): accumulates the
-// cotangents of x0, v0 from those of x1, v1.
-POS_HD void kepler_vjp(double mu, double dt, double X, V3 x0, V3 v0, V3 x1b, V3 v1b, V3 &x0b, V3 &v0b) {
+// cotangents of x0, v0 from those of x1, v1; g holds the drift's Stiefel
+// functions.
+POS_HD void kepler_vjp_g(double mu, double dt, double X, V3 x0, V3 v0, V3 x1b, V3 v1b, V3 &x0b, V3 &v0b,
+                         const double g[6]) {
     const double r0 = sqrt(dot(x0, x0));
     const double v2 = dot(v0, v0);
     const double beta = 2. * mu / r0 - v2;
     const double eta0 = dot(x0, v0);
     const double zeta0 = mu - beta * r0;
-    double g[6];
-    stiefel_g05(beta, X, g);
     const double r = r0 + eta0 * g[1] + zeta0 * g[2];
     const double f = -mu * g[2] / r0, gg = dt - mu * g[3];
     const double fd = -mu * g[1] / (r0 * r), gd = -mu * g[2] / r;
@@ -511,6 +524,13 @@ POS_HD void kepler_vjp(double mu, double dt, double X, V3 x0, V3 v0, V3 x1b, V3 
     xb += (r0_b / r0) * x0;
     x0b += xb;
     v0b += vb;
+}
+
+POS_HD void kepler_vjp(double mu, double dt, double X, V3 x0, V3 v0, V3 x1b, V3 v1b, V3 &x0b, V3 &v0b) {
+    const double r0 = sqrt(dot(x0, x0));
+    double g[6];
+    stiefel_g05(2. * mu / r0 - dot(v0, v0), X, g);
+    kepler_vjp_g(mu, dt, X, x0, v0, x1b, v1b, x0b, v0b, g);
 }
 
 // ---------------------------------------------------------------------------

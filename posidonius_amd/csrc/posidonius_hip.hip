@@ -22,6 +22,7 @@
 #include "whfast_step.hpp"
 #include "whfast_fixed.hpp"
 #include "adjoint_kernels.hpp"
+#include "adjoint_sweep.hpp"
 
 #ifndef POS_WAVES_PER_EU
 #define POS_WAVES_PER_EU 2   // occupancy target of the step kernel (waves per SIMD)
@@ -271,6 +272,26 @@ __global__ __launch_bounds__(64) void adjoint_segment_kernel(AdjArgs Ar) {
     }
 }
 
+// The coefficients of steps [row0, row0 + len) of the recorded segment: one
+// wavefront per set of systems, step and part of the step.
+template <bool ALT, bool EVO>
+__global__ __launch_bounds__(64) void adjoint_prepare_kernel(AdjArgs Ar, Coefficients Cf, int row0, int len, int slots) {
+    __shared__ PrepareLds L;
+    const int part = blockIdx.x / Ar.E.n_waves, t = part >> 1;
+    if (t >= len) return;
+    AdjLane A;
+    adjoint_load(Ar, L, A, blockIdx.x - part * Ar.E.n_waves);
+    if (Ar.seg_start + row0 + t < A.done) prepare_step<ALT, EVO>(Ar, L, A, Cf, row0 + t, t, slots, part & 1);
+}
+
+// Reverse sweep over those steps, last step first: 16 / NM systems per wavefront.
+template <int NM, bool ALT>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
+void adjoint_sweep_kernel(AdjArgs Ar, Coefficients Cf, int row0, int len) {
+    __shared__ SweepLds S;
+    sweep_stretch<NM, ALT>(Ar, S, Cf, row0, len);
+}
+
 // initialize_physical_values (whfast.rs:226-233) for systems at t == 0:
 // evolution at t, then spin = L / I.
 __global__ __launch_bounds__(64) void init_kernel(DevEnsemble E) {
@@ -511,6 +532,10 @@ struct pos_ens {
         hipEvent_t recorded_ev[2] = {nullptr, nullptr}, swept_ev[2] = {nullptr, nullptr};
         long long *iter0 = nullptr, *steps_done = nullptr;
         double *lx = nullptr, *lv = nullptr, *lL = nullptr, *gs = nullptr, *gk2 = nullptr, *gkf = nullptr;
+        // the prepared sweep's coefficients of `stretch` steps, systems of at
+        // most `slots` bodies; none: the sweep in one kernel
+        double2 *coef = nullptr;
+        int stretch = 0, slots = 0;
         std::vector<void *> allocs;
     } adj;
 };
@@ -951,6 +976,63 @@ void adjoint_release(pos_ens *h) {
     }
     if (A.sweep) (void)hipStreamDestroy(A.sweep);
     A = pos_ens::Adjoint();
+}
+
+// The prepared sweep's workspace, if this ensemble is one it serves better: up to
+// one set of systems per CU.  The whole adjoint of 32 steps took, in one kernel
+// and prepared, us a step: 128 sets of four bodies each 66.9 and 44.8, 256 sets
+// 70.2 and 59.9, 384 sets 76.1 and 83.3; of 2 to 12 bodies 118 sets 96.5 and
+// 69.2, 243 sets 101.7 and 100.8, 487 sets 117 and 170.  The workspace is
+// bounded, a segment is swept by stretches of the steps that fit; without
+// memory for a single one the sweep is the one kernel's.
+constexpr int PREPARED_SETS_PER_CU = 1;
+constexpr size_t COEFFICIENT_BYTES = (size_t)256 << 20;
+void plan_prepared_sweep(pos_ens *h, int seg) {
+    pos_ens::Adjoint &A = h->adj;
+    if (h->E.n_waves > PREPARED_SETS_PER_CU * h->n_cus) return;
+    int max_n = 0;
+    for (int s = 0; s < h->n_systems; ++s) max_n = std::max(max_n, h->body_offset_dev[s + 1] - h->body_offset_dev[s]);
+    const int slots = max_n <= 4 ? 4 : max_n <= 8 ? 8 : 16;
+    const size_t step_bytes = (size_t)coefficient_planes(slots) * h->n_bodies * sizeof(double2);
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) { (void)hipGetLastError(); return; }
+    const size_t stretch = std::min<size_t>(seg, std::min(COEFFICIENT_BYTES, free_b / 4) / step_bytes);
+    if (stretch == 0) return;
+    void *q = nullptr;
+    if (hipMalloc(&q, stretch * step_bytes) != hipSuccess) { (void)hipGetLastError(); return; }
+    A.allocs.push_back(q);
+    A.coef = (double2 *)q;
+    A.stretch = (int)stretch;
+    A.slots = slots;
+}
+
+// One segment's sweep on the adjoint's stream, last step first.
+int launch_sweep(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo) {
+    const pos_ens::Adjoint &A = h->adj;
+    if (!A.coef) {
+        auto kernel = alt ? (evo ? adjoint_segment_kernel<true, true> : adjoint_segment_kernel<true, false>)
+                          : (evo ? adjoint_segment_kernel<false, true> : adjoint_segment_kernel<false, false>);
+        hipLaunchKernelGGL(kernel, dim3(h->grid), dim3(64), 0, A.sweep, Ar);
+        HIP_TRY(hipGetLastError());
+        return POS_OK;
+    }
+    const Coefficients Cf{A.coef, coefficient_planes(A.slots), h->n_bodies};
+    auto prepare = alt ? (evo ? adjoint_prepare_kernel<true, true> : adjoint_prepare_kernel<true, false>)
+                       : (evo ? adjoint_prepare_kernel<false, true> : adjoint_prepare_kernel<false, false>);
+    auto sweep = A.slots == 4 ? (alt ? adjoint_sweep_kernel<4, true> : adjoint_sweep_kernel<4, false>)
+               : A.slots == 8 ? (alt ? adjoint_sweep_kernel<8, true> : adjoint_sweep_kernel<8, false>)
+                              : (alt ? adjoint_sweep_kernel<16, true> : adjoint_sweep_kernel<16, false>);
+    const int per_wave = 16 / A.slots;
+    for (int end = Ar.seg_len; end > 0;) {
+        const int len = std::min(A.stretch, end), row0 = end - len;
+        hipLaunchKernelGGL(prepare, dim3(2 * h->E.n_waves * len), dim3(64), 0, A.sweep, Ar, Cf, row0, len,
+                           A.slots);
+        HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(sweep, dim3((h->n_systems + per_wave - 1) / per_wave), dim3(64), 0, A.sweep, Ar, Cf, row0, len);
+        HIP_TRY(hipGetLastError());
+        end = row0;
+    }
+    return POS_OK;
 }
 
 // The mutable device state of an ensemble (what a checkpoint must hold).
@@ -1937,6 +2019,7 @@ int32_t pos_adjoint_record(pos_ens *h, int64_t n_steps, int32_t segment_steps) {
         (rc = aalloc((void **)&A.lL, 3 * nb * sizeof(double))) || (rc = aalloc((void **)&A.gs, nb * sizeof(double))) ||
         (rc = aalloc((void **)&A.gk2, nb * sizeof(double))) || (rc = aalloc((void **)&A.gkf, nb * sizeof(double))))
         return rc;
+    plan_prepared_sweep(h, seg);
     HIP_TRY(hipStreamCreateWithFlags(&A.sweep, hipStreamNonBlocking));
     for (int i = 0; i < 2; ++i) {
         HIP_TRY(hipEventCreateWithFlags(&A.recorded_ev[i], hipEventDisableTiming));
@@ -2029,8 +2112,6 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
                                  [](int c) { return c != POS_COORD_DEMOCRATIC_HELIOCENTRIC; });
     const bool evo = std::any_of(h->eff_dev.begin(), h->eff_dev.end(),
                                  [](uint32_t e) { return (e & POS_EFFECT_EVOLUTION) != 0; });
-    void (*sweep_kernel)(AdjArgs) = alt ? (evo ? adjoint_segment_kernel<true, true> : adjoint_segment_kernel<true, false>)
-                                    : (evo ? adjoint_segment_kernel<false, true> : adjoint_segment_kernel<false, false>);
     // the sweep stream must also see the seeds uploaded on the handle's stream
     HIP_TRY(hipEventRecord(A.swept_ev[0], h->stream));
     HIP_TRY(hipStreamWaitEvent(A.sweep, A.swept_ev[0], 0));
@@ -2041,9 +2122,7 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
         Ar.T = TapeRef{A.tape[buf], nb};
         Ar.seg_start = (int64_t)s * A.seg;
         Ar.seg_len = seg_len(s);
-        void *args[] = {&Ar};
-        HIP_TRY(hipLaunchKernel((const void *)sweep_kernel, dim3(h->grid), dim3(64), args, 0, A.sweep));
-        HIP_TRY(hipGetLastError());
+        if ((rc = launch_sweep(h, Ar, alt, evo))) return rc;
         HIP_TRY(hipEventRecord(A.swept_ev[buf], A.sweep));
         if (s > 0 && (rc = recompute(s - 1))) return rc;
     }
