@@ -430,6 +430,21 @@ __global__ __launch_bounds__(256) void read_fields_kernel(ReadTable t, char *__r
     }
 }
 
+// A checkpoint's fields, saved or restored in one launch: sixteen copies of a
+// small ensemble's fields took 5 us each and more in gaps.  blockIdx.y is the
+// field; addresses are multiples of 256 bytes, sizes of 4.
+constexpr int STATE_FIELDS = 16;
+struct StateCopy {
+    struct { const void *src; void *dst; size_t bytes; } f[STATE_FIELDS];
+};
+__global__ __launch_bounds__(256) void copy_state_kernel(StateCopy c) {
+    const auto f = c.f[blockIdx.y];
+    const size_t n16 = f.bytes / 16, first = blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = first; i < n16; i += (size_t)gridDim.x * 256) ((uint4 *)f.dst)[i] = ((const uint4 *)f.src)[i];
+    const size_t tail = n16 * 4 + first;
+    if (tail < f.bytes / 4) ((uint32_t *)f.dst)[tail] = ((const uint32_t *)f.src)[tail];
+}
+
 // The inverse of unpermute_kernel: caller order (comps per body) to device
 // order (component q of device body d at q * n + d).
 __global__ __launch_bounds__(256) void permute_kernel(const double *__restrict__ src, const int *__restrict__ perm, int n,
@@ -524,17 +539,25 @@ struct pos_ens {
     struct Adjoint {
         bool recorded = false;
         int64_t n_steps = 0;
-        int seg = 0, n_seg = 0;
+        int seg = 0, n_seg = 0, n_waves = 0;   // what the buffers are for (n_waves: of the launch table)
         size_t state_bytes = 0;
-        char *ckpt = nullptr;              // (n_seg + 1) states: segment starts, then the final state
-        double *tape[2] = {nullptr, nullptr};   // two segment tapes, (seg + 1) * TAPE_FIELDS * n_bodies each
+        char *final_state = nullptr;       // the last of ckpt
+        char *ckpt = nullptr;              // states: segment starts (unless every tape is kept), then the final one
+        // segment tapes, (seg + 1) * TAPE_FIELDS * n_bodies each; segment s uses
+        // tape s % tapes, held[] tells whose rows a tape has
+        int tapes = 0;
+        double *tape = nullptr;
+        size_t tape_values = 0;
+        std::vector<int> held;
         hipStream_t sweep = nullptr;            // stream of the reverse sweeps
-        hipEvent_t recorded_ev[2] = {nullptr, nullptr}, swept_ev[2] = {nullptr, nullptr};
+        // of each of two tapes: its rows are there; its sweep has read them
+        hipEvent_t taped_ev[2] = {nullptr, nullptr}, swept_ev[2] = {nullptr, nullptr};
         long long *iter0 = nullptr, *steps_done = nullptr;
         double *lx = nullptr, *lv = nullptr, *lL = nullptr, *gs = nullptr, *gk2 = nullptr, *gkf = nullptr;
-        // the prepared sweep's coefficients of `stretch` steps, systems of at
-        // most `slots` bodies; none: the sweep in one kernel
+        // the prepared sweep's coefficients: two halves of `stretch` steps,
+        // systems of at most `slots` bodies; none: the sweep in one kernel
         double2 *coef = nullptr;
+        hipEvent_t prepared_ev[2] = {nullptr, nullptr}, spent_ev[2] = {nullptr, nullptr};   // of each half
         int stretch = 0, slots = 0;
         std::vector<void *> allocs;
     } adj;
@@ -970,69 +993,11 @@ double host_roche(double ma, double mb, double ra, double rb) {
 void adjoint_release(pos_ens *h) {
     pos_ens::Adjoint &A = h->adj;
     for (void *p : A.allocs) (void)hipFree(p);
-    for (int i = 0; i < 2; ++i) {
-        if (A.recorded_ev[i]) (void)hipEventDestroy(A.recorded_ev[i]);
-        if (A.swept_ev[i]) (void)hipEventDestroy(A.swept_ev[i]);
-    }
+    for (hipEvent_t *e : {A.taped_ev, A.swept_ev, A.prepared_ev, A.spent_ev})
+        for (int i = 0; i < 2; ++i)
+            if (e[i]) (void)hipEventDestroy(e[i]);
     if (A.sweep) (void)hipStreamDestroy(A.sweep);
     A = pos_ens::Adjoint();
-}
-
-// The prepared sweep's workspace, if this ensemble is one it serves better: up to
-// one set of systems per CU.  The whole adjoint of 32 steps took, in one kernel
-// and prepared, us a step: 128 sets of four bodies each 66.9 and 44.8, 256 sets
-// 70.2 and 59.9, 384 sets 76.1 and 83.3; of 2 to 12 bodies 118 sets 96.5 and
-// 69.2, 243 sets 101.7 and 100.8, 487 sets 117 and 170.  The workspace is
-// bounded, a segment is swept by stretches of the steps that fit; without
-// memory for a single one the sweep is the one kernel's.
-constexpr int PREPARED_SETS_PER_CU = 1;
-constexpr size_t COEFFICIENT_BYTES = (size_t)256 << 20;
-void plan_prepared_sweep(pos_ens *h, int seg) {
-    pos_ens::Adjoint &A = h->adj;
-    if (h->E.n_waves > PREPARED_SETS_PER_CU * h->n_cus) return;
-    int max_n = 0;
-    for (int s = 0; s < h->n_systems; ++s) max_n = std::max(max_n, h->body_offset_dev[s + 1] - h->body_offset_dev[s]);
-    const int slots = max_n <= 4 ? 4 : max_n <= 8 ? 8 : 16;
-    const size_t step_bytes = (size_t)coefficient_planes(slots) * h->n_bodies * sizeof(double2);
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) { (void)hipGetLastError(); return; }
-    const size_t stretch = std::min<size_t>(seg, std::min(COEFFICIENT_BYTES, free_b / 4) / step_bytes);
-    if (stretch == 0) return;
-    void *q = nullptr;
-    if (hipMalloc(&q, stretch * step_bytes) != hipSuccess) { (void)hipGetLastError(); return; }
-    A.allocs.push_back(q);
-    A.coef = (double2 *)q;
-    A.stretch = (int)stretch;
-    A.slots = slots;
-}
-
-// One segment's sweep on the adjoint's stream, last step first.
-int launch_sweep(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo) {
-    const pos_ens::Adjoint &A = h->adj;
-    if (!A.coef) {
-        auto kernel = alt ? (evo ? adjoint_segment_kernel<true, true> : adjoint_segment_kernel<true, false>)
-                          : (evo ? adjoint_segment_kernel<false, true> : adjoint_segment_kernel<false, false>);
-        hipLaunchKernelGGL(kernel, dim3(h->grid), dim3(64), 0, A.sweep, Ar);
-        HIP_TRY(hipGetLastError());
-        return POS_OK;
-    }
-    const Coefficients Cf{A.coef, coefficient_planes(A.slots), h->n_bodies};
-    auto prepare = alt ? (evo ? adjoint_prepare_kernel<true, true> : adjoint_prepare_kernel<true, false>)
-                       : (evo ? adjoint_prepare_kernel<false, true> : adjoint_prepare_kernel<false, false>);
-    auto sweep = A.slots == 4 ? (alt ? adjoint_sweep_kernel<4, true> : adjoint_sweep_kernel<4, false>)
-               : A.slots == 8 ? (alt ? adjoint_sweep_kernel<8, true> : adjoint_sweep_kernel<8, false>)
-                              : (alt ? adjoint_sweep_kernel<16, true> : adjoint_sweep_kernel<16, false>);
-    const int per_wave = 16 / A.slots;
-    for (int end = Ar.seg_len; end > 0;) {
-        const int len = std::min(A.stretch, end), row0 = end - len;
-        hipLaunchKernelGGL(prepare, dim3(2 * h->E.n_waves * len), dim3(64), 0, A.sweep, Ar, Cf, row0, len,
-                           A.slots);
-        HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(sweep, dim3((h->n_systems + per_wave - 1) / per_wave), dim3(64), 0, A.sweep, Ar, Cf, row0, len);
-        HIP_TRY(hipGetLastError());
-        end = row0;
-    }
-    return POS_OK;
 }
 
 // The mutable device state of an ensemble (what a checkpoint must hold).
@@ -1048,14 +1013,20 @@ std::vector<std::pair<void *, size_t>> adjoint_state_fields(pos_ens *h) {
 
 // Copy the mutable state into (save) or out of (restore) a checkpoint slot.
 int adjoint_copy_state(pos_ens *h, char *slot, bool save) {
-    size_t off = 0;
+    StateCopy c{};
+    size_t off = 0, most = 1;
+    int n = 0;
     for (const auto &f : adjoint_state_fields(h)) {
-        if (save)
-            HIP_TRY(hipMemcpyAsync(slot + off, f.first, f.second, hipMemcpyDeviceToDevice, h->stream));
-        else
-            HIP_TRY(hipMemcpyAsync(f.first, slot + off, f.second, hipMemcpyDeviceToDevice, h->stream));
+        if (n == STATE_FIELDS) return fail(POS_E_INVALID, "internal error: state fields");
+        c.f[n].src = save ? f.first : slot + off;
+        c.f[n].dst = save ? (void *)(slot + off) : f.first;
+        c.f[n++].bytes = f.second;
+        most = std::max(most, f.second);
         off += (f.second + 255) / 256 * 256;
     }
+    const int blocks = (int)std::min<size_t>((most / 16 + 255) / 256 + 1, 1024);
+    hipLaunchKernelGGL(copy_state_kernel, dim3(blocks, n), dim3(256), 0, h->stream, c);
+    HIP_TRY(hipGetLastError());
     return POS_OK;
 }
 
@@ -1164,6 +1135,152 @@ int launch_steps(pos_ens *h, int n_steps, int *launches = nullptr) {
         }
         HIP_TRY(hipGetLastError());
     }
+    return POS_OK;
+}
+
+// The prepared sweep's workspace, if this ensemble is one it serves better: up to
+// one set of systems per CU.  The whole adjoint of 32 steps took, in one kernel
+// and prepared, us a step: 128 sets of four bodies each 66.9 and 44.8, 256 sets
+// 70.2 and 59.9, 384 sets 76.1 and 83.3; of 2 to 12 bodies 118 sets 96.5 and
+// 69.2, 243 sets 101.7 and 100.8, 487 sets 117 and 170.  The workspace is
+// bounded, a segment is swept by stretches of the steps that fit; without
+// memory for a single one the sweep is the one kernel's.
+constexpr int PREPARED_SETS_PER_CU = 1;
+constexpr size_t COEFFICIENT_BYTES = (size_t)256 << 20;
+void plan_prepared_sweep(pos_ens *h, int seg) {
+    pos_ens::Adjoint &A = h->adj;
+    if (h->E.n_waves > PREPARED_SETS_PER_CU * h->n_cus) return;
+    int max_n = 0;
+    for (int s = 0; s < h->n_systems; ++s) max_n = std::max(max_n, h->body_offset_dev[s + 1] - h->body_offset_dev[s]);
+    const int slots = max_n <= 4 ? 4 : max_n <= 8 ? 8 : 16;
+    const size_t step_bytes = (size_t)coefficient_planes(slots) * h->n_bodies * sizeof(double2);
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) { (void)hipGetLastError(); return; }
+    const size_t stretch = std::min<size_t>(seg, std::min(COEFFICIENT_BYTES, free_b / 4) / 2 / step_bytes);
+    if (stretch == 0) return;
+    void *q = nullptr;
+    if (hipMalloc(&q, 2 * stretch * step_bytes) != hipSuccess) { (void)hipGetLastError(); return; }
+    A.allocs.push_back(q);
+    A.coef = (double2 *)q;
+    A.stretch = (int)stretch;
+    A.slots = slots;
+}
+
+// One segment's sweep, last step first, once its tape is there (`taped`); `swept` is
+// recorded where the tape has been read.  The prepared sweep's coefficients are
+// formed on the handle's stream, where the tape was written, a stretch ahead of
+// the sweep's own; `stretches` counts those launched.
+int launch_sweep(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo, int &stretches, hipEvent_t taped, hipEvent_t swept) {
+    const pos_ens::Adjoint &A = h->adj;
+    if (!A.coef) {
+        auto kernel = alt ? (evo ? adjoint_segment_kernel<true, true> : adjoint_segment_kernel<true, false>)
+                          : (evo ? adjoint_segment_kernel<false, true> : adjoint_segment_kernel<false, false>);
+        HIP_TRY(hipStreamWaitEvent(A.sweep, taped, 0));
+        hipLaunchKernelGGL(kernel, dim3(h->grid), dim3(64), 0, A.sweep, Ar);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipEventRecord(swept, A.sweep));
+        return POS_OK;
+    }
+    const int planes = coefficient_planes(A.slots);
+    auto prepare = alt ? (evo ? adjoint_prepare_kernel<true, true> : adjoint_prepare_kernel<true, false>)
+                       : (evo ? adjoint_prepare_kernel<false, true> : adjoint_prepare_kernel<false, false>);
+    auto sweep = A.slots == 4 ? (alt ? adjoint_sweep_kernel<4, true> : adjoint_sweep_kernel<4, false>)
+               : A.slots == 8 ? (alt ? adjoint_sweep_kernel<8, true> : adjoint_sweep_kernel<8, false>)
+                              : (alt ? adjoint_sweep_kernel<16, true> : adjoint_sweep_kernel<16, false>);
+    const int per_wave = 16 / A.slots;
+    for (int end = Ar.seg_len; end > 0;) {
+        const int len = std::min(A.stretch, end), row0 = end - len, half = stretches & 1;
+        const Coefficients Cf{A.coef + (size_t)half * A.stretch * planes * h->n_bodies, planes, h->n_bodies};
+        if (stretches >= 2) HIP_TRY(hipStreamWaitEvent(h->stream, A.spent_ev[half], 0));
+        hipLaunchKernelGGL(prepare, dim3(2 * h->E.n_waves * len), dim3(64), 0, h->stream, Ar, Cf, row0, len, A.slots);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipEventRecord(A.prepared_ev[half], h->stream));
+        HIP_TRY(hipStreamWaitEvent(A.sweep, A.prepared_ev[half], 0));
+        hipLaunchKernelGGL(sweep, dim3((h->n_systems + per_wave - 1) / per_wave), dim3(64), 0, A.sweep, Ar, Cf, row0, len);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipEventRecord(A.spent_ev[half], A.sweep));
+        end = row0;
+        ++stretches;
+    }
+    HIP_TRY(hipEventRecord(swept, h->stream));   // only the preparation reads the tape
+    return POS_OK;
+}
+
+// `len` steps of every system that also write a segment's tape: one launch per
+// kernel variant (the adjoint admits 0, 8, 24 and 40 only).
+int launch_record(pos_ens *h, const DevEnsemble &E, int len, const TapeRef &tape, int *launches) {
+    *launches = 0;
+    for (int v = 0; v < N_VARIANTS; ++v) {
+        const int w0 = h->variant_waves[v][0], w1 = h->variant_waves[v][1];
+        if (w1 <= w0) continue;
+        ++*launches;
+        const int grid = std::min(h->grid, w1 - w0);
+        switch (v) {
+            case GRV_KIDDER:
+                hipLaunchKernelGGL(whfast_record_kernel<GRV_KIDDER>, dim3(grid), dim3(64), 0, h->stream, E, len, tape, w0, w1);
+                break;
+            case 8: launch_fixed<true, 8>(h, E, grid, len, tape, w0, w1); break;
+            case 24: launch_fixed<true, 24>(h, E, grid, len, tape, w0, w1); break;
+            case 40: launch_fixed<true, 40>(h, E, grid, len, tape, w0, w1); break;
+            default: return fail(POS_E_INVALID, "internal error: kernel variant without an adjoint");
+        }
+        HIP_TRY(hipGetLastError());
+    }
+    return POS_OK;
+}
+
+// The tapes of a whole run are kept up to this: 1,024 systems of four bodies and
+// 256 steps (162 MB) take 3.7 ms to record and 3.0 to differentiate, against 4.5
+// and 5.1 with every segment run a second time.
+constexpr size_t KEPT_TAPE_BYTES = (size_t)1 << 30;
+
+// The buffers, streams and events of a recorded run of n_steps steps.
+int adjoint_allocate(pos_ens *h, int64_t n_steps, int seg) {
+    pos_ens::Adjoint &A = h->adj;
+    adjoint_release(h);
+    const int64_t n_seg = (n_steps + seg - 1) / seg;
+    const size_t nb = h->n_bodies, ns = h->n_systems;
+    const std::vector<std::pair<void *, size_t>> fields = adjoint_state_fields(h);
+    size_t state_bytes = 0;
+    for (const auto &f : fields) state_bytes += (f.second + 255) / 256 * 256;
+    const size_t ckpt_bytes = state_bytes * (size_t)(n_seg + 1);
+    const size_t tape_bytes = (size_t)(seg + 1) * TAPE_FIELDS * nb * sizeof(double);
+    size_t free_b = 0, total_b = 0;
+    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
+    if (ckpt_bytes + 2 * tape_bytes + 64 * nb * sizeof(double) > free_b * 9 / 10)
+        return fail(POS_E_LIMIT, "checkpoints (" + std::to_string(ckpt_bytes >> 20) + " MiB) and segment tape (" +
+                                 std::to_string(tape_bytes >> 20) + " MiB) exceed free device memory; use fewer steps "
+                                 "per segment or fewer systems");
+    auto aalloc = [&](void **p, size_t bytes) -> int {
+        if (hipMalloc(p, std::max<size_t>(bytes, 256)) != hipSuccess) return fail(POS_E_HIP, "hipMalloc failed (adjoint)");
+        A.allocs.push_back(*p);
+        return POS_OK;
+    };
+    int rc;
+    // Every segment's tape is kept where that takes no more memory than two (the
+    // least a recomputation needs) or a small part of the device's: nothing is
+    // recomputed then and the only checkpoint is the final state.
+    const size_t all_bytes = tape_bytes * (size_t)n_seg;
+    const bool keep = n_seg <= 2 || all_bytes <= std::min(KEPT_TAPE_BYTES, free_b / 4);
+    A.tapes = (int)std::min<int64_t>(n_seg, keep ? n_seg : 2);
+    if ((rc = aalloc((void **)&A.ckpt, keep ? state_bytes : ckpt_bytes)) ||
+        (rc = aalloc((void **)&A.tape, tape_bytes * A.tapes)) ||
+        (rc = aalloc((void **)&A.iter0, ns * sizeof(long long))) ||
+        (rc = aalloc((void **)&A.steps_done, ns * sizeof(long long))) ||
+        (rc = aalloc((void **)&A.lx, 3 * nb * sizeof(double))) || (rc = aalloc((void **)&A.lv, 3 * nb * sizeof(double))) ||
+        (rc = aalloc((void **)&A.lL, 3 * nb * sizeof(double))) || (rc = aalloc((void **)&A.gs, nb * sizeof(double))) ||
+        (rc = aalloc((void **)&A.gk2, nb * sizeof(double))) || (rc = aalloc((void **)&A.gkf, nb * sizeof(double))))
+        return rc;
+    plan_prepared_sweep(h, seg);
+    HIP_TRY(hipStreamCreateWithFlags(&A.sweep, hipStreamNonBlocking));
+    for (hipEvent_t *e : {A.taped_ev, A.swept_ev, A.prepared_ev, A.spent_ev})
+        for (int i = 0; i < 2; ++i) HIP_TRY(hipEventCreateWithFlags(&e[i], hipEventDisableTiming));
+    A.seg = seg;
+    A.n_seg = (int)n_seg;
+    A.n_steps = n_steps;
+    A.state_bytes = state_bytes;
+    A.tape_values = tape_bytes / sizeof(double);
+    A.n_waves = h->E.n_waves;
     return POS_OK;
 }
 
@@ -1988,54 +2105,39 @@ int32_t pos_adjoint_record(pos_ens *h, int64_t n_steps, int32_t segment_steps) {
     HIP_TRY(hipSetDevice(h->device));
     pos_ens::Adjoint &A = h->adj;
     HIP_TRY(hipStreamSynchronize(h->stream));
-    adjoint_release(h);
+    A.recorded = false;
     const int64_t seg64 = std::min<int64_t>(segment_steps > 0 ? segment_steps : 1000, n_steps);
     if (seg64 > (1 << 24)) return fail(POS_E_LIMIT, "segment_steps too large");
     const int seg = (int)seg64;
     const int64_t n_seg = (n_steps + seg - 1) / seg;
-    const size_t nb = h->n_bodies, ns = h->n_systems;
-    const std::vector<std::pair<void *, size_t>> fields = adjoint_state_fields(h);
-    size_t state_bytes = 0;
-    for (const auto &f : fields) state_bytes += (f.second + 255) / 256 * 256;
-    const size_t ckpt_bytes = state_bytes * (size_t)(n_seg + 1);
-    const size_t tape_bytes = (size_t)(seg + 1) * TAPE_FIELDS * nb * sizeof(double);
-    size_t free_b = 0, total_b = 0;
-    HIP_TRY(hipMemGetInfo(&free_b, &total_b));
-    if (ckpt_bytes + 2 * tape_bytes + 64 * nb * sizeof(double) > free_b * 9 / 10)
-        return fail(POS_E_LIMIT, "checkpoints (" + std::to_string(ckpt_bytes >> 20) + " MiB) and segment tape (" +
-                                 std::to_string(tape_bytes >> 20) + " MiB) exceed free device memory; use fewer steps "
-                                 "per segment or fewer systems");
-    auto aalloc = [&](void **p, size_t bytes) -> int {
-        if (hipMalloc(p, std::max<size_t>(bytes, 256)) != hipSuccess) return fail(POS_E_HIP, "hipMalloc failed (adjoint)");
-        A.allocs.push_back(*p);
-        return POS_OK;
-    };
+    const size_t ns = h->n_systems;
     int rc;
-    if ((rc = aalloc((void **)&A.ckpt, ckpt_bytes)) || (rc = aalloc((void **)&A.tape[0], tape_bytes)) ||
-        (rc = aalloc((void **)&A.tape[1], tape_bytes)) ||
-        (rc = aalloc((void **)&A.iter0, ns * sizeof(long long))) ||
-        (rc = aalloc((void **)&A.steps_done, ns * sizeof(long long))) ||
-        (rc = aalloc((void **)&A.lx, 3 * nb * sizeof(double))) || (rc = aalloc((void **)&A.lv, 3 * nb * sizeof(double))) ||
-        (rc = aalloc((void **)&A.lL, 3 * nb * sizeof(double))) || (rc = aalloc((void **)&A.gs, nb * sizeof(double))) ||
-        (rc = aalloc((void **)&A.gk2, nb * sizeof(double))) || (rc = aalloc((void **)&A.gkf, nb * sizeof(double))))
+    if (A.sweep) HIP_TRY(hipStreamSynchronize(A.sweep));
+    // a run of the same length and mapping finds its buffers here
+    if ((A.n_steps != n_steps || A.seg != seg || A.n_waves != h->E.n_waves) && (rc = adjoint_allocate(h, n_steps, seg))) {
+        adjoint_release(h);
         return rc;
-    plan_prepared_sweep(h, seg);
-    HIP_TRY(hipStreamCreateWithFlags(&A.sweep, hipStreamNonBlocking));
-    for (int i = 0; i < 2; ++i) {
-        HIP_TRY(hipEventCreateWithFlags(&A.recorded_ev[i], hipEventDisableTiming));
-        HIP_TRY(hipEventCreateWithFlags(&A.swept_ev[i], hipEventDisableTiming));
     }
-    A.seg = seg;
-    A.n_seg = (int)n_seg;
-    A.n_steps = n_steps;
-    A.state_bytes = state_bytes;
+    const bool keep = A.tapes == A.n_seg;
+    const size_t state_bytes = A.state_bytes;
+    A.held.assign(A.tapes, -1);
     HIP_TRY(hipMemcpyAsync(A.iter0, h->E.iteration, ns * sizeof(long long), hipMemcpyDeviceToDevice, h->stream));
     for (int64_t s = 0; s < n_seg; ++s) {
-        if ((rc = adjoint_copy_state(h, A.ckpt + (size_t)s * state_bytes, true))) return rc;
+        if (!keep && (rc = adjoint_copy_state(h, A.ckpt + (size_t)s * state_bytes, true))) return rc;
         const int64_t len = std::min<int64_t>(seg, n_steps - s * seg);
-        if ((rc = pos_step(h, len))) return rc;
+        if (s < n_seg - A.tapes) {
+            if ((rc = pos_step(h, len))) return rc;
+            continue;
+        }
+        const int slot = (int)(s % A.tapes);
+        int nl = 0;
+        if ((rc = launch_record(h, h->E, (int)len, TapeRef{A.tape + slot * A.tape_values, h->n_bodies}, &nl))) return rc;
+        A.held[slot] = (int)s;
+        h->stats.steps += len;
+        h->stats.kernel_launches += nl;
     }
-    if ((rc = adjoint_copy_state(h, A.ckpt + (size_t)n_seg * state_bytes, true))) return rc;
+    A.final_state = A.ckpt + (keep ? 0 : (size_t)n_seg * state_bytes);
+    if ((rc = adjoint_copy_state(h, A.final_state, true))) return rc;
     std::vector<long long> i0(ns), i1(ns);
     if ((rc = download(h, i0, A.iter0, ns)) || (rc = download(h, i1, h->E.iteration, ns))) return rc;
     HIP_TRY(hipStreamSynchronize(h->stream));
@@ -2076,58 +2178,52 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
     Ar.steps_done = A.steps_done;
     Ar.lx = A.lx; Ar.lv = A.lv; Ar.lL = A.lL;
     Ar.gs = A.gs; Ar.gk2 = A.gk2; Ar.gkf = A.gkf;
-    // Segment s is recomputed from its checkpoint on the handle's stream
-    // (writing tape s % 2) while segment s + 1 is swept in reverse on the
-    // sweep stream: the sweep of s waits for the recomputation of s, and the
-    // recomputation of s - 2 waits for the sweep of s, which frees its tape.
+    // The state is the recorded run's final one from here on, as the sweep finds
+    // the bodies' constants in it, whatever the caller did since; where segments
+    // are recomputed, again afterwards.
+    if ((rc = adjoint_copy_state(h, A.final_state, false))) return rc;
+    // Segment s is swept from its tape; one that is not there any more is
+    // recomputed from its checkpoint on the handle's stream, into the tape of
+    // the segment swept `tapes` before, while the sweeps in between run.
     auto seg_len = [&](int s) { return (int)std::min<int64_t>(A.seg, A.n_steps - (int64_t)s * A.seg); };
-    auto recompute = [&](int s) -> int {
-        const int buf = s & 1;
-        if (s + 2 < A.n_seg) HIP_TRY(hipStreamWaitEvent(h->stream, A.swept_ev[buf], 0));
-        int r = adjoint_copy_state(h, A.ckpt + (size_t)s * A.state_bytes, false);
-        if (r) return r;
-        for (int v = 0; v < N_VARIANTS; ++v) {   // pos_adjoint_record admits variants 0, 8, 24 and 40 only
-            const int w0 = h->variant_waves[v][0], w1 = h->variant_waves[v][1];
-            if (w1 <= w0) continue;
-            const dim3 grid(std::min(h->grid, w1 - w0));
-            const TapeRef tape{A.tape[buf], nb};
+    const bool keep = A.tapes == A.n_seg;
+    bool recomputed = false;
+    auto taped = [&](int s) -> int {
+        const int slot = s % A.tapes;
+        if (A.held[slot] != s) {
+            A.held[slot] = -1;
+            recomputed = true;
+            int r = adjoint_copy_state(h, A.ckpt + (size_t)s * A.state_bytes, false), nl = 0;
+            if (r) return r;
             // the recomputed steps were recorded once already: no historic records
-            const DevEnsemble Er = without_history(h->E);
-            if (v == GRV_KIDDER)
-                hipLaunchKernelGGL(whfast_record_kernel<GRV_KIDDER>, grid, dim3(64), 0, h->stream, Er, seg_len(s), tape, w0, w1);
-            else if (v == (GRV_KIDDER | VAR_FAST))
-                launch_fixed<true, GRV_KIDDER | VAR_FAST>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
-            else if (v == (GRV_KIDDER | VAR_FAST | VAR_JACOBI))
-                launch_fixed<true, GRV_KIDDER | VAR_FAST | VAR_JACOBI>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
-            else if (v == (GRV_KIDDER | VAR_FAST | VAR_WHDS))
-                launch_fixed<true, GRV_KIDDER | VAR_FAST | VAR_WHDS>(h, Er, (int)grid.x, seg_len(s), tape, w0, w1);
-            else
-                return fail(POS_E_INVALID, "internal error: kernel variant without an adjoint");
-            HIP_TRY(hipGetLastError());
+            const TapeRef tape{A.tape + slot * A.tape_values, nb};
+            if ((r = launch_record(h, without_history(h->E), seg_len(s), tape, &nl))) return r;
+            A.held[slot] = s;
         }
-        HIP_TRY(hipEventRecord(A.recorded_ev[buf], h->stream));
+        HIP_TRY(hipEventRecord(A.taped_ev[slot & 1], h->stream));
         return POS_OK;
     };
     const bool alt = std::any_of(h->coord_dev.begin(), h->coord_dev.end(),
                                  [](int c) { return c != POS_COORD_DEMOCRATIC_HELIOCENTRIC; });
     const bool evo = std::any_of(h->eff_dev.begin(), h->eff_dev.end(),
                                  [](uint32_t e) { return (e & POS_EFFECT_EVOLUTION) != 0; });
-    // the sweep stream must also see the seeds uploaded on the handle's stream
-    HIP_TRY(hipEventRecord(A.swept_ev[0], h->stream));
-    HIP_TRY(hipStreamWaitEvent(A.sweep, A.swept_ev[0], 0));
-    if ((rc = recompute(A.n_seg - 1))) return rc;
+    int stretches = 0;
+    for (int s = A.n_seg - 1; s >= std::max(0, A.n_seg - 2); --s)
+        if ((rc = taped(s))) return rc;
     for (int s = A.n_seg - 1; s >= 0; --s) {
-        const int buf = s & 1;
-        HIP_TRY(hipStreamWaitEvent(A.sweep, A.recorded_ev[buf], 0));
-        Ar.T = TapeRef{A.tape[buf], nb};
+        const int slot = s % A.tapes;
+        Ar.T = TapeRef{A.tape + slot * A.tape_values, nb};
         Ar.seg_start = (int64_t)s * A.seg;
         Ar.seg_len = seg_len(s);
-        if ((rc = launch_sweep(h, Ar, alt, evo))) return rc;
-        HIP_TRY(hipEventRecord(A.swept_ev[buf], A.sweep));
-        if (s > 0 && (rc = recompute(s - 1))) return rc;
+        if ((rc = launch_sweep(h, Ar, alt, evo, stretches, A.taped_ev[slot & 1], A.swept_ev[slot & 1]))) return rc;
+        if (!keep && s >= 2) {
+            HIP_TRY(hipStreamWaitEvent(h->stream, A.swept_ev[slot & 1], 0));
+            if ((rc = taped(s - 2))) return rc;
+        }
     }
+    HIP_TRY(hipEventRecord(A.swept_ev[0], A.sweep));
     HIP_TRY(hipStreamWaitEvent(h->stream, A.swept_ev[0], 0));
-    if ((rc = adjoint_copy_state(h, A.ckpt + (size_t)A.n_seg * A.state_bytes, false))) return rc;
+    if (recomputed && (rc = adjoint_copy_state(h, A.final_state, false))) return rc;
     // results, device -> input order
     std::vector<double> lx, lv, lL, gs, gk2, gkf;
     if ((rc = download(h, lx, A.lx, 3 * (size_t)nb)) || (rc = download(h, lv, A.lv, 3 * (size_t)nb)) ||
