@@ -104,6 +104,34 @@ def _host_index(spec: EnsembleSpec) -> np.ndarray:
     return hosts[_system_index(spec)]
 
 
+def _equal(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two tensors hold the same values, False where that cannot be
+    asked for (while tracing, or of a transformed tensor)."""
+    if torch.compiler.is_compiling():
+        return False
+    try:
+        return torch.equal(a, b)
+    except RuntimeError:
+        return False
+
+
+def _eccentric_anomaly(e, M, iterations):
+    """Newton's iteration for E - e sin E = M from E = M, `iterations` times.
+
+    Each iterate depends on the one before alone, so one that equals an earlier
+    iterate makes the sequence periodic: once every body repeats its last value
+    or alternates between two (rounding does that), the final iterate is known.
+    That is looked up every eighth iteration, which as a rule ends the loop at
+    the first look (six launches an iteration are 30 us)."""
+    E2 = E1 = E = M.clone()
+    for k in range(1, iterations + 1):
+        E2, E1 = E1, E
+        E = E - (E - e * torch.sin(E) - M) / (1.0 - e * torch.cos(E))
+        if k % 8 == 0 and k >= 2 and _equal(E, E2):
+            return E if (iterations - k) % 2 == 0 else E1
+    return E
+
+
 def state_from_elements(spec: EnsembleSpec, a: torch.Tensor, e: torch.Tensor):
     """Initial barycentric positions and velocities from per-body semi-major
     axis and eccentricity (host rows ignored); the other elements are the
@@ -125,9 +153,7 @@ def state_from_elements(spec: EnsembleSpec, a: torch.Tensor, e: torch.Tensor):
     # eccentric anomaly: converged without gradient, then one Newton step that
     # carries the implicit derivative dE = (dM + sin E de) / (1 - e cos E)
     with torch.no_grad():
-        E0 = M.clone()
-        for _ in range(60):
-            E0 = E0 - (E0 - e_ * torch.sin(E0) - M) / (1.0 - e_ * torch.cos(E0))
+        E0 = _eccentric_anomaly(e_, M, 60)
     E = E0 - (E0 - e_ * torch.sin(E0) - M) / (1.0 - e_ * torch.cos(E0))
     g = varpi - node
     si, ci = torch.sin(inc), torch.cos(inc)
