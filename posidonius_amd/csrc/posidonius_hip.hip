@@ -206,6 +206,32 @@ void whfast_steps_kernel(DevEnsemble E, int n_steps, int wave_begin, int wave_en
     }
 }
 
+// K steps of waves [wave_begin, wave_end) of the Newhall variant by teams of four
+// wavefronts (NewhallTeam).
+__global__ __launch_bounds__(64 * (1 + NEWHALL_HELPERS))
+void whfast_newhall_kernel(DevEnsemble E, int n_steps, int wave_begin, int wave_end) {
+    constexpr int V = GRV_NEWHALL | VAR_TEAM;
+    __shared__ NewhallLds lds;
+    const int role = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    for (int wave = wave_begin + blockIdx.x; wave < wave_end; wave += gridDim.x) {
+        if (role == 0) {
+            Lane B;
+            load_lane<V>(E, lds, B, wave);
+            const TapeRef none{nullptr, 0};
+            for (int step = 0; step < n_steps; ++step) {
+                const bool go = !(B.status & FROZEN);
+                if (!__any(go)) break;   // the barriers of a step need a lane that takes it
+                if (go) iterate<false, V>(E, lds, B, none, 0);
+            }
+            newhall_command(lds, NEWHALL_END);
+            store_lane(E, lds, B);
+        } else {
+            newhall_helper(E, lds, wave, role - 1);
+        }
+        __syncthreads();
+    }
+}
+
 // The same K steps over waves [wave_begin, wave_end) of variant V, also writing the step tape of the adjoint (one row per step plus the final
 // state).
 template <int V>
@@ -1124,7 +1150,14 @@ int launch_steps(pos_ens *h, int n_steps, int *launches = nullptr) {
         switch (v) {
             case 0: launch_steps_variant<0>(h, grid, n_steps, w0, w1); break;
             case 1: launch_steps_variant<1>(h, grid, n_steps, w0, w1); break;
-            case 2: launch_steps_variant<2>(h, grid, n_steps, w0, w1); break;
+            case 2:
+                // A team's LDS fills a CU, so teams serve up to one set of systems per CU
+                if (w1 - w0 <= h->n_cus)
+                    hipLaunchKernelGGL(whfast_newhall_kernel, dim3(grid), dim3(64 * (1 + NEWHALL_HELPERS)), 0, h->stream, h->E,
+                                       n_steps, w0, w1);
+                else
+                    launch_steps_variant<2>(h, grid, n_steps, w0, w1);
+                break;
             case 4: launch_steps_variant<4>(h, grid, n_steps, w0, w1); break;
             case 5: launch_steps_variant<5>(h, grid, n_steps, w0, w1); break;
             case 6: launch_steps_variant<6>(h, grid, n_steps, w0, w1); break;

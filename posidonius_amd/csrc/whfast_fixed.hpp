@@ -131,9 +131,7 @@ __device__ __forceinline__ void team_sync() {
     if constexpr (M == 1) {
         wsync();
     } else {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+        team_barrier();
     }
 }
 

@@ -196,6 +196,13 @@ __device__ __forceinline__ void wsync() {
 // this lane's index in it.  A lane past the wave's groups gets gvalid =
 // false, the wave's first system and its own lane as group start (so that
 // every LDS index it forms stays inside the wave's columns).
+// Meeting point of the wavefronts of a team.
+__device__ __forceinline__ void team_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
 struct LaneGroup {
     int sys, gbase, k;
     bool gvalid;
@@ -474,6 +481,7 @@ constexpr int VAR_FAST = 8;
 constexpr int VAR_JACOBI = 16;   // only with VAR_FAST
 constexpr int VAR_WHDS = 32;     // only with VAR_FAST
 constexpr int N_VARIANTS = 64;
+constexpr int VAR_TEAM = 64;     // of a kernel only: Newhall's pair terms by a team (NewhallTeam)
 constexpr uint32_t EFF_VAR_SHIFT = 16;
 __host__ __device__ __forceinline__ int eff_variant(uint32_t eff) { return (int)((eff >> EFF_VAR_SHIFT) & 63u); }
 __host__ __device__ __forceinline__ int eff_gr_variant(uint32_t eff) { return eff_variant(eff) & 3; }
@@ -652,29 +660,171 @@ __device__ inline void gr_anderson1975(WaveLds &lds, Lane &B, double g[3], Solve
     wsync();
 }
 
+// The pair terms of Newhall et al. 1983 on body i from body j, whose fixed order of
+// addition is the caller's.  geometry: positions and masses only.
+struct NewhallPair {
+    double d[3], rij, rij2, gm;
+    Rcp R3;
+};
+__device__ __forceinline__ NewhallPair newhall_pair(const double xi[3], double x0, double x1, double x2, double mj) {
+    NewhallPair P;
+    P.d[0] = xi[0] - x0; P.d[1] = xi[1] - x1; P.d[2] = xi[2] - x2;
+    P.rij = sqrt(p2(P.d[0]) + p2(P.d[1]) + p2(P.d[2]));
+    P.rij2 = p2(P.rij);
+    P.R3 = rcp(P.rij2 * P.rij);
+    P.gm = G * mj;
+    return P;
+}
+// terms of a1 and a2
+__device__ __forceinline__ void newhall_mass_terms(double mj, const Rcp &R1, double t[2]) {
+    constexpr double c2 = SPEED_OF_LIGHT_2;
+    t[0] = divr((4. / c2) * G * mj, R1);
+    t[1] = divr((1. / c2) * G * mj, R1);
+}
+// two terms per component from the other body's acceleration s
+__device__ __forceinline__ void newhall_acceleration_terms(const NewhallPair &P, const Rcp &R1, double mj, const double s[3],
+                                                           double t[6]) {
+    constexpr double c2 = SPEED_OF_LIGHT_2;
+    constexpr Rcp R2C2{2. * c2, 1. / (2. * c2)};
+    const double proj = P.d[0] * s[0] + P.d[1] * s[1] + P.d[2] * s[2];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        t[q] = divr(divr(P.gm * P.d[q], P.R3) * proj, R2C2);
+        t[3 + q] = divr((7. / (2. * c2)) * G * mj * s[q], R1);
+    }
+}
+// two terms per component from the velocities; a1 and a3 of body i, a2 of body j
+__device__ __forceinline__ void newhall_velocity_terms(const NewhallPair &P, const double vi[3], const double vj[3], double a1,
+                                                       double a2, double a3, double t[6]) {
+    constexpr double c2 = SPEED_OF_LIGHT_2;
+    const double vj2 = p2(vj[0]) + p2(vj[1]) + p2(vj[2]);
+    const double a4 = divr(-2. * vj2, RC2);
+    const double a5 = (4. / c2) * (vi[0] * vj[0] + vi[1] * vj[1] + vi[2] * vj[2]);
+    const double a60 = P.d[0] * vj[0] + P.d[1] * vj[1] + P.d[2] * vj[2];
+    const double a6 = (3. / (2. * c2)) * p2(a60) / P.rij2;
+    const double f1 = a1 + a2 + a3 + a4 + a5 + a6;
+    const double f2 = P.d[0] * (4. * vi[0] - 3. * vj[0]) + P.d[1] * (4. * vi[1] - 3. * vj[1]) + P.d[2] * (4. * vi[2] - 3. * vj[2]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        t[q] = divr(P.gm * P.d[q] * f1, P.R3);
+        t[3 + q] = divr(divr(P.gm * f2 * (vi[q] - vj[q]), P.R3), RC2);
+    }
+}
+
+// A team of four wavefronts for small ensembles: wave 0 runs the step, the
+// others form the Newhall pair terms, a third of the pairs each, while it is at
+// the tides and flattening, and hand them over in LDS for it to add in order.
+// An evaluation is a command and two barriers; the first one of a solve is two
+// commands (the sums a1 and a2 enter every velocity term), and the pairs'
+// geometry stays in the helpers' registers for the others.
+// 64 steps of 777 systems of 2 to 10 bodies in WHDS coordinates: 4,576 -> 3,004
+// us; of 200 systems of 3 to 12 bodies 5,009 -> 3,086, in Jacobi coordinates
+// 5,439 -> 3,440.  The rest of the step, in one wavefront, is what bounds it.
+constexpr int NEWHALL_HELPERS = 3;
+constexpr int NEWHALL_SHARE = (POS_MAX_BODIES + NEWHALL_HELPERS - 1) / NEWHALL_HELPERS;
+enum { NEWHALL_END = 0, NEWHALL_FIRST = 1, NEWHALL_VELOCITIES = 2 };
+struct NewhallTeam {
+    int command;
+    double x[3][WAVE], v[3][WAVE], an[3][WAVE];
+    double a1[WAVE], a2[WAVE];
+    double term[POS_MAX_BODIES][8][WAVE];   // of the body at this place in the chain
+};
+struct NewhallLds : WaveLds { NewhallTeam team; };
+
+__device__ __forceinline__ void newhall_command(NewhallLds &lds, int command) {
+    lds.team.command = command;
+    team_barrier();
+}
+
+// A helper's whole launch on one set of systems: `part` of NEWHALL_HELPERS.
+// Ends when the step's wavefront commands it.
+__device__ inline void newhall_helper(const DevEnsemble &E, NewhallLds &lds, int wave, int part) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    const LaneGroup lg = lane_group(E, wave, lane);
+    const int n = lg.gvalid ? E.body_offset[lg.sys + 1] - E.body_offset[lg.sys] : 0;
+    const int host = E.host[lg.sys];
+    const bool valid = lg.gvalid && lg.k < n;
+    const int me = lg.k == host ? 0 : (lg.k < host ? lg.k + 1 : lg.k);
+    auto other = [&](int c) { return lg.gbase + (c == 0 ? host : (c - 1 < host ? c - 1 : c)); };
+    NewhallTeam &T = lds.team;
+    NewhallPair P[NEWHALL_SHARE];
+    __syncthreads();   // load_lane's
+    for (;;) {
+        team_barrier();
+        const int command = __builtin_amdgcn_readfirstlane(T.command);
+        if (command == NEWHALL_END) break;
+        if (command == NEWHALL_FIRST) {
+            const double xi[3] = {T.x[0][lane], T.x[1][lane], T.x[2][lane]};
+#pragma unroll
+            for (int u = 0; u < NEWHALL_SHARE; ++u) {
+                const int c = part + NEWHALL_HELPERS * u;
+                if (!valid || c >= n || c == me) continue;
+                const int l = other(c);
+                const double mj = lds.m[l];
+                P[u] = newhall_pair(xi, T.x[0][l], T.x[1][l], T.x[2][l], mj);
+                const Rcp R1 = rcp(P[u].rij);
+                const double s[3] = {T.an[0][l] + 0., T.an[1][l] + 0., T.an[2][l] + 0.};
+                double m[2], t[6];
+                newhall_mass_terms(mj, R1, m);
+                newhall_acceleration_terms(P[u], R1, mj, s, t);
+                T.term[c][6][lane] = m[0];
+                T.term[c][7][lane] = m[1];
+#pragma unroll
+                for (int q = 0; q < 6; ++q) T.term[c][q][lane] = t[q];
+            }
+        } else {
+            const double vi[3] = {T.v[0][lane], T.v[1][lane], T.v[2][lane]};
+            const double a1 = T.a1[lane], a3 = divr(-(p2(vi[0]) + p2(vi[1]) + p2(vi[2])), RC2);
+#pragma unroll
+            for (int u = 0; u < NEWHALL_SHARE; ++u) {
+                const int c = part + NEWHALL_HELPERS * u;
+                if (!valid || c >= n || c == me) continue;
+                const int l = other(c);
+                const double vj[3] = {T.v[0][l], T.v[1][l], T.v[2][l]};
+                double t[6];
+                newhall_velocity_terms(P[u], vi, vj, a1, T.a2[l], a3, t);
+#pragma unroll
+                for (int q = 0; q < 6; ++q) T.term[c][q][lane] = t[q];
+            }
+        }
+        team_barrier();
+    }
+}
+
 // Newhall et al. 1983, every pair (general_relativity.rs:683-895).  Most of the
 // pair terms depend on the positions alone: the sums a1 and a2 and, the first
 // pass of the fixed point starting from zero, its acceleration terms.  They are
 // formed by the first evaluation of a solve; an evaluation then costs the
 // velocity terms, one square root and two reciprocals a pair (430 against 110
 // instructions; quotients by a shared or constant divisor go through divr).
-__device__ inline void gr_newhall1983(WaveLds &lds, Lane &B, double g[3], SolveCache &sc, bool first) {
-    const int lane = B.lane;
-    const int n = B.n;
-    if (B.valid()) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
-    wsync();
+//
+// In a team, newhall_start hands the positions and velocities to the helpers
+// (rows 0-2 must hold the positions) and gr_newhall1983 collects their terms.
+__device__ inline void newhall_start(NewhallLds &lds, Lane &B, SolveCache &sc, bool first) {
     if (first) gr_newtonian(lds, B, sc.an);
     if (B.valid()) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) { lds.xb[3 + q][lane] = B.v[q]; lds.xb[6 + q][lane] = sc.an[q]; }
+        for (int q = 0; q < 3; ++q) {
+            lds.team.v[q][B.lane] = B.v[q];
+            if (first) { lds.team.x[q][B.lane] = B.x[q]; lds.team.an[q][B.lane] = sc.an[q]; }
+        }
     }
-    constexpr double c2 = SPEED_OF_LIGHT_2;
-    constexpr Rcp R2C2{2. * c2, 1. / (2. * c2)};
+    newhall_command(lds, first ? NEWHALL_FIRST : NEWHALL_VELOCITIES);
+}
+
+template <bool TEAM>
+__device__ inline void gr_newhall1983(WaveLds &lds, Lane &B, double g[3], SolveCache &sc, bool first) {
+    const int lane = B.lane;
+    const int n = B.n;
     const int me = chained_pos(B, B.k);
-    auto separation = [&](int l, double d[3]) {
+    auto publish = [&] {
+        if (B.valid()) {
 #pragma unroll
-        for (int q = 0; q < 3; ++q) d[q] = B.x[q] - lds.xb[q][l];
-        return sqrt(p2(d[0]) + p2(d[1]) + p2(d[2]));
+            for (int q = 0; q < 3; ++q) {
+                lds.xb[q][lane] = B.x[q]; lds.xb[3 + q][lane] = B.v[q]; lds.xb[6 + q][lane] = sc.an[q];
+            }
+        }
+        wsync();
     };
     // the acceleration terms of one fixed-point pass; rows 10-12 hold the
     // previous iterate of every body (with START it is zero everywhere)
@@ -683,63 +833,74 @@ __device__ inline void gr_newhall1983(WaveLds &lds, Lane &B, double g[3], SolveC
         for (int c = 0; c < n; ++c) {
             if (c == me) continue;
             const int l = B.gbase + chained_body(B, c);
-            double d[3], s[3];
-            const double rij = separation(l, d);
-            const double rij2 = p2(rij);
-            const Rcp R1 = rcp(rij), R3 = rcp(rij2 * rij);
+            const NewhallPair P = newhall_pair(B.x, lds.xb[0][l], lds.xb[1][l], lds.xb[2][l], lds.m[l]);
+            double s[3], t[6];
 #pragma unroll
             for (int q = 0; q < 3; ++q) s[q] = lds.xb[6 + q][l] + (start ? 0. : lds.xb[10 + q][l]);
-            const double proj = d[0] * s[0] + d[1] * s[1] + d[2] * s[2];
-            const double gm = G * lds.m[l];
+            newhall_acceleration_terms(P, rcp(P.rij), lds.m[l], s, t);
 #pragma unroll
-            for (int q = 0; q < 3; ++q)
-                nc[q] = nc[q] + divr(divr(gm * d[q], R3) * proj, R2C2) + divr((7. / (2. * c2)) * G * lds.m[l] * s[q], R1);
+            for (int q = 0; q < 3; ++q) nc[q] = nc[q] + t[q] + t[3 + q];
         }
     };
-    wsync();
-    if (first && B.valid()) {
-        // a2 depends only on the second body j: sum_l G m_l / (c^2 r_lj), which
-        // body j evaluates from its own distances (|x_l - x_j| = |x_j - x_l|)
-        sc.a1 = sc.a2 = 0.;
-        for (int c = 0; c < n; ++c) {
-            if (c == me) continue;
-            const int l = B.gbase + chained_body(B, c);
-            const double mk = lds.m[l];
-            double d[3];
-            const Rcp R1 = rcp(separation(l, d));
-            sc.a1 = sc.a1 + divr((4. / c2) * G * mk, R1);
-            sc.a2 = sc.a2 + divr((1. / c2) * G * mk, R1);
-        }
-        acceleration_terms(sc.nc, std::true_type{});
-    }
-    if (B.valid()) lds.xb[9][lane] = sc.a2;
-    wsync();
     double ac[3] = {0., 0., 0.};
-    if (B.valid()) {
-        const double vi2 = p2(B.v[0]) + p2(B.v[1]) + p2(B.v[2]);
-        const double a3 = divr(-vi2, RC2);
+    if constexpr (TEAM) {
+        NewhallLds &tl = static_cast<NewhallLds &>(lds);
+        team_barrier();
+        // a scalar branch: the barriers inside are the whole wavefront's
+        if (__builtin_amdgcn_readfirstlane(first ? 1 : 0)) {
+            sc.a1 = sc.a2 = 0.;
+#pragma unroll
+            for (int q = 0; q < 3; ++q) sc.nc[q] = 0.;
+            for (int c = 0; c < n; ++c) {
+                if (!B.valid() || c == me) continue;
+                sc.a1 = sc.a1 + tl.team.term[c][6][lane];
+                sc.a2 = sc.a2 + tl.team.term[c][7][lane];
+#pragma unroll
+                for (int q = 0; q < 3; ++q) sc.nc[q] = sc.nc[q] + tl.team.term[c][q][lane] + tl.team.term[c][3 + q][lane];
+            }
+            if (B.valid()) { tl.team.a1[lane] = sc.a1; tl.team.a2[lane] = sc.a2; }
+            newhall_command(tl, NEWHALL_VELOCITIES);
+            team_barrier();
+        }
         for (int c = 0; c < n; ++c) {
-            if (c == me) continue;
-            const int l = B.gbase + chained_body(B, c);
-            double d[3];
-            const double rij = separation(l, d);
-            const double rij2 = p2(rij);
-            const Rcp R3 = rcp(rij2 * rij);
-            const double vj0 = lds.xb[3][l], vj1 = lds.xb[4][l], vj2c = lds.xb[5][l];
-            const double a2 = lds.xb[9][l];
-            const double vj2 = p2(vj0) + p2(vj1) + p2(vj2c);
-            const double a4 = divr(-2. * vj2, RC2);
-            const double a5 = (4. / c2) * (B.v[0] * vj0 + B.v[1] * vj1 + B.v[2] * vj2c);
-            const double a60 = d[0] * vj0 + d[1] * vj1 + d[2] * vj2c;
-            const double a6 = (3. / (2. * c2)) * p2(a60) / rij2;
-            const double f1 = sc.a1 + a2 + a3 + a4 + a5 + a6;
-            const double gm = G * lds.m[l];
+            if (!B.valid() || c == me) continue;
 #pragma unroll
-            for (int q = 0; q < 3; ++q) ac[q] = ac[q] + divr(gm * d[q] * f1, R3);
-            const double dv[3] = {B.v[0] - vj0, B.v[1] - vj1, B.v[2] - vj2c};
-            const double f2 = d[0] * (4. * B.v[0] - 3. * vj0) + d[1] * (4. * B.v[1] - 3. * vj1) + d[2] * (4. * B.v[2] - 3. * vj2c);
+            for (int q = 0; q < 3; ++q) ac[q] = ac[q] + tl.team.term[c][q][lane] + tl.team.term[c][3 + q][lane];
+        }
+    } else {
+        if (B.valid()) { lds.xb[0][lane] = B.x[0]; lds.xb[1][lane] = B.x[1]; lds.xb[2][lane] = B.x[2]; }
+        wsync();
+        if (first) gr_newtonian(lds, B, sc.an);
+        publish();
+        if (first && B.valid()) {
+            // a2 depends only on the second body j: sum_l G m_l / (c^2 r_lj), which
+            // body j evaluates from its own distances (|x_l - x_j| = |x_j - x_l|)
+            sc.a1 = sc.a2 = 0.;
+            for (int c = 0; c < n; ++c) {
+                if (c == me) continue;
+                const int l = B.gbase + chained_body(B, c);
+                const NewhallPair P = newhall_pair(B.x, lds.xb[0][l], lds.xb[1][l], lds.xb[2][l], lds.m[l]);
+                double t[2];
+                newhall_mass_terms(lds.m[l], rcp(P.rij), t);
+                sc.a1 = sc.a1 + t[0];
+                sc.a2 = sc.a2 + t[1];
+            }
+            acceleration_terms(sc.nc, std::true_type{});
+        }
+        if (B.valid()) lds.xb[9][lane] = sc.a2;
+        wsync();
+        if (B.valid()) {
+            const double a3 = divr(-(p2(B.v[0]) + p2(B.v[1]) + p2(B.v[2])), RC2);
+            for (int c = 0; c < n; ++c) {
+                if (c == me) continue;
+                const int l = B.gbase + chained_body(B, c);
+                const NewhallPair P = newhall_pair(B.x, lds.xb[0][l], lds.xb[1][l], lds.xb[2][l], lds.m[l]);
+                const double vj[3] = {lds.xb[3][l], lds.xb[4][l], lds.xb[5][l]};
+                double t[6];
+                newhall_velocity_terms(P, B.v, vj, sc.a1, lds.xb[9][l], a3, t);
 #pragma unroll
-            for (int q = 0; q < 3; ++q) ac[q] = ac[q] + divr(divr(gm * f2 * dv[q], R3), RC2);
+                for (int q = 0; q < 3; ++q) ac[q] = ac[q] + t[q] + t[3 + q];
+            }
         }
     }
     // The fixed point's convergence test of the reference only looks at
@@ -755,6 +916,7 @@ __device__ inline void gr_newhall1983(WaveLds &lds, Lane &B, double g[3], SolveC
         // new one.  A group stops iterating when its own test passes (every
         // lane of the group evaluates it identically); the wavefront leaves
         // the loop once every group has.
+        if constexpr (TEAM) publish();
         anew[0] = anew[1] = anew[2] = 0.;
         bool done = !B.valid();
         for (int k = 0; k < 10; ++k) {
@@ -860,6 +1022,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
                                           double a_add[3], double dLdt[3], SolveCache &sc, bool first) {
     constexpr int GRV = V & 3;
     constexpr bool EXT = (V & VAR_EXT) != 0;
+    constexpr bool TEAM = (V & VAR_TEAM) != 0;
     const LaneTests<V> LT(B);
     const int lane = B.lane;
     const int hl = B.hl();
@@ -893,6 +1056,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
     const Rcp Rd = rcp(d);
     const double vr = orbiting ? divr(px[0] * pv[0] + px[1] * pv[1] + px[2] * pv[2], Rd) : 0.;
     wsync();
+    if constexpr (TEAM) newhall_start(static_cast<NewhallLds &>(lds), B, sc, first);
     // ---- evolution and spin = L / I (universe.rs:305-316) ----
     if (evolution && (B.flags & F_EVOLUTION)) evolve_body(E, lds, B, B.t);
     own_spin(lds, B);
@@ -1223,7 +1387,7 @@ __device__ inline void additional_effects(const DevEnsemble &E, WaveLds &lds, La
     if (GRV != GRV_KIDDER) {   // uniform: such a launch holds only systems of this variant
         double g[3];
         if (GRV == GRV_ANDERSON) gr_anderson1975(lds, B, g, sc, first);
-        else gr_newhall1983(lds, B, g, sc, first);
+        else gr_newhall1983<TEAM>(lds, B, g, sc, first);
         if (B.valid() && LT.gr) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) a_add[q] = a_add[q] + g[q];

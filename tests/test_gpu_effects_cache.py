@@ -71,3 +71,21 @@ def test_gr_solves_against_oracle(oracle, impl, coords, plane):
     assert np.all(np.isfinite(z))
     if plane < 1.:
         assert z.max() < 1e-20
+
+
+@pytest.mark.parametrize("coords", [abi.COORD_DEMOCRATIC_HELIOCENTRIC, abi.COORD_JACOBI])
+@pytest.mark.parametrize("more", [0, 1], ids=["teams", "single_wavefronts"])
+def test_newhall_teams_against_oracle(oracle, more, coords):
+    """As many sets of systems as the teams serve and one more: systems of 2 to
+    16 bodies, some stopping on the way, one colliding in its first step, some
+    launches with every system of a wavefront stopped."""
+    from posidonius_amd.ensemble import Ensemble
+    systems, steps = edge(1, more), 24
+    spec = ensemble(systems, coords, 73)
+    spec.system["gr_implementation"][:] = abi.GR_NEWHALL1983
+    print(f"{systems} sets of systems, coordinates {coords}", flush=True)
+    ref = oracle.run(spec, steps, threads=THREADS)
+    with Ensemble(spec, mapping="packed", group_size=64, steps_per_launch=8) as ens:
+        ens.step(steps)
+        out = ens.get_state()
+    assert_same_state(out, ref, where=f"Newhall {systems} sets")
