@@ -142,9 +142,11 @@ POS_HD PairOut pair_forward(const PairConst &C, const PairPar &P, const PairIn &
 
 // Vector-Jacobian product of pair_forward: given the cotangents of the
 // outputs, accumulate the cotangents of the inputs (into Ib) and of the
-// parameters (into Pb).
-POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, const PairOut &ob, PairIn &Ib,
-                     PairParBar &Pb) {
+// parameters (into Pb).  FA, FP, FH: of F and g, of Np, of Nh; what only the
+// others need is left out.
+template <bool FA, bool FP, bool FH>
+POS_HD void pair_vjp_of(const PairConst &C, const PairPar &P, const PairIn &I, const PairOut &ob, PairIn &Ib,
+                        PairParBar &Pb) {
     const V3 r = I.r, u = I.u;
     const double d2 = dot(r, r), d = sqrt(d2), id = 1. / d;
     const double u2 = dot(u, u);
@@ -174,14 +176,31 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
         const V3 wh = cross(I.Wh, r) - u, wp = cross(I.Wp, r) - u;
         const V3 Fb = ob.F;
         // F_t = f3 id r + os id wh + op id wp
-        const double f3_b = id * dot(Fb, r);
-        id_b += f3 * dot(Fb, r) + os * dot(Fb, wh) + op * dot(Fb, wp);
-        r_b += (f3 * id) * Fb;
-        double os_b = id * dot(Fb, wh), op_b = id * dot(Fb, wp);
-        const V3 wh_b = (os * id) * Fb, wp_b = (op * id) * Fb;
+        double os_b = 0., op_b = 0., SA_b = 0.;
+        if (FA) {
+            const double f3_b = id * dot(Fb, r);
+            id_b += f3 * dot(Fb, r) + os * dot(Fb, wh) + op * dot(Fb, wp);
+            r_b += (f3 * id) * Fb;
+            os_b = id * dot(Fb, wh);
+            op_b = id * dot(Fb, wp);
+            const V3 wh_b = (os * id) * Fb, wp_b = (op * id) * Fb;
+            // wh = Wh x r - u, wp = Wp x r - u
+            cross_adj(I.Wh, r, wh_b, Wh_b, r_b);
+            u_b -= wh_b;
+            cross_adj(I.Wp, r, wp_b, Wp_b, r_b);
+            u_b -= wp_b;
+            // f3 = -3 K2 Ck / d7 - 2 vr SA / d8
+            const double Ck_b = f3_b * (-3. * G_K2 / d7);
+            d7_b += f3_b * (3. * G_K2 * Ck * id7 * id7);
+            vr_b += f3_b * (-2. * SA / d8);
+            SA_b = f3_b * (-2. * vr / d8);
+            d8_b += f3_b * (2. * vr * SA * id8 * id8);
+            Pb.k2h += Ck_b * Kh;
+            Pb.k2p += Ck_b * Kp;
+        }
         // N_tp = -op T_p,  T_p = d Wp - rsp id r - id c
         V3 c_b = zero3();
-        {
+        if (FP) {
             const V3 T = d * I.Wp - (rsp * id) * r - id * c;
             op_b += -dot(ob.Np, T);
             const V3 Tb = (-op) * ob.Np;
@@ -192,7 +211,7 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
             r_b += (-rsp * id) * Tb;
             c_b += (-id) * Tb;
         }
-        {
+        if (FH) {
             const V3 T = d * I.Wh - (rsh * id) * r - id * c;
             os_b += -dot(ob.Nh, T);
             const V3 Tb = (-os) * ob.Nh;
@@ -203,25 +222,12 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
             r_b += (-rsh * id) * Tb;
             c_b += (-id) * Tb;
         }
-        // wh = Wh x r - u, wp = Wp x r - u, c = r x u
-        cross_adj(I.Wh, r, wh_b, Wh_b, r_b);
-        u_b -= wh_b;
-        cross_adj(I.Wp, r, wp_b, Wp_b, r_b);
-        u_b -= wp_b;
-        cross_adj(r, u, c_b, r_b, u_b);
-        // f3 = -3 K2 Ck / d7 - 2 vr SA / d8
-        const double Ck_b = f3_b * (-3. * G_K2 / d7);
-        d7_b += f3_b * (3. * G_K2 * Ck * id7 * id7);
-        vr_b += f3_b * (-2. * SA / d8);
-        const double SA_b = f3_b * (-2. * vr / d8);
-        d8_b += f3_b * (2. * vr * SA * id8 * id8);
+        if (FP || FH) cross_adj(r, u, c_b, r_b, u_b);   // c = r x u
         // os = Ah / d7, op = Ap / d7
         const double Ah_b = os_b * id7 + SA_b, Ap_b = op_b * id7 + SA_b;
         d7_b += -(os_b * (Ah * id7 * id7)) - op_b * (Ap * id7 * id7);
         Pb.sh += Ah_b * Ah_c;
         Pb.sp += Ap_b * Ap_c;
-        Pb.k2h += Ck_b * Kh;
-        Pb.k2p += Ck_b * Kp;
     }
     if (C.flat) {
         const double Bh_c = C.mp * pw5(C.Rh) / 6., Bp_c = C.mh * pw5(C.Rp) / 6.;
@@ -230,36 +236,48 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
         const double ofs = -6. * Bh * rsh / d5, ofp = -6. * Bp * rsp / d5;
         const double radf = -3. * (Bp * Wp2 + Bh * Wh2) / d5 + 15. * (Bh * rsh * rsh + Bp * rsp * rsp) / d7;
         const V3 Fb = ob.F;
-        // F_f = radf r + ofp Wp + ofs Wh
-        const double radf_b = dot(Fb, r);
-        r_b += radf * Fb;
-        double ofp_b = dot(Fb, I.Wp), ofs_b = dot(Fb, I.Wh);
-        Wp_b += ofp * Fb;
-        Wh_b += ofs * Fb;
+        double ofp_b = 0., ofs_b = 0., Bp_b = 0., Bh_b = 0.;
+        if (FA) {
+            // F_f = radf r + ofp Wp + ofs Wh
+            const double radf_b = dot(Fb, r);
+            r_b += radf * Fb;
+            ofp_b = dot(Fb, I.Wp);
+            ofs_b = dot(Fb, I.Wh);
+            Wp_b += ofp * Fb;
+            Wh_b += ofs * Fb;
+            // radf
+            const double Wp2_b = radf_b * (-3. * Bp / d5), Wh2_b = radf_b * (-3. * Bh / d5);
+            d5_b += radf_b * (3. * (Bp * Wp2 + Bh * Wh2) * id5 * id5);
+            rsh_b += radf_b * (30. * Bh * rsh * id7);
+            rsp_b += radf_b * (30. * Bp * rsp * id7);
+            d7_b += -radf_b * (15. * (Bh * rsh * rsh + Bp * rsp * rsp) * id7 * id7);
+            Bp_b = radf_b * (-3. * Wp2 / d5 + 15. * rsp * rsp / d7);
+            Bh_b = radf_b * (-3. * Wh2 / d5 + 15. * rsh * rsh / d7);
+            Wh_b += (2. * Wh2_b) * I.Wh;
+            Wp_b += (2. * Wp2_b) * I.Wp;
+        }
         // N_fp = -ofp (r x Wp), N_fh = -ofs (r x Wh)
-        ofp_b += -dot(ob.Np, cross(r, I.Wp));
-        cross_adj(r, I.Wp, (-ofp) * ob.Np, r_b, Wp_b);
-        ofs_b += -dot(ob.Nh, cross(r, I.Wh));
-        cross_adj(r, I.Wh, (-ofs) * ob.Nh, r_b, Wh_b);
-        // radf
-        const double Wp2_b = radf_b * (-3. * Bp / d5), Wh2_b = radf_b * (-3. * Bh / d5);
-        d5_b += radf_b * (3. * (Bp * Wp2 + Bh * Wh2) * id5 * id5);
-        rsh_b += radf_b * (30. * Bh * rsh * id7);
-        rsp_b += radf_b * (30. * Bp * rsp * id7);
-        d7_b += -radf_b * (15. * (Bh * rsh * rsh + Bp * rsp * rsp) * id7 * id7);
-        double Bp_b = radf_b * (-3. * Wp2 / d5 + 15. * rsp * rsp / d7);
-        double Bh_b = radf_b * (-3. * Wh2 / d5 + 15. * rsh * rsh / d7);
+        if (FP) {
+            ofp_b += -dot(ob.Np, cross(r, I.Wp));
+            cross_adj(r, I.Wp, (-ofp) * ob.Np, r_b, Wp_b);
+        }
+        if (FH) {
+            ofs_b += -dot(ob.Nh, cross(r, I.Wh));
+            cross_adj(r, I.Wh, (-ofs) * ob.Nh, r_b, Wh_b);
+        }
         // ofs, ofp
-        Bh_b += ofs_b * (-6. * rsh / d5);
-        rsh_b += ofs_b * (-6. * Bh / d5);
-        d5_b += ofs_b * (6. * Bh * rsh * id5 * id5);
-        Bp_b += ofp_b * (-6. * rsp / d5);
-        rsp_b += ofp_b * (-6. * Bp / d5);
-        d5_b += ofp_b * (6. * Bp * rsp * id5 * id5);
-        Wh_b += (2. * Wh2_b) * I.Wh;
-        Wp_b += (2. * Wp2_b) * I.Wp;
-        Pb.kfh += Bh_b * Bh_c;
-        Pb.kfp += Bp_b * Bp_c;
+        if (FA || FH) {
+            Bh_b += ofs_b * (-6. * rsh / d5);
+            rsh_b += ofs_b * (-6. * Bh / d5);
+            d5_b += ofs_b * (6. * Bh * rsh * id5 * id5);
+            Pb.kfh += Bh_b * Bh_c;
+        }
+        if (FA || FP) {
+            Bp_b += ofp_b * (-6. * rsp / d5);
+            rsp_b += ofp_b * (-6. * Bp / d5);
+            d5_b += ofp_b * (6. * Bp * rsp * id5 * id5);
+            Pb.kfp += Bp_b * Bp_c;
+        }
     }
     if (C.gr) {
         const double mgh = G_K2 * C.mh, mgp = G_K2 * C.mp, mg = mgh + mgp;
@@ -275,31 +293,33 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
         const double rad = mgc * P1 + mgc * P2;
         const double orth = -mgc * 2. * (2. - f) * vr - 0.5 * mgc * vr * Q2;
         const V3 gb = ob.g;
-        // g12 = rad id r + orth u
-        const double rdot = dot(gb, r);
-        const double rad_b = id * rdot;
-        id_b += rad * rdot;
-        r_b += (rad * id) * gb;
-        const double orth_b = dot(gb, u);
-        u_b += orth * gb;
-        double mgc_b = rad_b * (P1 + P2) + orth_b * (-2. * (2. - f) * vr - 0.5 * vr * Q2);
-        vr_b += orth_b * (-mgc * 2. * (2. - f) - 0.5 * mgc * Q2);
-        const double P1_b = rad_b * mgc, P2_b = rad_b * mgc, Q2_b = orth_b * (-0.5 * mgc * vr);
-        double mgd_b = 0., vr2_b = 0.;
-        // P1
-        u2_b += P1_b * (1. + 3. * f);
-        mgd_b += P1_b * (-2. * (2. + f));
-        vr2_b += P1_b * (-1.5 * f);
-        // P2
-        d2_b += P2_b * (-0.75 * (12. + 29. * f) * mg * mg / (d2 * d2));
-        u2_b += P2_b * (f * (3. - 4. * f) * 2. * u2 - 1.5 * f * (3. - 4. * f) * vr2 - 0.5 * f * (13. - 4. * f) * mgd);
-        vr2_b += P2_b * (15. / 8. * f * (1. - 3. * f) * 2. * vr2 - 1.5 * f * (3. - 4. * f) * u2
-                         - (2. + 25. * f + 2. * f * f) * mgd);
-        mgd_b += P2_b * (-0.5 * f * (13. - 4. * f) * u2 - (2. + 25. * f + 2. * f * f) * vr2);
-        // Q2
-        u2_b += Q2_b * f * (15. + 4. * f);
-        mgd_b += Q2_b * (-(4. + 41. * f + 8. * f * f));
-        vr2_b += Q2_b * (-3. * f * (3. + 2. * f));
+        double mgc_b = 0., mgd_b = 0., vr2_b = 0.;
+        if (FA) {
+            // g12 = rad id r + orth u
+            const double rdot = dot(gb, r);
+            const double rad_b = id * rdot;
+            id_b += rad * rdot;
+            r_b += (rad * id) * gb;
+            const double orth_b = dot(gb, u);
+            u_b += orth * gb;
+            mgc_b = rad_b * (P1 + P2) + orth_b * (-2. * (2. - f) * vr - 0.5 * vr * Q2);
+            vr_b += orth_b * (-mgc * 2. * (2. - f) - 0.5 * mgc * Q2);
+            const double P1_b = rad_b * mgc, P2_b = rad_b * mgc, Q2_b = orth_b * (-0.5 * mgc * vr);
+            // P1
+            u2_b += P1_b * (1. + 3. * f);
+            mgd_b += P1_b * (-2. * (2. + f));
+            vr2_b += P1_b * (-1.5 * f);
+            // P2
+            d2_b += P2_b * (-0.75 * (12. + 29. * f) * mg * mg / (d2 * d2));
+            u2_b += P2_b * (f * (3. - 4. * f) * 2. * u2 - 1.5 * f * (3. - 4. * f) * vr2 - 0.5 * f * (13. - 4. * f) * mgd);
+            vr2_b += P2_b * (15. / 8. * f * (1. - 3. * f) * 2. * vr2 - 1.5 * f * (3. - 4. * f) * u2
+                             - (2. + 25. * f + 2. * f * f) * mgd);
+            mgd_b += P2_b * (-0.5 * f * (13. - 4. * f) * u2 - (2. + 25. * f + 2. * f * f) * vr2);
+            // Q2
+            u2_b += Q2_b * f * (15. + 4. * f);
+            mgd_b += Q2_b * (-(4. + 41. * f + 8. * f * f));
+            vr2_b += Q2_b * (-3. * f * (3. + 2. * f));
+        }
         // spin-orbit
         const double fa = G_K2 / C2;
         const V3 Ls = C.Ih * I.Wh, Lp = C.Ip * I.Wp;
@@ -311,20 +331,22 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
         const V3 nu = cross(n, u);
         V3 n_b = zero3(), nu_b = zero3(), e7_b = zero3(), e3_b = zero3(), e2_b = zero3();
         V3 Ls_b = zero3(), Lp_b = zero3(), Lo_b = zero3();
-        // a3 = fa (e1 - u x e7 + 3 vr (n x e3)),  e1 = 6 n * nu * e2 (component-wise)
-        const V3 e1_b = fa * gb;
-        cross_adj(u, e7, (-fa) * gb, u_b, e7_b);
-        cross_adj(n, e3, (3. * fa * vr) * gb, n_b, e3_b);
-        vr_b += 3. * fa * dot(gb, cross(n, e3));
-        n_b += 6. * hadamard(hadamard(e1_b, nu), e2);
-        nu_b += 6. * hadamard(hadamard(e1_b, n), e2);
-        e2_b += 6. * hadamard(hadamard(e1_b, n), nu);
-        cross_adj(n, u, nu_b, n_b, u_b);
+        if (FA) {
+            // a3 = fa (e1 - u x e7 + 3 vr (n x e3)),  e1 = 6 n * nu * e2 (component-wise)
+            const V3 e1_b = fa * gb;
+            cross_adj(u, e7, (-fa) * gb, u_b, e7_b);
+            cross_adj(n, e3, (3. * fa * vr) * gb, n_b, e3_b);
+            vr_b += 3. * fa * dot(gb, cross(n, e3));
+            n_b += 6. * hadamard(hadamard(e1_b, nu), e2);
+            nu_b += 6. * hadamard(hadamard(e1_b, n), e2);
+            e2_b += 6. * hadamard(hadamard(e1_b, n), nu);
+            cross_adj(n, u, nu_b, n_b, u_b);
+        }
         // torques
         const double mu = C.mh * C.mp / (C.mh + C.mp);
         const V3 Lo = mu * cross(r, u);
         const double fmh = 2. + 1.5 * C.mp / C.mh, fmp = 2. + 1.5 * C.mh / C.mp;
-        {
+        if (FH) {
             const V3 q = fa * ob.Nh;
             cross_adj(Lo, Ls, fmh * q, Lo_b, Ls_b);
             cross_adj(Lp, Ls, -q, Lp_b, Ls_b);
@@ -334,7 +356,7 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
             n_b += s1_b * Lp;
             Lp_b += s1_b * n;
         }
-        {
+        if (FP) {
             const V3 q = fa * ob.Np;
             cross_adj(Lo, Lp, fmp * q, Lo_b, Lp_b);
             cross_adj(Ls, Lp, -q, Ls_b, Lp_b);
@@ -344,11 +366,13 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
             n_b += s2_b * Ls;
             Ls_b += s2_b * n;
         }
-        cross_adj(r, u, mu * Lo_b, r_b, u_b);
-        const V3 S_b = 7. * e7_b + 3. * e3_b + 2. * e2_b;
-        const V3 msf_b = 3. * e7_b + e3_b + e2_b;
-        Lp_b += (dm / C.mp) * msf_b + S_b;
-        Ls_b += (-(dm / C.mh)) * msf_b + S_b;
+        if (FP || FH) cross_adj(r, u, mu * Lo_b, r_b, u_b);
+        if (FA) {
+            const V3 S_b = 7. * e7_b + 3. * e3_b + 2. * e2_b;
+            const V3 msf_b = 3. * e7_b + e3_b + e2_b;
+            Lp_b += (dm / C.mp) * msf_b + S_b;
+            Ls_b += (-(dm / C.mh)) * msf_b + S_b;
+        }
         Wh_b += C.Ih * Ls_b;
         Wp_b += C.Ip * Lp_b;
         // n = id r
@@ -378,6 +402,11 @@ POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, cons
     Ib.u += u_b;
     Ib.Wh += Wh_b;
     Ib.Wp += Wp_b;
+}
+
+POS_HD void pair_vjp(const PairConst &C, const PairPar &P, const PairIn &I, const PairOut &ob, PairIn &Ib,
+                     PairParBar &Pb) {
+    pair_vjp_of<true, true, true>(C, P, I, ob, Ib, Pb);
 }
 
 // ---------------------------------------------------------------------------

@@ -1,5 +1,5 @@
-// adjoint_sweep.hpp -- the reverse sweep in two kernels, for ensembles that
-// leave most of the chip idle.
+// adjoint_sweep.hpp -- the reverse sweep in two parts, for ensembles that leave
+// most of the chip idle.
 //
 // The reverse of a step is linear in the cotangents and everything else in it
 // follows from the tape: only the chain of small products below is serial.
@@ -7,11 +7,12 @@
 // writes the coefficients of every product of a stretch of steps;
 // sweep_stretch walks the stretch backwards and only multiplies.  In place of
 // 40 us a step (one wavefront a SIMD at most, 11,000 vector instructions in
-// one chain) the preparation, spread over the chip, takes 5.4 us and the sweep
-// 6.7 us, bound by the latency of its 20 exchanges through LDS (1,024 systems of
-// four bodies).  An ensemble that fills the chip is bound by its instructions,
-// not by their chain, and would be by the coefficients' traffic (3 KB a body
-// and step each way): there adjoint_segment_kernel, which keeps nothing, is
+// one chain) the preparation, spread over the chip, takes 4.6 us and the sweep
+// 5.4 us, bound by the latency of its 20 exchanges through LDS; both at once 7.4
+// us (1,024 systems of four bodies).  An ensemble that fills the chip is bound by
+// its instructions, not by their chain, and would be by the coefficients'
+// traffic (3 KB a body and step each way): there adjoint_segment_kernel, which
+// keeps nothing, is
 // the faster one.
 //
 // Coefficients of a step, planes of two doubles per body, body fastest:
@@ -54,39 +55,45 @@ struct PrepareLds {
 };
 
 // The coefficients of one kick: the columns of the pair's vector-Jacobian
-// product (a host's are zero but for its own wind torque).
-__device__ inline void write_kick(const Coefficients &Cf, int t, int plane, const AdjLane &A, const KickPoint &K,
-                                  double h) {
+// product (a host's are zero but for its own wind torque).  KIND: the three
+// columns of the acceleration's cotangent, of dL_p/dt's or of dL_h/dt's, each of
+// which needs its part of the product only.
+template <int KIND>
+__device__ __forceinline__ void write_kick_columns(const Coefficients &Cf, int t, int plane, const AdjLane &A,
+                                                   const KickPoint &K, double h) {
     const double hh = 0.5 * h;
     const double im = 1. / A.m, sI = hh / A.I, sIh = hh / A.Ih;
+    const size_t nb = Cf.n_bodies;
 #pragma unroll 1
-    for (int i = 0; i < 9; ++i) {
-        const V3 e{i % 3 == 0 ? 1. : 0., i % 3 == 1 ? 1. : 0., i % 3 == 2 ? 1. : 0.};
+    for (int i = 0; i < 3; ++i) {
+        const V3 e{i == 0 ? 1. : 0., i == 1 ? 1. : 0., i == 2 ? 1. : 0.};
         const V3 z{0., 0., 0.};
         posadj::PairIn Ib{z, z, z, z};
         posadj::PairParBar Pb{0., 0., 0., 0., 0., 0.};
         if (A.orbiting()) {
-            const V3 ea = i < 3 ? e : z;
             // the force on the body and its acceleration enter as F / m + g
-            const posadj::PairOut ob{im * ea, ea, i >= 3 && i < 6 ? e : z, i >= 6 ? e : z};
-            posadj::pair_vjp(K.C, K.P, K.in, ob, Ib, Pb);
+            const posadj::PairOut ob{KIND == 0 ? im * e : z, KIND == 0 ? e : z, KIND == 1 ? e : z, KIND == 2 ? e : z};
+            posadj::pair_vjp_of<KIND == 0, KIND == 1, KIND == 2>(K.C, K.P, K.in, ob, Ib, Pb);
         }
-        if (A.wind && i >= 3 && i < 6) Ib.Wp += wind_vjp(A, K.in.Wp, e);
+        if (KIND == 1 && A.wind) Ib.Wp += wind_vjp(A, K.in.Wp, e);
         const V3 U = hh * Ib.u, P = sI * Ib.Wp, H = sIh * Ib.Wh, R = h * Ib.r;
-        double2 *o = Cf.at(t, plane + 6 * i, A.body);
-        const size_t nb = Cf.n_bodies;
+        double2 *o = Cf.at(t, plane + 6 * (3 * KIND + i), A.body);
         o[0] = double2{U.x, P.x}; o[nb] = double2{U.y, P.y}; o[2 * nb] = double2{U.z, P.z};
         o[3 * nb] = double2{H.x, R.x}; o[4 * nb] = double2{H.y, R.y}; o[5 * nb] = double2{H.z, R.z};
         const double2 ph{h * Pb.sh, h * Pb.kfh}, pp{h * Pb.sp, h * Pb.kfp};
-        if (i < 3) {
+        if (KIND == 0) {
             double2 *q = Cf.at(t, plane + 54 + 3 * i, A.body);
             q[0] = ph; q[nb] = pp; q[2 * nb] = double2{h * Pb.k2h, h * Pb.k2p};
-        } else if (i < 6) {
-            *Cf.at(t, plane + 63 + 2 * (i - 3) + 1, A.body) = pp;
         } else {
-            *Cf.at(t, plane + 63 + 2 * (i - 6), A.body) = ph;
+            *Cf.at(t, plane + 63 + 2 * i + (KIND == 1 ? 1 : 0), A.body) = KIND == 1 ? pp : ph;
         }
     }
+}
+__device__ inline void write_kick(const Coefficients &Cf, int t, int plane, const AdjLane &A, const KickPoint &K,
+                                  double h) {
+    write_kick_columns<0>(Cf, t, plane, A, K, h);
+    write_kick_columns<1>(Cf, t, plane, A, K, h);
+    write_kick_columns<2>(Cf, t, plane, A, K, h);
 }
 
 // The coefficients of one Kepler drift; N: the interaction's indirect term at Q,
@@ -112,10 +119,10 @@ __device__ inline void write_drift(const Coefficients &Cf, int t, int plane, con
 // workspace: the first kick's, or all others; slots: the chain positions the
 // sweep's kernel reads.
 template <bool ALT, bool EVO>
-__device__ inline void prepare_step(const AdjArgs &Ar, PrepareLds &L, AdjLane &A, const Coefficients &Cf, int row, int t,
+__device__ inline void prepare_step(const TapeRef &T, PrepareLds &L, AdjLane &A, const Coefficients &Cf, int row, int t,
                                     int slots, bool first_kick) {
-    const StepTape S = step_tape(Ar.T, A, row);
-    step_radii<EVO>(Ar.T, L, A, row);
+    const StepTape S = step_tape(T, A, row);
+    step_radii<EVO>(T, L, A, row);
     const double h = 0.5 * A.dt;
     if (first_kick) {
         wsync();
@@ -503,15 +510,25 @@ __device__ __forceinline__ void sweep_store(const AdjArgs &Ar, SweepLds &S, cons
     if (A.c == 2) Ar.gk2[A.body] += A.orb ? A.p1 : s0;
 }
 
-// Steps row0 + len - 1 down to row0 of the segment, whose coefficients are
-// steps len - 1 .. 0 of the workspace.
+// Steps [row0, row0 + len) of a segment and where their coefficients are, as the
+// workspace's steps 0 .. len - 1.
+struct Stretch {
+    TapeRef T;
+    long long seg_start;
+    int row0, len;
+    Coefficients Cf;
+};
+
+// The reverse of a stretch, last step first.
 template <int NM, bool ALT>
-__device__ inline void sweep_stretch(const AdjArgs &Ar, SweepLds &S, const Coefficients &Cf, int row0, int len) {
+__device__ inline void sweep_stretch(const AdjArgs &Ar, SweepLds &S, const Stretch &W) {
+    const Coefficients &Cf = W.Cf;
+    const int len = W.len;
     SweepLane A;
     int sys;
     bool jacobi;
     sweep_load<NM>(Ar, S, A, sys, jacobi);
-    const long long done = Ar.steps_done[sys] - Ar.seg_start - row0;   // steps of the stretch the system took
+    const long long done = Ar.steps_done[sys] - W.seg_start - W.row0;   // steps of the stretch the system took
     const unsigned long long group = (NM == 16 ? ~0ull : ((1ull << (4 * NM % 64)) - 1) << A.g0);
     // Each part's coefficients are asked for a part or more before their use:
     // while a kick runs, those of the drifts and of the step's other kick (at 16

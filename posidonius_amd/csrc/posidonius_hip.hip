@@ -298,24 +298,27 @@ __global__ __launch_bounds__(64) void adjoint_segment_kernel(AdjArgs Ar) {
     }
 }
 
-// The coefficients of steps [row0, row0 + len) of the recorded segment: one
-// wavefront per set of systems, step and part of the step.
-template <bool ALT, bool EVO>
-__global__ __launch_bounds__(64) void adjoint_prepare_kernel(AdjArgs Ar, Coefficients Cf, int row0, int len, int slots) {
-    __shared__ PrepareLds L;
-    const int part = blockIdx.x / Ar.E.n_waves, t = part >> 1;
-    if (t >= len) return;
+// The sweep of one stretch of steps, by the first workgroups (16 / NM systems
+// each), and the coefficients of the next one by the others, one wavefront per set
+// of systems, step and part of the step.  Either may be empty.  One launch of
+// both keeps the few long wavefronts of the sweep from waiting for SIMDs that the
+// many of the preparation hold: 1,024 systems of four bodies, 10 steps: 79 us,
+// against 58 and 49 us one after the other and 97 in two streams.  ALT, EVO: see
+// adjoint_segment_kernel.
+template <int NM, bool ALT, bool EVO>
+__global__ __launch_bounds__(64) void adjoint_stretch_kernel(AdjArgs Ar, Stretch sweep, Stretch prepare) {
+    __shared__ union { PrepareLds prepare; SweepLds sweep; } lds;
+    const int sweeps = sweep.len > 0 ? (Ar.E.n_systems + 16 / NM - 1) / (16 / NM) : 0;
+    if ((int)blockIdx.x < sweeps) {
+        sweep_stretch<NM, ALT>(Ar, lds.sweep, sweep);
+        return;
+    }
+    const int part = (blockIdx.x - sweeps) / Ar.E.n_waves, t = part >> 1;
+    if (t >= prepare.len) return;
     AdjLane A;
-    adjoint_load(Ar, L, A, blockIdx.x - part * Ar.E.n_waves);
-    if (Ar.seg_start + row0 + t < A.done) prepare_step<ALT, EVO>(Ar, L, A, Cf, row0 + t, t, slots, part & 1);
-}
-
-// Reverse sweep over those steps, last step first: 16 / NM systems per wavefront.
-template <int NM, bool ALT>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2)))
-void adjoint_sweep_kernel(AdjArgs Ar, Coefficients Cf, int row0, int len) {
-    __shared__ SweepLds S;
-    sweep_stretch<NM, ALT>(Ar, S, Cf, row0, len);
+    adjoint_load(Ar, lds.prepare, A, blockIdx.x - sweeps - part * Ar.E.n_waves);
+    if (prepare.seg_start + prepare.row0 + t < A.done)
+        prepare_step<ALT, EVO>(prepare.T, lds.prepare, A, prepare.Cf, prepare.row0 + t, t, NM, part & 1);
 }
 
 // initialize_physical_values (whfast.rs:226-233) for systems at t == 0:
@@ -583,7 +586,6 @@ struct pos_ens {
         // the prepared sweep's coefficients: two halves of `stretch` steps,
         // systems of at most `slots` bodies; none: the sweep in one kernel
         double2 *coef = nullptr;
-        hipEvent_t prepared_ev[2] = {nullptr, nullptr}, spent_ev[2] = {nullptr, nullptr};   // of each half
         int stretch = 0, slots = 0;
         std::vector<void *> allocs;
     } adj;
@@ -1019,7 +1021,7 @@ double host_roche(double ma, double mb, double ra, double rb) {
 void adjoint_release(pos_ens *h) {
     pos_ens::Adjoint &A = h->adj;
     for (void *p : A.allocs) (void)hipFree(p);
-    for (hipEvent_t *e : {A.taped_ev, A.swept_ev, A.prepared_ev, A.spent_ev})
+    for (hipEvent_t *e : {A.taped_ev, A.swept_ev})
         for (int i = 0; i < 2; ++i)
             if (e[i]) (void)hipEventDestroy(e[i]);
     if (A.sweep) (void)hipStreamDestroy(A.sweep);
@@ -1172,12 +1174,14 @@ int launch_steps(pos_ens *h, int n_steps, int *launches = nullptr) {
 }
 
 // The prepared sweep's workspace, if this ensemble is one it serves better: up to
-// one set of systems per CU.  The whole adjoint of 32 steps took, in one kernel
-// and prepared, us a step: 128 sets of four bodies each 66.9 and 44.8, 256 sets
-// 70.2 and 59.9, 384 sets 76.1 and 83.3; of 2 to 12 bodies 118 sets 96.5 and
-// 69.2, 243 sets 101.7 and 100.8, 487 sets 117 and 170.  The workspace is
-// bounded, a segment is swept by stretches of the steps that fit; without
-// memory for a single one the sweep is the one kernel's.
+// one set of systems per CU.  The adjoint of 32 steps in one kernel and
+// prepared, us a step: 128 sets of systems of four bodies 48.1 and 23.1, 256
+// sets 51.1 and 38.9, 384 sets 56.4 and 63.3; of 2 to 12 bodies 118 sets 74.8 and
+// 36.2, 243 sets 79.9 and 66.9, 487 sets 90.5 and 137; of two bodies 128 sets
+// 42.1 and 26.4, 256 sets 44.4 and 46.5; of 16 bodies 256 sets 93.8 and 50.7.
+// The workspace (two halves, one swept while the other is filled) is bounded, a
+// segment is swept by stretches of the steps that fit; without memory for a
+// single one the sweep is the one kernel's.
 constexpr int PREPARED_SETS_PER_CU = 1;
 constexpr size_t COEFFICIENT_BYTES = (size_t)256 << 20;
 void plan_prepared_sweep(pos_ens *h, int seg) {
@@ -1199,43 +1203,44 @@ void plan_prepared_sweep(pos_ens *h, int seg) {
     A.slots = slots;
 }
 
-// One segment's sweep, last step first, once its tape is there (`taped`); `swept` is
-// recorded where the tape has been read.  The prepared sweep's coefficients are
-// formed on the handle's stream, where the tape was written, a stretch ahead of
-// the sweep's own; `stretches` counts those launched.
-int launch_sweep(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo, int &stretches, hipEvent_t taped, hipEvent_t swept) {
+// One stretch's sweep and the next one's preparation, on the adjoint's stream.
+int launch_stretch(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo, const Stretch &sweep, const Stretch &prepare) {
     const pos_ens::Adjoint &A = h->adj;
-    if (!A.coef) {
+    const bool general = alt || evo;
+    auto kernel = A.slots == 4 ? (general ? adjoint_stretch_kernel<4, true, true> : adjoint_stretch_kernel<4, false, false>)
+                : A.slots == 8 ? (general ? adjoint_stretch_kernel<8, true, true> : adjoint_stretch_kernel<8, false, false>)
+                               : (general ? adjoint_stretch_kernel<16, true, true> : adjoint_stretch_kernel<16, false, false>);
+    const int per_wave = 16 / A.slots;
+    const int blocks = (sweep.len > 0 ? (h->n_systems + per_wave - 1) / per_wave : 0) + 2 * h->E.n_waves * prepare.len;
+    hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, A.sweep, Ar, sweep, prepare);
+    HIP_TRY(hipGetLastError());
+    return POS_OK;
+}
+
+// One segment's sweep, last step first, once its tape is there (`taped`); `swept` is
+// recorded where the tape has been read.  Prepared: `last` is the stretch
+// whose coefficients wait for their sweep.
+int launch_sweep(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo, Stretch &last, hipEvent_t taped, hipEvent_t swept) {
+    const pos_ens::Adjoint &A = h->adj;
+    HIP_TRY(hipStreamWaitEvent(A.sweep, taped, 0));
+    if (A.coef) {
+        const int planes = coefficient_planes(A.slots);
+        double2 *const half = A.coef + (size_t)A.stretch * planes * h->n_bodies;
+        for (int end = Ar.seg_len, rc; end > 0;) {
+            const int len = std::min(A.stretch, end), row0 = end - len;
+            const Stretch next{Ar.T, Ar.seg_start, row0, len,
+                               Coefficients{last.Cf.base == A.coef ? half : A.coef, planes, h->n_bodies}};
+            if ((rc = launch_stretch(h, Ar, alt, evo, last, next))) return rc;
+            last = next;
+            end = row0;
+        }
+    } else {
         auto kernel = alt ? (evo ? adjoint_segment_kernel<true, true> : adjoint_segment_kernel<true, false>)
                           : (evo ? adjoint_segment_kernel<false, true> : adjoint_segment_kernel<false, false>);
-        HIP_TRY(hipStreamWaitEvent(A.sweep, taped, 0));
         hipLaunchKernelGGL(kernel, dim3(h->grid), dim3(64), 0, A.sweep, Ar);
         HIP_TRY(hipGetLastError());
-        HIP_TRY(hipEventRecord(swept, A.sweep));
-        return POS_OK;
     }
-    const int planes = coefficient_planes(A.slots);
-    auto prepare = alt ? (evo ? adjoint_prepare_kernel<true, true> : adjoint_prepare_kernel<true, false>)
-                       : (evo ? adjoint_prepare_kernel<false, true> : adjoint_prepare_kernel<false, false>);
-    auto sweep = A.slots == 4 ? (alt ? adjoint_sweep_kernel<4, true> : adjoint_sweep_kernel<4, false>)
-               : A.slots == 8 ? (alt ? adjoint_sweep_kernel<8, true> : adjoint_sweep_kernel<8, false>)
-                              : (alt ? adjoint_sweep_kernel<16, true> : adjoint_sweep_kernel<16, false>);
-    const int per_wave = 16 / A.slots;
-    for (int end = Ar.seg_len; end > 0;) {
-        const int len = std::min(A.stretch, end), row0 = end - len, half = stretches & 1;
-        const Coefficients Cf{A.coef + (size_t)half * A.stretch * planes * h->n_bodies, planes, h->n_bodies};
-        if (stretches >= 2) HIP_TRY(hipStreamWaitEvent(h->stream, A.spent_ev[half], 0));
-        hipLaunchKernelGGL(prepare, dim3(2 * h->E.n_waves * len), dim3(64), 0, h->stream, Ar, Cf, row0, len, A.slots);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipEventRecord(A.prepared_ev[half], h->stream));
-        HIP_TRY(hipStreamWaitEvent(A.sweep, A.prepared_ev[half], 0));
-        hipLaunchKernelGGL(sweep, dim3((h->n_systems + per_wave - 1) / per_wave), dim3(64), 0, A.sweep, Ar, Cf, row0, len);
-        HIP_TRY(hipGetLastError());
-        HIP_TRY(hipEventRecord(A.spent_ev[half], A.sweep));
-        end = row0;
-        ++stretches;
-    }
-    HIP_TRY(hipEventRecord(swept, h->stream));   // only the preparation reads the tape
+    HIP_TRY(hipEventRecord(swept, A.sweep));
     return POS_OK;
 }
 
@@ -1306,7 +1311,7 @@ int adjoint_allocate(pos_ens *h, int64_t n_steps, int seg) {
         return rc;
     plan_prepared_sweep(h, seg);
     HIP_TRY(hipStreamCreateWithFlags(&A.sweep, hipStreamNonBlocking));
-    for (hipEvent_t *e : {A.taped_ev, A.swept_ev, A.prepared_ev, A.spent_ev})
+    for (hipEvent_t *e : {A.taped_ev, A.swept_ev})
         for (int i = 0; i < 2; ++i) HIP_TRY(hipEventCreateWithFlags(&e[i], hipEventDisableTiming));
     A.seg = seg;
     A.n_seg = (int)n_seg;
@@ -2240,7 +2245,7 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
                                  [](int c) { return c != POS_COORD_DEMOCRATIC_HELIOCENTRIC; });
     const bool evo = std::any_of(h->eff_dev.begin(), h->eff_dev.end(),
                                  [](uint32_t e) { return (e & POS_EFFECT_EVOLUTION) != 0; });
-    int stretches = 0;
+    Stretch last{};
     for (int s = A.n_seg - 1; s >= std::max(0, A.n_seg - 2); --s)
         if ((rc = taped(s))) return rc;
     for (int s = A.n_seg - 1; s >= 0; --s) {
@@ -2248,12 +2253,13 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
         Ar.T = TapeRef{A.tape + slot * A.tape_values, nb};
         Ar.seg_start = (int64_t)s * A.seg;
         Ar.seg_len = seg_len(s);
-        if ((rc = launch_sweep(h, Ar, alt, evo, stretches, A.taped_ev[slot & 1], A.swept_ev[slot & 1]))) return rc;
+        if ((rc = launch_sweep(h, Ar, alt, evo, last, A.taped_ev[slot & 1], A.swept_ev[slot & 1]))) return rc;
         if (!keep && s >= 2) {
             HIP_TRY(hipStreamWaitEvent(h->stream, A.swept_ev[slot & 1], 0));
             if ((rc = taped(s - 2))) return rc;
         }
     }
+    if (last.len > 0 && (rc = launch_stretch(h, Ar, alt, evo, last, Stretch{}))) return rc;
     HIP_TRY(hipEventRecord(A.swept_ev[0], A.sweep));
     HIP_TRY(hipStreamWaitEvent(h->stream, A.swept_ev[0], 0));
     if (recomputed && (rc = adjoint_copy_state(h, A.final_state, false))) return rc;
