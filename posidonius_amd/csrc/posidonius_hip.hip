@@ -675,6 +675,19 @@ int read_back(pos_ens *h, const std::vector<ReadRequest> &want) {
         if (fits) total += bytes(w);
         (fits ? packed : direct).push_back(&w);
     }
+    if (h->pinned_bytes < total) {
+        if (h->pinned) (void)hipHostFree(h->pinned);
+        h->pinned = nullptr;
+        h->pinned_bytes = 0;
+        if (hipHostMalloc((void **)&h->pinned, total, hipHostMallocDefault) == hipSuccess) {
+            h->pinned_bytes = total;
+        } else {   // no pinned memory to be had: field by field
+            (void)hipGetLastError();
+            h->pinned = nullptr;
+            direct.insert(direct.end(), packed.begin(), packed.end());
+            packed.clear();
+        }
+    }
     int rc;
     std::vector<char> buf;
     for (const ReadRequest *w : direct) {
@@ -690,13 +703,6 @@ int read_back(pos_ens *h, const std::vector<ReadRequest> &want) {
         for (int d = 0; d < count; ++d) std::memcpy((char *)w->dst + perm[d] * each, buf.data() + d * each, each);
     }
     if (packed.empty()) return POS_OK;
-    if (h->pinned_bytes < total) {
-        if (h->pinned) (void)hipHostFree(h->pinned);
-        h->pinned = nullptr;
-        h->pinned_bytes = 0;
-        HIP_TRY(hipHostMalloc((void **)&h->pinned, total, hipHostMallocDefault));
-        h->pinned_bytes = total;
-    }
     ReadTable t{};
     size_t off = 0;
     int n = 0, most = 1;
