@@ -456,7 +456,7 @@ def main():
                                f"{traffic['model']} ({traffic['source']})") if traffic else None,
             "achieved_hbm_gbs": (traffic["bytes_per_launch"] / (kernel_ms * 1e-3) / 1e9) if traffic else None,
             "hbm_peak_gbs": HBM_PEAK_GBS,
-            "kernel": "whfast_steps_kernel",
+            "kernel": "whfast_fixed_kernel",
             "kernel_ms_per_launch": kernel_ms,
             "steps_per_launch": launch_steps,
             "flops_per_launch": flops_per_launch,

@@ -366,15 +366,18 @@ int32_t pos_history_drain(pos_ens *ens, pos_history_record *out, int64_t max_rec
  * No counterpart in the reference,
  * which has no derivatives; it differentiates the step of whfast.rs:235-305.
  *
- * pos_adjoint_record advances every system by n_steps like pos_step and
- * keeps a checkpoint of the state every segment_steps steps (0 = 1000).
+ * pos_adjoint_record advances every system by n_steps like pos_step, in
+ * segments of segment_steps steps (0 = 1000), and keeps each segment's step
+ * tape, or a checkpoint of the state at its start where all tapes together
+ * exceed 1 GiB (and are more than two).  Its buffers stay with the handle and
+ * serve the next recording of the same length.
  * pos_adjoint then returns the vector-Jacobian product of that run: from
  * the cotangents of the final position, velocity and spin angular momentum
  * (seed), the cotangents of the state at the start of the recording and the
  * gradients with respect to every body's CTL dissipation factor sigma
  * (dissipation_factor_scale * dissipation_factor), tidal Love number and
- * fluid Love number (grad).  It recomputes each segment from its checkpoint,
- * runs the reverse sweep over it, and leaves the ensemble's state where
+ * fluid Love number (grad).  It runs the reverse sweep over each segment,
+ * recomputed from its checkpoint where its tape was not kept, and leaves the ensemble's state where
  * pos_adjoint_record left it.  Arrays are in input body order, [3*nb] for
  * vectors and [nb] for parameters; NULL seed arrays count as zero and NULL
  * grad arrays are skipped.  Systems that stop early (completion or a fatal

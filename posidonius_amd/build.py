@@ -23,7 +23,8 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc", "posidonius_hip.hip")
-HEADERS = [os.path.join(HERE, "csrc", "whfast_step.hpp"),
+HEADERS = [*(os.path.join(HERE, "csrc", h) for h in ("whfast_step.hpp", "whfast_fixed.hpp", "adjoint_math.hpp",
+                                                     "adjoint_kernels.hpp", "adjoint_sweep.hpp", "crmath.hpp")),
            os.path.join(os.path.dirname(HERE), "include", "posidonius_hip.h")]
 OUT = os.path.join(HERE, "libposidonius_hip.so")
 ARCH = os.environ.get("POSIDONIUS_OFFLOAD_ARCH", "gfx950")

@@ -12,8 +12,7 @@
 // us (1,024 systems of four bodies).  An ensemble that fills the chip is bound by
 // its instructions, not by their chain, and would be by the coefficients'
 // traffic (3 KB a body and step each way): there adjoint_segment_kernel, which
-// keeps nothing, is
-// the faster one.
+// keeps nothing, is the faster one.
 //
 // Coefficients of a step, planes of two doubles per body, body fastest:
 //   each kick (the second one first), for every component i of the cotangents

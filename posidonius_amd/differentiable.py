@@ -2,10 +2,11 @@
 
 ``WHFastSteps`` is a ``torch.autograd.Function`` whose forward pass runs
 ``n_steps`` WHFast steps of every system on the GPU (``pos_adjoint_record``:
-the regular step kernel plus a state checkpoint every ``segment_steps``
-steps) and whose backward pass is the library's hand-written discrete adjoint
-(``pos_adjoint``: each segment is recomputed from its checkpoint while its
-step tape is recorded, then swept in reverse).  Inputs are the initial
+the regular steps, which also write the step tape of every ``segment_steps``
+steps, or of a run whose tapes would be too large a state checkpoint) and whose
+backward pass is the library's hand-written discrete adjoint (``pos_adjoint``:
+the segments are swept in reverse, one without a tape after its steps have
+been repeated from its checkpoint).  Inputs are the initial
 barycentric positions, velocities and spin angular momenta ([n_bodies, 3])
 and per-body log dissipation factors, tidal and fluid Love numbers
 ([n_bodies]); outputs are the final positions, velocities and spin angular
