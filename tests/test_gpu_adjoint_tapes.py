@@ -81,3 +81,31 @@ def test_recording_again_uses_the_new_run():
         ens.step(40)
         ens.adjoint_record(9, 4)
         np.testing.assert_array_equal(ens.adjoint(position=w)["position"], third["position"])
+
+
+@pytest.mark.parametrize("wind", [False, True], ids=["fixed_effect_set", "generic"])
+def test_recording_takes_the_historic_snapshots_of_stepping(wind):
+    """The recorded steps append the records that pos_step would; the adjoint
+    appends none."""
+    from posidonius_amd import abi
+    from posidonius_amd.ensemble import Ensemble
+    spec = gen.config2(30, seed=9, n_min=2, n_max=7)
+    spec.system["historic_snapshot_period"][:] = 3.3 * spec.system["time_step"]
+    if wind:
+        spec.system["effects"][:] |= abi.EFFECT_WIND
+    w = np.ones((spec.n_bodies, 3))
+    got = []
+    for record in (True, False):
+        with Ensemble(spec, mapping="packed") as ens:
+            ens.enable_history(16)
+            if record:
+                ens.adjoint_record(30, 11)
+                ens.adjoint(position=w)
+            else:
+                ens.step(30)
+            got.append((ens.drain_history(), ens.get_state()))
+    assert len(got[0][0]) > 0
+    for k in got[0][0].dtype.names:
+        np.testing.assert_array_equal(got[0][0][k], got[1][0][k], err_msg=k)
+    for k in got[0][1]:
+        np.testing.assert_array_equal(got[0][1][k], got[1][1][k], err_msg=k)
