@@ -222,6 +222,16 @@ typedef struct pos_state {
 #define POS_MAPPING_PLAIN       1   /* one system per wavefront, one step per launch */
 #define POS_MAPPING_PACKED      2   /* lane groups, K steps per launch      */
 
+/* Places in pos_options.reserved; 0 in each is the default. */
+#define POS_OPT_PERSISTENT_GRID 0     /* workgroups of a launch (0 = one per wavefront set)      */
+#define POS_OPT_ADJOINT_TAPE_MIB 1    /* most MiB of step tapes pos_adjoint_record keeps
+                                         (0 = 1024, negative = none beyond the last two)         */
+#define POS_OPT_ADJOINT_SWEEP 2       /* POS_ADJOINT_SWEEP_*                                     */
+
+#define POS_ADJOINT_SWEEP_AUTO 0      /* by the size of the ensemble                             */
+#define POS_ADJOINT_SWEEP_KERNEL 1    /* each segment in one kernel, no workspace                */
+#define POS_ADJOINT_SWEEP_PREPARED 2  /* coefficients in parallel, then a chain of products      */
+
 typedef struct pos_options {
     int32_t device;            /* HIP device ordinal                          */
     int32_t mapping;           /* POS_MAPPING_*                               */
@@ -231,7 +241,7 @@ typedef struct pos_options {
                                   sharing a wavefront, best-fit decreasing) */
     int32_t steps_per_launch;  /* K for PACKED (0 = default 64)               */
     int32_t use_graph;         /* capture chunk sequences in a hipGraph       */
-    int32_t reserved[3];
+    int32_t reserved[3];       /* POS_OPT_*                                   */
 } pos_options;
 
 typedef struct pos_ens pos_ens;   /* opaque */
@@ -369,7 +379,8 @@ int32_t pos_history_drain(pos_ens *ens, pos_history_record *out, int64_t max_rec
  * pos_adjoint_record advances every system by n_steps like pos_step, in
  * segments of segment_steps steps (0 = 1000), and keeps each segment's step
  * tape, or a checkpoint of the state at its start where all tapes together
- * exceed 1 GiB (and are more than two).  Its buffers stay with the handle and
+ * exceed 1 GiB (POS_OPT_ADJOINT_TAPE_MIB) or a quarter of the free device
+ * memory (and are more than two).  Its buffers stay with the handle and
  * serve the next recording of the same length.
  * pos_adjoint then returns the vector-Jacobian product of that run: from
  * the cotangents of the final position, velocity and spin angular momentum

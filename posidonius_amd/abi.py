@@ -78,6 +78,14 @@ MAPPING_AUTO = 0
 MAPPING_PLAIN = 1
 MAPPING_PACKED = 2
 
+# places in Options.reserved
+OPT_PERSISTENT_GRID = 0
+OPT_ADJOINT_TAPE_MIB = 1
+OPT_ADJOINT_SWEEP = 2
+ADJOINT_SWEEP_AUTO = 0
+ADJOINT_SWEEP_KERNEL = 1
+ADJOINT_SWEEP_PREPARED = 2
+
 _pd = C.POINTER(C.c_double)
 _pi32 = C.POINTER(C.c_int32)
 _pu32 = C.POINTER(C.c_uint32)

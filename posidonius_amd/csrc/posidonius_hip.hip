@@ -860,7 +860,8 @@ int build_launch(pos_ens *h, const pos_options &o) {
     h->E.wave_count = h->d_wave_count;
     h->E.wave_group = h->d_wave_group;
     h->E.n_waves = nw;
-    h->grid = o.reserved[0] > 0 ? std::min(o.reserved[0], nw) : nw;   // reserved[0]: persistent grid size
+    const int persistent = o.reserved[POS_OPT_PERSISTENT_GRID];
+    h->grid = persistent > 0 ? std::min(persistent, nw) : nw;
     h->opts = o;
     h->opts.steps_per_launch = h->steps_per_launch;
     if (h->graph_exec) { (void)hipGraphExecDestroy(h->graph_exec); h->graph_exec = nullptr; }
@@ -1192,7 +1193,9 @@ constexpr int PREPARED_SETS_PER_CU = 1;
 constexpr size_t COEFFICIENT_BYTES = (size_t)256 << 20;
 void plan_prepared_sweep(pos_ens *h, int seg) {
     pos_ens::Adjoint &A = h->adj;
-    if (h->E.n_waves > PREPARED_SETS_PER_CU * h->n_cus) return;
+    const int sweep = h->opts.reserved[POS_OPT_ADJOINT_SWEEP];
+    if (sweep == POS_ADJOINT_SWEEP_KERNEL) return;
+    if (sweep != POS_ADJOINT_SWEEP_PREPARED && h->E.n_waves > PREPARED_SETS_PER_CU * h->n_cus) return;
     int max_n = 0;
     for (int s = 0; s < h->n_systems; ++s) max_n = std::max(max_n, h->body_offset_dev[s + 1] - h->body_offset_dev[s]);
     const int slots = max_n <= 4 ? 4 : max_n <= 8 ? 8 : 16;
@@ -1277,6 +1280,10 @@ int launch_record(pos_ens *h, const DevEnsemble &E, int len, const TapeRef &tape
 // 256 steps (162 MB) take 3.7 ms to record and 3.0 to differentiate, against 4.5
 // and 5.1 with every segment run a second time.
 constexpr size_t KEPT_TAPE_BYTES = (size_t)1 << 30;
+size_t kept_tape_bytes(const pos_options &o) {
+    const int mib = o.reserved[POS_OPT_ADJOINT_TAPE_MIB];
+    return mib == 0 ? KEPT_TAPE_BYTES : mib > 0 ? (size_t)mib << 20 : 0;
+}
 
 // The buffers, streams and events of a recorded run of n_steps steps.
 int adjoint_allocate(pos_ens *h, int64_t n_steps, int seg) {
@@ -1305,7 +1312,7 @@ int adjoint_allocate(pos_ens *h, int64_t n_steps, int seg) {
     // least a recomputation needs) or a small part of the device's: nothing is
     // recomputed then and the only checkpoint is the final state.
     const size_t all_bytes = tape_bytes * (size_t)n_seg;
-    const bool keep = n_seg <= 2 || all_bytes <= std::min(KEPT_TAPE_BYTES, free_b / 4);
+    const bool keep = n_seg <= 2 || all_bytes <= std::min(kept_tape_bytes(h->opts), free_b / 4);
     A.tapes = (int)std::min<int64_t>(n_seg, keep ? n_seg : 2);
     if ((rc = aalloc((void **)&A.ckpt, keep ? state_bytes : ckpt_bytes)) ||
         (rc = aalloc((void **)&A.tape, tape_bytes * A.tapes)) ||
@@ -1985,6 +1992,7 @@ int32_t pos_tune(pos_ens *h, int32_t probe_steps, pos_options *chosen) {
             o.group_size = g;
             o.steps_per_launch = K;
             o.use_graph = 0;
+            for (int r : {POS_OPT_ADJOINT_TAPE_MIB, POS_OPT_ADJOINT_SWEEP}) o.reserved[r] = h->opts.reserved[r];
             if ((rc = build_launch(h, o))) return rc;
             const int steps = std::max(probe_steps, K);
             if ((rc = pos_step(h, K))) return rc;   // warm-up

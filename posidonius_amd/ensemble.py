@@ -18,13 +18,15 @@ import numpy as np
 from . import abi
 from .case import EnsembleSpec
 
+ADJOINT_SWEEPS = {"auto": abi.ADJOINT_SWEEP_AUTO, "kernel": abi.ADJOINT_SWEEP_KERNEL,
+                  "prepared": abi.ADJOINT_SWEEP_PREPARED}
 MAPPINGS = {"auto": abi.MAPPING_AUTO, "plain": abi.MAPPING_PLAIN, "packed": abi.MAPPING_PACKED}
 
 
 class Ensemble:
     def __init__(self, spec: EnsembleSpec, mapping: str = "packed", group_size: int = 0,
                  steps_per_launch: int = 0, use_graph: bool = False, device: int = 0,
-                 persistent_grid: int = 0):
+                 persistent_grid: int = 0, adjoint_tape_mib: int = 0, adjoint_sweep: str = "auto"):
         self._lib = abi.library()
         self.spec = spec
         self._holder = spec.desc()
@@ -34,7 +36,9 @@ class Ensemble:
         opts.group_size = group_size
         opts.steps_per_launch = steps_per_launch
         opts.use_graph = 1 if use_graph else 0
-        opts.reserved[0] = persistent_grid
+        opts.reserved[abi.OPT_PERSISTENT_GRID] = persistent_grid
+        opts.reserved[abi.OPT_ADJOINT_TAPE_MIB] = adjoint_tape_mib
+        opts.reserved[abi.OPT_ADJOINT_SWEEP] = ADJOINT_SWEEPS[adjoint_sweep]
         h = C.c_void_p()
         abi.check(self._lib.pos_create(self._holder.ref, C.byref(opts), C.byref(h)))
         self._h = h

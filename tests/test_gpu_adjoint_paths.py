@@ -1,0 +1,131 @@
+"""Every way through the adjoint, whatever an ensemble's size would choose: the
+step tapes kept or the segments recomputed, and either reverse sweep, with
+evolving stars, wind, every coordinate type, hosts anywhere and systems that
+stop on their way."""
+import os
+
+import numpy as np
+import pytest
+
+from posidonius_amd import abi, generators as gen
+from posidonius_amd.case import EnsembleSpec
+from tests.test_gpu_adjoint import (BLOCKS, check_against_tangent, coordinate_workloads, directions, evolving_workload,
+                                    wind_workload)
+from tests.test_gpu_adjoint_sweep import RTOL, sizes
+
+pytestmark = pytest.mark.gpu
+
+SWEEPS = ("prepared", "kernel")
+TAPES = {"kept": 0, "recomputed": -1}      # adjoint_tape_mib
+STEPS, SEGMENT = 300, 70                   # five segments, the last one shorter
+
+
+def handle(spec, sweep, tapes):
+    from posidonius_amd.ensemble import Ensemble
+    return Ensemble(spec, mapping="packed", adjoint_sweep=sweep, adjoint_tape_mib=TAPES[tapes])
+
+
+def evolving_in_jacobi(n_systems, steps):
+    spec = evolving_workload(n_systems, steps)
+    spec.system["coordinates"][::2] = abi.COORD_JACOBI
+    return spec
+
+
+WORKLOADS = {"star_3planets": lambda: gen.config4(16), "wind": lambda: wind_workload(16),
+             "evolution": lambda: evolving_workload(16, STEPS), "evolution_jacobi": lambda: evolving_in_jacobi(16, STEPS),
+             "host_moved": lambda: coordinate_workloads()["host_moved"],
+             "all_three_coordinates": lambda: coordinate_workloads()["all_three_coordinates"]}
+
+
+@pytest.mark.parametrize("name", sorted(WORKLOADS))
+def test_each_path_equals_tangent_linear(oracle, name):
+    """Every seed block against every tangent direction to 1e-6 relative, and
+    the same bits whether the tapes were kept or not."""
+    spec = WORKLOADS[name]()
+    d = directions(spec, np.random.default_rng(51))
+    ref, tan = oracle.tangent(spec, STEPS, d, threads=max(1, min(16, os.cpu_count() or 1)))
+    w = np.random.default_rng(52).standard_normal((spec.n_bodies, 3))
+    for sweep in SWEEPS:
+        got = {}
+        for tapes in TAPES:
+            print(f"{name}: {sweep} sweep, tapes {tapes}", flush=True)
+            with handle(spec, sweep, tapes) as ens:
+                ens.adjoint_record(STEPS, SEGMENT)
+                fin = ens.get_state()
+                for k in BLOCKS:
+                    np.testing.assert_array_equal(fin[k], ref[k], err_msg=f"recorded forward run differs in {k}")
+                check_against_tangent(ens, spec, np.random.default_rng(53), d, tan, f"{name} {sweep} {tapes}")
+                got[tapes] = ens.adjoint(position=w, velocity=w, angular_momentum=w)
+                for k, a in ens.get_state().items():
+                    np.testing.assert_array_equal(a, fin[k], err_msg=k)
+        for k, a in got["kept"].items():
+            np.testing.assert_array_equal(a, got["recomputed"][k], err_msg=f"{sweep}: {k}")
+
+
+def stopping(seed):
+    """Sizes and coordinates mixed, hosts anywhere, wind on half of the stars;
+    every fourth system stops on its way (9, 17, 25, ... steps)."""
+    spec = sizes((2, 3, 5, 6, 8), seed, abi.COORD_JACOBI)
+    n = spec.n_systems
+    spec.system["coordinates"][:] = np.arange(n) % 3
+    host = np.zeros(spec.n_bodies, dtype=bool)
+    for b0, b1 in zip(spec.body_offset[:-1], spec.body_offset[1:]):
+        host[b0 + np.argmax(spec.body["mass"][b0:b1])] = True
+    spec.system["effects"][n // 2:] |= abi.EFFECT_WIND
+    spec.body["roles"] = np.where(host, spec.body["roles"] | abi.ROLE_WIND, spec.body["roles"]).astype(spec.body["roles"].dtype)
+    spec.body["wind_k_factor"] = np.where(host, 4e-12, 0.)
+    spec.body["wind_rotation_saturation"] = np.full(spec.n_bodies, 1.7592918860102842)
+    stop = np.where(np.arange(n) % 4 == 1, 2 * np.arange(n) + 7, 1000)
+    spec.system["time_limit"][:] = (stop + 0.5) * spec.system["time_step"]
+    spec.system["historic_snapshot_period"][:] = 3.3 * spec.system["time_step"]
+    return spec
+
+
+@pytest.mark.parametrize("sweep", SWEEPS)
+def test_recomputed_segments_append_no_records(sweep):
+    """Recomputing the segments of a run with snapshots and stopped systems
+    gives the kept run's bits and no records of its own."""
+    spec = stopping(61)
+    steps, segment = 60, 9
+    w = np.random.default_rng(62).standard_normal((spec.n_bodies, 3))
+    got = []
+    for tapes in TAPES:
+        with handle(spec, sweep, tapes) as ens:
+            ens.enable_history(32)
+            ens.adjoint_record(steps, segment)
+            rec = ens.drain_history()
+            grad = [ens.adjoint(position=w, velocity=w, angular_momentum=w) for _ in range(2)]
+            assert len(ens.drain_history()) == 0
+            got.append((grad, rec, ens.get_state()))
+    assert np.any(got[0][2]["current_iteration"] < steps) and len(got[0][1]) > 0
+    with handle(spec, sweep, "kept") as ens:
+        ens.enable_history(32)
+        ens.step(steps)
+        plain, state = ens.drain_history(), ens.get_state()
+    for grad, rec, st in got:
+        for k in plain.dtype.names:
+            np.testing.assert_array_equal(rec[k], plain[k], err_msg=k)
+        for k in state:
+            np.testing.assert_array_equal(st[k], state[k], err_msg=k)
+        for g in grad:
+            for k, a in g.items():
+                assert np.all(np.isfinite(a)), k
+                np.testing.assert_array_equal(a, got[0][0][0][k], err_msg=k)
+
+
+def test_the_two_sweeps_on_evolving_stars():
+    """Evolving stars in heliocentric and Jacobi coordinates among systems of
+    other sizes: the sweeps differ by the roundings of 24 steps (see RTOL)."""
+    steps, segment = 24, 9
+    spec = EnsembleSpec.concat([evolving_in_jacobi(8, steps), sizes((2, 5, 16), 65, abi.COORD_WHDS)])
+    w = np.random.default_rng(66).standard_normal((spec.n_bodies, 3))
+    out = {}
+    for sweep in SWEEPS:
+        with handle(spec, sweep, "kept") as ens:
+            ens.adjoint_record(steps, segment)
+            out[sweep] = ens.adjoint(position=w, velocity=w, angular_momentum=w)
+    for k, a in out["prepared"].items():
+        b = out["kernel"][k]
+        for s in range(spec.n_systems):
+            i = slice(spec.body_offset[s], spec.body_offset[s + 1])
+            assert np.abs(a[i] - b[i]).max() <= RTOL * np.abs(b[i]).max(), (k, s)
