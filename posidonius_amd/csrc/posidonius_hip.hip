@@ -572,6 +572,8 @@ struct pos_ens {
         size_t state_bytes = 0;
         char *final_state = nullptr;       // the last of ckpt
         char *ckpt = nullptr;              // states: segment starts (unless every tape is kept), then the final one
+        // the settings of the recorded run, for the segments recomputed later
+        double *time_limit = nullptr, *hist_period = nullptr, *roche = nullptr;
         // segment tapes, (seg + 1) * TAPE_FIELDS * n_bodies each; segment s uses
         // tape s % tapes, held[] tells whose rows a tape has
         int tapes = 0;
@@ -1321,6 +1323,10 @@ int adjoint_allocate(pos_ens *h, int64_t n_steps, int seg) {
         (rc = aalloc((void **)&A.lx, 3 * nb * sizeof(double))) || (rc = aalloc((void **)&A.lv, 3 * nb * sizeof(double))) ||
         (rc = aalloc((void **)&A.lL, 3 * nb * sizeof(double))) || (rc = aalloc((void **)&A.gs, nb * sizeof(double))) ||
         (rc = aalloc((void **)&A.gk2, nb * sizeof(double))) || (rc = aalloc((void **)&A.gkf, nb * sizeof(double))))
+        return rc;
+    if (!keep && ((rc = aalloc((void **)&A.time_limit, ns * sizeof(double))) ||
+                  (rc = aalloc((void **)&A.hist_period, ns * sizeof(double))) ||
+                  (rc = aalloc((void **)&A.roche, nb * POS_MAX_BODIES * sizeof(double)))))
         return rc;
     plan_prepared_sweep(h, seg);
     HIP_TRY(hipStreamCreateWithFlags(&A.sweep, hipStreamNonBlocking));
@@ -2174,6 +2180,12 @@ int32_t pos_adjoint_record(pos_ens *h, int64_t n_steps, int32_t segment_steps) {
     const size_t state_bytes = A.state_bytes;
     A.held.assign(A.tapes, -1);
     HIP_TRY(hipMemcpyAsync(A.iter0, h->E.iteration, ns * sizeof(long long), hipMemcpyDeviceToDevice, h->stream));
+    if (!keep) {
+        const size_t system_bytes = ns * sizeof(double), roche_bytes = (size_t)h->n_bodies * POS_MAX_BODIES * sizeof(double);
+        HIP_TRY(hipMemcpyAsync(A.time_limit, h->E.time_limit, system_bytes, hipMemcpyDeviceToDevice, h->stream));
+        HIP_TRY(hipMemcpyAsync(A.hist_period, h->E.hist_period, system_bytes, hipMemcpyDeviceToDevice, h->stream));
+        HIP_TRY(hipMemcpyAsync(A.roche, h->E.roche, roche_bytes, hipMemcpyDeviceToDevice, h->stream));
+    }
     for (int64_t s = 0; s < n_seg; ++s) {
         if (!keep && (rc = adjoint_copy_state(h, A.ckpt + (size_t)s * state_bytes, true))) return rc;
         const int64_t len = std::min<int64_t>(seg, n_steps - s * seg);
@@ -2247,9 +2259,16 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
             recomputed = true;
             int r = adjoint_copy_state(h, A.ckpt + (size_t)s * A.state_bytes, false), nl = 0;
             if (r) return r;
-            // the recomputed steps were recorded once already: no historic records
+            // The recomputed steps were recorded once already: no historic
+            // records. What a step reads and a checkpoint does not hold is as it
+            // was then: a lower time limit or larger Roche radii, set since,
+            // would stop systems early and leave older rows on the tape.
+            DevEnsemble Er = without_history(h->E);
+            Er.time_limit = A.time_limit;
+            Er.hist_period = A.hist_period;
+            Er.roche = A.roche;
             const TapeRef tape{A.tape + slot * A.tape_values, nb};
-            if ((r = launch_record(h, without_history(h->E), seg_len(s), tape, &nl))) return r;
+            if ((r = launch_record(h, Er, seg_len(s), tape, &nl))) return r;
             A.held[slot] = s;
         }
         HIP_TRY(hipEventRecord(A.taped_ev[slot & 1], h->stream));

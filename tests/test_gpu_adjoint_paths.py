@@ -129,3 +129,30 @@ def test_the_two_sweeps_on_evolving_stars():
         for s in range(spec.n_systems):
             i = slice(spec.body_offset[s], spec.body_offset[s + 1])
             assert np.abs(a[i] - b[i]).max() <= RTOL * np.abs(b[i]).max(), (k, s)
+
+
+@pytest.mark.parametrize("setting", ["time_limit", "snapshot_period", "roche_radius"])
+@pytest.mark.parametrize("tapes", sorted(TAPES))
+def test_settings_changed_after_the_recording(tapes, setting):
+    """The adjoint is of the run as it was recorded: a time limit, snapshot
+    period or Roche radii set afterwards stay as set but do not enter it."""
+    spec = stopping(67)
+    steps, segment = 60, 9
+    w = np.random.default_rng(68).standard_normal((spec.n_bodies, 3))
+    got = []
+    for change in (False, True):
+        with handle(spec, "kernel", tapes) as ens:
+            ens.adjoint_record(steps, segment)
+            end = ens.get_state()
+            if change and setting == "time_limit":
+                ens.set_time_limit(12.5 * spec.system["time_step"].min())
+            if change and setting == "snapshot_period":
+                ens.set_historic_snapshot_period(1.1 * spec.system["time_step"].max())
+            roche = np.full_like(end["roche_radius"], 1e3) if change and setting == "roche_radius" else end["roche_radius"]
+            ens.set_state({"roche_radius": roche})
+            got.append(ens.adjoint(position=w, velocity=w, angular_momentum=w))
+            after = ens.get_state()
+        for k in end:
+            np.testing.assert_array_equal(after[k], roche if k == "roche_radius" else end[k], err_msg=k)
+    for k in got[0]:
+        np.testing.assert_array_equal(got[1][k], got[0][k], err_msg=k)
