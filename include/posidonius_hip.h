@@ -228,7 +228,7 @@ typedef struct pos_state {
                                          (0 = 1024, negative = none beyond the last two)         */
 #define POS_OPT_ADJOINT_SWEEP 2       /* POS_ADJOINT_SWEEP_*                                     */
 
-#define POS_ADJOINT_SWEEP_AUTO 0      /* by the size of the ensemble                             */
+#define POS_ADJOINT_SWEEP_AUTO 0      /* by the size of the ensemble, see pos_adjoint            */
 #define POS_ADJOINT_SWEEP_KERNEL 1    /* each segment in one kernel, no workspace                */
 #define POS_ADJOINT_SWEEP_PREPARED 2  /* coefficients in parallel, then a chain of products      */
 
@@ -391,7 +391,13 @@ int32_t pos_history_drain(pos_ens *ens, pos_history_record *out, int64_t max_rec
  * recomputed from its checkpoint where its tape was not kept, and leaves the ensemble's state where
  * pos_adjoint_record left it.  Arrays are in input body order, [3*nb] for
  * vectors and [nb] for parameters; NULL seed arrays count as zero and NULL
- * grad arrays are skipped.  Systems that stop early (completion or a fatal
+ * grad arrays are skipped.  There are two reverse sweeps, whose gradients
+ * differ by rounding: the prepared one serves ensembles of up to as many
+ * wavefronts of 64 lanes (a system of N bodies taking the next power of two of
+ * lanes) as the device has compute units, the one-kernel one larger ensembles
+ * and devices without memory for the first one's workspace.
+ * POS_OPT_ADJOINT_SWEEP sets either; under the same sweep a system's gradient
+ * does not depend on mapping, tuning, kept tapes or, prepared, the segments.  Systems that stop early (completion or a fatal
  * status) are differentiated over the steps they executed.
  */
 typedef struct pos_adjoint_seed {

@@ -69,6 +69,7 @@ struct AdjArgs {
     const long long *steps_done;    // [n_systems] steps each system executed in the recorded run
     double *lx, *lv, *lL;           // [3][n_bodies] cotangents: in = after the segment, out = before it
     double *gs, *gk2, *gkf;         // [n_bodies] accumulated parameter gradients
+    double *carry;                  // [CARRY_ROWS][n_bodies], prepared sweep only (see sweep_store)
 };
 
 struct AdjLane {

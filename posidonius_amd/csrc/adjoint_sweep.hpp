@@ -435,9 +435,15 @@ __device__ __forceinline__ void sweep_middle_jacobi(SweepLds &S, SweepLane &A, c
     wsync();
 }
 
-// Lane state of the systems of one wavefront: systems first.., NM slots each.
+// What a stretch hands to the one before it in time: the midpoint solve's last
+// correction and the sums of the lane's parameters, three components each.  The
+// stretches' length then leaves no trace in the result.
+enum { CARRY_WV = 0, CARRY_WL = 3, CARRY_P0 = 6, CARRY_P1 = 9, CARRY_ROWS = 12 };
+
+// Lane state of the systems of one wavefront: systems first.., NM slots each;
+// first: no stretch was swept before.
 template <int NM>
-__device__ __forceinline__ void sweep_load(const AdjArgs &Ar, SweepLds &S, SweepLane &A, int &sys, bool &jacobi) {
+__device__ __forceinline__ void sweep_load(const AdjArgs &Ar, SweepLds &S, SweepLane &A, int &sys, bool &jacobi, bool first) {
     const DevEnsemble &E = Ar.E;
     const int lane = threadIdx.x;
     const int quad = lane >> 2;
@@ -487,13 +493,16 @@ __device__ __forceinline__ void sweep_load(const AdjArgs &Ar, SweepLds &S, Sweep
     A.lx = A.live ? Ar.lx[A.c * nb + A.body] : 0.;
     A.lv = A.live ? Ar.lv[A.c * nb + A.body] : 0.;
     A.lL = A.live ? Ar.lL[A.c * nb + A.body] : 0.;
-    A.wv = A.wL = 0.;
-    A.p0 = A.p1 = 0.;
+    auto carried = [&](int row) { return A.live && !first ? Ar.carry[(size_t)(row + A.c) * nb + A.body] : 0.; };
+    A.wv = carried(CARRY_WV);
+    A.wL = carried(CARRY_WL);
+    A.p0 = carried(CARRY_P0);
+    A.p1 = carried(CARRY_P1);
     wsync();
 }
 
-// The cotangents, and the parameters' gradients added to what is there; a
-// host's are the sums over its pairs.
+// The cotangents, the parameters' gradients so far (a host's are the sums over
+// its pairs) and what the next stretch goes on from.
 template <int NM>
 __device__ __forceinline__ void sweep_store(const AdjArgs &Ar, SweepLds &S, const SweepLane &A) {
     const int nb = Ar.E.n_bodies;
@@ -504,9 +513,14 @@ __device__ __forceinline__ void sweep_store(const AdjArgs &Ar, SweepLds &S, cons
     Ar.lx[A.c * nb + A.body] = A.lx;
     Ar.lv[A.c * nb + A.body] = A.lv;
     Ar.lL[A.c * nb + A.body] = A.lL;
-    if (A.c == 0 && !A.orb) { Ar.gs[A.body] += s0; Ar.gkf[A.body] += s1; }
-    if (A.c == 1 && A.orb) { Ar.gs[A.body] += A.p0; Ar.gkf[A.body] += A.p1; }
-    if (A.c == 2) Ar.gk2[A.body] += A.orb ? A.p1 : s0;
+    auto carry = [&](int row, double x) { Ar.carry[(size_t)(row + A.c) * nb + A.body] = x; };
+    carry(CARRY_WV, A.wv);
+    carry(CARRY_WL, A.wL);
+    carry(CARRY_P0, A.p0);
+    carry(CARRY_P1, A.p1);
+    if (A.c == 0 && !A.orb) { Ar.gs[A.body] = s0; Ar.gkf[A.body] = s1; }
+    if (A.c == 1 && A.orb) { Ar.gs[A.body] = A.p0; Ar.gkf[A.body] = A.p1; }
+    if (A.c == 2) Ar.gk2[A.body] = A.orb ? A.p1 : s0;
 }
 
 // Steps [row0, row0 + len) of a segment and where their coefficients are, as the
@@ -515,6 +529,7 @@ struct Stretch {
     TapeRef T;
     long long seg_start;
     int row0, len;
+    bool first;           // the first to be swept
     Coefficients Cf;
 };
 
@@ -526,7 +541,7 @@ __device__ inline void sweep_stretch(const AdjArgs &Ar, SweepLds &S, const Stret
     SweepLane A;
     int sys;
     bool jacobi;
-    sweep_load<NM>(Ar, S, A, sys, jacobi);
+    sweep_load<NM>(Ar, S, A, sys, jacobi, W.first);
     const long long done = Ar.steps_done[sys] - W.seg_start - W.row0;   // steps of the stretch the system took
     const unsigned long long group = (NM == 16 ? ~0ull : ((1ull << (4 * NM % 64)) - 1) << A.g0);
     // Each part's coefficients are asked for a part or more before their use:

@@ -568,7 +568,7 @@ struct pos_ens {
     struct Adjoint {
         bool recorded = false;
         int64_t n_steps = 0;
-        int seg = 0, n_seg = 0, n_waves = 0;   // what the buffers are for (n_waves: of the launch table)
+        int seg = 0, n_seg = 0;            // what the buffers are for
         size_t state_bytes = 0;
         char *final_state = nullptr;       // the last of ckpt
         char *ckpt = nullptr;              // states: segment starts (unless every tape is kept), then the final one
@@ -589,6 +589,9 @@ struct pos_ens {
         // systems of at most `slots` bodies; none: the sweep in one kernel
         double2 *coef = nullptr;
         int stretch = 0, slots = 0;
+        double *carry = nullptr;           // what the sweep hands from stretch to stretch
+        int *wave_table = nullptr;         // its launch table: first, count and group of `sets` sets
+        int sets = 0;
         std::vector<void *> allocs;
     } adj;
 };
@@ -1182,36 +1185,68 @@ int launch_steps(pos_ens *h, int n_steps, int *launches = nullptr) {
     return POS_OK;
 }
 
+// The sets of systems of the prepared sweep: power-of-two groups of lanes, in
+// device order.  They follow from the ensemble alone, not from the mapping of its
+// steps: a system's gradient is the same under every mapping and after tuning.
+void adjoint_sets(const pos_ens *h, std::vector<int> &first, std::vector<int> &count, std::vector<int> &group) {
+    for (int s = 0; s < h->n_systems;) {
+        const int G = group_lanes(0, h->n_per_sys_dev[s]);
+        int e = s;
+        while (e < h->n_systems && e - s < WAVE / G && group_lanes(0, h->n_per_sys_dev[e]) == G) ++e;
+        first.push_back(s);
+        count.push_back(e - s);
+        group.push_back(G);
+        s = e;
+    }
+}
+
 // The prepared sweep's workspace, if this ensemble is one it serves better: up to
 // one set of systems per CU.  The adjoint of 32 steps in one kernel and
 // prepared, us a step: 128 sets of systems of four bodies 48.1 and 23.1, 256
 // sets 51.1 and 38.9, 384 sets 56.4 and 63.3; of 2 to 12 bodies 118 sets 74.8 and
 // 36.2, 243 sets 79.9 and 66.9, 487 sets 90.5 and 137; of two bodies 128 sets
 // 42.1 and 26.4, 256 sets 44.4 and 46.5; of 16 bodies 256 sets 93.8 and 50.7.
-// The workspace (two halves, one swept while the other is filled) is bounded, a
-// segment is swept by stretches of the steps that fit; without memory for a
-// single one the sweep is the one kernel's.
+// The two sweeps' gradients differ in their last digits, so nothing but the
+// ensemble (and the handle's option) decides.  The workspace (two halves, one
+// swept while the other is filled) is bounded, a segment is swept by stretches of
+// the steps that fit, which leave no trace in the result; only a device without
+// memory for a single step makes the sweep the one kernel's.
 constexpr int PREPARED_SETS_PER_CU = 1;
 constexpr size_t COEFFICIENT_BYTES = (size_t)256 << 20;
-void plan_prepared_sweep(pos_ens *h, int seg) {
+int plan_prepared_sweep(pos_ens *h, int seg) {
     pos_ens::Adjoint &A = h->adj;
     const int sweep = h->opts.reserved[POS_OPT_ADJOINT_SWEEP];
-    if (sweep == POS_ADJOINT_SWEEP_KERNEL) return;
-    if (sweep != POS_ADJOINT_SWEEP_PREPARED && h->E.n_waves > PREPARED_SETS_PER_CU * h->n_cus) return;
-    int max_n = 0;
-    for (int s = 0; s < h->n_systems; ++s) max_n = std::max(max_n, h->body_offset_dev[s + 1] - h->body_offset_dev[s]);
+    if (sweep == POS_ADJOINT_SWEEP_KERNEL) return POS_OK;
+    std::vector<int> table, count, group;
+    adjoint_sets(h, table, count, group);
+    const int sets = (int)table.size();
+    if (sweep != POS_ADJOINT_SWEEP_PREPARED && sets > PREPARED_SETS_PER_CU * h->n_cus) return POS_OK;
+    table.insert(table.end(), count.begin(), count.end());
+    table.insert(table.end(), group.begin(), group.end());
+    const int max_n = *std::max_element(h->n_per_sys_dev.begin(), h->n_per_sys_dev.end());
     const int slots = max_n <= 4 ? 4 : max_n <= 8 ? 8 : 16;
     const size_t step_bytes = (size_t)coefficient_planes(slots) * h->n_bodies * sizeof(double2);
+    const size_t fixed_bytes = CARRY_ROWS * (size_t)h->n_bodies * sizeof(double) + table.size() * sizeof(int);
     size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) { (void)hipGetLastError(); return; }
-    const size_t stretch = std::min<size_t>(seg, std::min(COEFFICIENT_BYTES, free_b / 4) / 2 / step_bytes);
-    if (stretch == 0) return;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) { (void)hipGetLastError(); return POS_OK; }
+    size_t stretch = std::min<size_t>(seg, std::max<size_t>(1, std::min(COEFFICIENT_BYTES, free_b / 4) / 2 / step_bytes));
     void *q = nullptr;
-    if (hipMalloc(&q, 2 * stretch * step_bytes) != hipSuccess) { (void)hipGetLastError(); return; }
+    while (hipMalloc(&q, 2 * stretch * step_bytes + fixed_bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        if (stretch == 1) return POS_OK;
+        stretch = 1;
+    }
     A.allocs.push_back(q);
     A.coef = (double2 *)q;
+    A.carry = (double *)(A.coef + 2 * stretch * step_bytes / sizeof(double2));
+    A.wave_table = (int *)(A.carry + CARRY_ROWS * (size_t)h->n_bodies);
     A.stretch = (int)stretch;
     A.slots = slots;
+    A.sets = sets;
+    int rc;
+    if ((rc = upload(h, A.wave_table, table))) return rc;
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    return POS_OK;
 }
 
 // One stretch's sweep and the next one's preparation, on the adjoint's stream.
@@ -1222,7 +1257,7 @@ int launch_stretch(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo, const Stre
                 : A.slots == 8 ? (general ? adjoint_stretch_kernel<8, true, true> : adjoint_stretch_kernel<8, false, false>)
                                : (general ? adjoint_stretch_kernel<16, true, true> : adjoint_stretch_kernel<16, false, false>);
     const int per_wave = 16 / A.slots;
-    const int blocks = (sweep.len > 0 ? (h->n_systems + per_wave - 1) / per_wave : 0) + 2 * h->E.n_waves * prepare.len;
+    const int blocks = (sweep.len > 0 ? (h->n_systems + per_wave - 1) / per_wave : 0) + 2 * A.sets * prepare.len;
     hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64), 0, A.sweep, Ar, sweep, prepare);
     HIP_TRY(hipGetLastError());
     return POS_OK;
@@ -1239,7 +1274,7 @@ int launch_sweep(pos_ens *h, const AdjArgs &Ar, bool alt, bool evo, Stretch &las
         double2 *const half = A.coef + (size_t)A.stretch * planes * h->n_bodies;
         for (int end = Ar.seg_len, rc; end > 0;) {
             const int len = std::min(A.stretch, end), row0 = end - len;
-            const Stretch next{Ar.T, Ar.seg_start, row0, len,
+            const Stretch next{Ar.T, Ar.seg_start, row0, len, last.len == 0,
                                Coefficients{last.Cf.base == A.coef ? half : A.coef, planes, h->n_bodies}};
             if ((rc = launch_stretch(h, Ar, alt, evo, last, next))) return rc;
             last = next;
@@ -1328,7 +1363,7 @@ int adjoint_allocate(pos_ens *h, int64_t n_steps, int seg) {
                   (rc = aalloc((void **)&A.hist_period, ns * sizeof(double))) ||
                   (rc = aalloc((void **)&A.roche, nb * POS_MAX_BODIES * sizeof(double)))))
         return rc;
-    plan_prepared_sweep(h, seg);
+    if ((rc = plan_prepared_sweep(h, seg))) return rc;
     HIP_TRY(hipStreamCreateWithFlags(&A.sweep, hipStreamNonBlocking));
     for (hipEvent_t *e : {A.taped_ev, A.swept_ev})
         for (int i = 0; i < 2; ++i) HIP_TRY(hipEventCreateWithFlags(&e[i], hipEventDisableTiming));
@@ -1337,7 +1372,6 @@ int adjoint_allocate(pos_ens *h, int64_t n_steps, int seg) {
     A.n_steps = n_steps;
     A.state_bytes = state_bytes;
     A.tape_values = tape_bytes / sizeof(double);
-    A.n_waves = h->E.n_waves;
     return POS_OK;
 }
 
@@ -2171,8 +2205,8 @@ int32_t pos_adjoint_record(pos_ens *h, int64_t n_steps, int32_t segment_steps) {
     const size_t ns = h->n_systems;
     int rc;
     if (A.sweep) HIP_TRY(hipStreamSynchronize(A.sweep));
-    // a run of the same length and mapping finds its buffers here
-    if ((A.n_steps != n_steps || A.seg != seg || A.n_waves != h->E.n_waves) && (rc = adjoint_allocate(h, n_steps, seg))) {
+    // a run of the same length finds its buffers here
+    if ((A.n_steps != n_steps || A.seg != seg) && (rc = adjoint_allocate(h, n_steps, seg))) {
         adjoint_release(h);
         return rc;
     }
@@ -2242,6 +2276,13 @@ int32_t pos_adjoint(pos_ens *h, const pos_adjoint_seed *seed, pos_adjoint_grad *
     Ar.steps_done = A.steps_done;
     Ar.lx = A.lx; Ar.lv = A.lv; Ar.lL = A.lL;
     Ar.gs = A.gs; Ar.gk2 = A.gk2; Ar.gkf = A.gkf;
+    if (A.coef) {
+        Ar.carry = A.carry;
+        Ar.E.n_waves = A.sets;
+        Ar.E.wave_first = A.wave_table;
+        Ar.E.wave_count = A.wave_table + A.sets;
+        Ar.E.wave_group = A.wave_table + 2 * A.sets;
+    }
     // The state is the recorded run's final one from here on, as the sweep finds
     // the bodies' constants in it, whatever the caller did since; where segments
     // are recomputed, again afterwards.

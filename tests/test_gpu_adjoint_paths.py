@@ -113,22 +113,47 @@ def test_recomputed_segments_append_no_records(sweep):
                 np.testing.assert_array_equal(a, got[0][0][0][k], err_msg=k)
 
 
-def test_the_two_sweeps_on_evolving_stars():
-    """Evolving stars in heliocentric and Jacobi coordinates among systems of
-    other sizes: the sweeps differ by the roundings of 24 steps (see RTOL)."""
-    steps, segment = 24, 9
-    spec = EnsembleSpec.concat([evolving_in_jacobi(8, steps), sizes((2, 5, 16), 65, abi.COORD_WHDS)])
+def both_sweeps(spec, steps, segment):
     w = np.random.default_rng(66).standard_normal((spec.n_bodies, 3))
     out = {}
-    for sweep in SWEEPS:
+    for sweep in SWEEPS + ("auto",):
         with handle(spec, sweep, "kept") as ens:
             ens.adjoint_record(steps, segment)
             out[sweep] = ens.adjoint(position=w, velocity=w, angular_momentum=w)
+    return out
+
+
+def sweeps_agree(spec, where):
+    """The sweeps differ by the roundings of 24 steps (see RTOL)."""
+    out = both_sweeps(spec, 24, 9)
     for k, a in out["prepared"].items():
         b = out["kernel"][k]
+        assert np.all(np.isfinite(b))
         for s in range(spec.n_systems):
             i = slice(spec.body_offset[s], spec.body_offset[s + 1])
-            assert np.abs(a[i] - b[i]).max() <= RTOL * np.abs(b[i]).max(), (k, s)
+            assert np.abs(a[i] - b[i]).max() <= RTOL * np.abs(b[i]).max(), (where, k, s)
+
+
+@pytest.mark.parametrize("coords", [abi.COORD_DEMOCRATIC_HELIOCENTRIC, abi.COORD_JACOBI, abi.COORD_WHDS])
+@pytest.mark.parametrize("counts", [(2, 3, 4), (5, 7, 8), (2, 9, 15, 16)], ids=["4_slots", "8_slots", "16_slots"])
+def test_the_two_sweeps(counts, coords):
+    sweeps_agree(sizes(counts, 40, coords), f"sizes {counts} coordinates {coords}")
+
+
+def test_the_two_sweeps_on_evolving_and_stopping_systems():
+    sweeps_agree(EnsembleSpec.concat([evolving_in_jacobi(8, 24), sizes((2, 5, 16), 65, abi.COORD_WHDS)]), "evolving")
+    sweeps_agree(stopping(61), "stopping")
+
+
+@pytest.mark.parametrize("more,sweep", [(0, "prepared"), (1, "kernel")])
+def test_the_sweep_by_size(more, sweep):
+    """Up to one set of systems per CU the prepared sweep, beyond it the kernel."""
+    from tests.test_gpu_teams import edge
+    spec = gen.config2((64 // 16) * edge(1, more), seed=75, n_min=9, n_max=16)
+    out = both_sweeps(spec, 6, 4)
+    for k, a in out["auto"].items():
+        np.testing.assert_array_equal(a, out[sweep][k], err_msg=k)
+    assert any(np.any(out["prepared"][k] != out["kernel"][k]) for k in out["auto"])
 
 
 @pytest.mark.parametrize("setting", ["time_limit", "snapshot_period", "roche_radius"])
@@ -156,3 +181,47 @@ def test_settings_changed_after_the_recording(tapes, setting):
             np.testing.assert_array_equal(after[k], roche if k == "roche_radius" else end[k], err_msg=k)
     for k in got[0]:
         np.testing.assert_array_equal(got[1][k], got[0][k], err_msg=k)
+
+
+def test_gradients_are_the_same_under_every_mapping():
+    """The choice of the sweep follows from the ensemble: the same bits from
+    few sets of systems and from more than one per CU, on each side of the
+    autotuner."""
+    from posidonius_amd.ensemble import Ensemble
+    from tests.test_gpu_teams import edge
+    spec = gen.config2(edge(1, 44), seed=71, n_min=2, n_max=9)
+    w = np.random.default_rng(72).standard_normal((spec.n_bodies, 3))
+    out = {}
+    for name, options in {"pow2": dict(), "exact": dict(group_size=-1), "mixed": dict(group_size=-2),
+                          "set_per_system": dict(group_size=64), "plain": dict(mapping="plain"), "tuned": dict()}.items():
+        with Ensemble(spec, **{"mapping": "packed", **options}) as ens:
+            if name == "tuned":
+                ens.tune(16)
+            ens.adjoint_record(24, 9)
+            out[name] = ens.adjoint(position=w, velocity=w, angular_momentum=w)
+    for name, grad in out.items():
+        for k, a in grad.items():
+            np.testing.assert_array_equal(a, out["pow2"][k], err_msg=f"{name}: {k}")
+
+
+def test_stretches_leave_no_trace():
+    """The prepared sweep walks a segment by as many steps as its workspace
+    holds: the same systems alone (all steps at once) and among enough others
+    to take several stretches, and segments of any length, give the same bits."""
+    steps = 40
+    spec = gen.config2(1024, seed=73, n_min=4, n_max=4)
+    planes, half = 174 + 2 * 4, 128 << 20                   # 16 bytes a body and plane
+    assert 1 < half // (16 * planes * spec.n_bodies) < steps // 2
+    w = np.random.default_rng(74).standard_normal((spec.n_bodies, 3))
+    few = spec.subset(range(16))
+
+    def gradients(s, segment):
+        with handle(s, "prepared", "kept") as ens:
+            ens.adjoint_record(steps, segment)
+            u = w[:s.n_bodies]
+            return ens.adjoint(position=u, velocity=u, angular_momentum=u)
+
+    whole = gradients(few, steps)
+    for s, segment in ((spec, steps), (spec, 17), (few, 1), (few, 17)):
+        for k, a in gradients(s, segment).items():
+            np.testing.assert_array_equal(a[:few.n_bodies], whole[k], err_msg=f"{s.n_systems} systems, segments of {segment}: {k}")
