@@ -397,7 +397,8 @@ int32_t pos_history_drain(pos_ens *ens, pos_history_record *out, int64_t max_rec
  * lanes) as the device has compute units, the one-kernel one larger ensembles
  * and devices without memory for the first one's workspace.
  * POS_OPT_ADJOINT_SWEEP sets either; under the same sweep a system's gradient
- * does not depend on mapping, tuning, kept tapes or, prepared, the segments.  Systems that stop early (completion or a fatal
+ * does not depend on the systems around it, nor on mapping, tuning, kept tapes
+ * or, prepared, the segments.  Systems that stop early (completion or a fatal
  * status) are differentiated over the steps they executed.
  */
 typedef struct pos_adjoint_seed {

@@ -30,7 +30,7 @@
 
 #include "adjoint_kernels.hpp"
 
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)   // see adjoint_kernels.hpp
 
 namespace posdev {
 

@@ -225,3 +225,27 @@ def test_stretches_leave_no_trace():
     for s, segment in ((spec, steps), (spec, 17), (few, 1), (few, 17)):
         for k, a in gradients(s, segment).items():
             np.testing.assert_array_equal(a[:few.n_bodies], whole[k], err_msg=f"{s.n_systems} systems, segments of {segment}: {k}")
+
+
+@pytest.mark.parametrize("sweep", SWEEPS)
+@pytest.mark.parametrize("coords", [abi.COORD_DEMOCRATIC_HELIOCENTRIC, abi.COORD_JACOBI, abi.COORD_WHDS])
+def test_gradients_do_not_depend_on_the_systems_around(sweep, coords):
+    """Each other kind of system (larger, in other coordinates, evolving) brings
+    other kernels; the first systems' gradients keep their bits."""
+    few = sizes((2, 3, 4), 40, coords)
+    w = np.random.default_rng(76).standard_normal((few.n_bodies, 3))
+
+    def gradients(spec):
+        u = np.zeros((spec.n_bodies, 3))
+        u[:few.n_bodies] = w
+        with handle(spec, sweep, "kept") as ens:
+            ens.adjoint_record(24, 9)
+            return ens.adjoint(position=u, velocity=u, angular_momentum=u)
+
+    alone = gradients(few)
+    others = {"8_slots": sizes((6,), 41, abi.COORD_DEMOCRATIC_HELIOCENTRIC), "16_slots": sizes((16,), 42, abi.COORD_JACOBI),
+              "jacobi": sizes((4,), 43, abi.COORD_JACOBI), "whds": sizes((3,), 44, abi.COORD_WHDS),
+              "evolving": evolving_workload(4, 24), "wind": wind_workload(4)}
+    for name, other in others.items():
+        for k, a in gradients(EnsembleSpec.concat([few, other])).items():
+            np.testing.assert_array_equal(a[:few.n_bodies], alone[k], err_msg=f"with {name}: {k}")
