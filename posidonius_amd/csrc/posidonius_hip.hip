@@ -557,7 +557,7 @@ struct pos_ens {
     std::vector<int> coord_dev, evo_dev, host_dev;
     int hist_cap = 0;
     // draining: the system of each device body, sys_perm, each system's first
-    // record, and a bounded stretch of packed records
+    // record, and a bounded stretch of packed records (allocated with the buffer)
     int *d_body_sys = nullptr, *d_sys_perm = nullptr;
     long long *d_hist_start = nullptr;
     pos_history_record *d_hist_out = nullptr;
@@ -2095,7 +2095,14 @@ int32_t pos_history_enable(pos_ens *h, int32_t capacity) {
     std::vector<int> body_sys(h->n_bodies);
     for (int ds = 0; ds < h->n_systems; ++ds)
         for (int b = h->body_offset_dev[ds]; b < h->body_offset_dev[ds + 1]; ++b) body_sys[b] = ds;
-    if ((rc = dalloc(h, &h->d_body_sys, h->n_bodies)) || (rc = dalloc(h, &h->d_sys_perm, h->n_systems)) ||
+    // The packing's own memory is had here too, as much as there is: draining
+    // then succeeds whatever memory is left by that time.
+    h->hist_out_records = (size_t)std::min<int64_t>((int64_t)capacity * h->n_bodies, HISTORY_CHUNK);
+    while ((rc = dalloc(h, &h->d_hist_out, h->hist_out_records)) && h->hist_out_records > 1) {
+        (void)hipGetLastError();
+        h->hist_out_records /= 2;
+    }
+    if (rc || (rc = dalloc(h, &h->d_body_sys, h->n_bodies)) || (rc = dalloc(h, &h->d_sys_perm, h->n_systems)) ||
         (rc = dalloc(h, &h->d_hist_start, h->n_systems)) || (rc = upload(h, h->d_body_sys, body_sys)) ||
         (rc = upload(h, h->d_sys_perm, h->sys_perm)))
         return rc;
@@ -2145,14 +2152,7 @@ int32_t pos_history_drain(pos_ens *h, pos_history_record *out, int64_t max_recor
             start[ds] = k;
             k += (long long)std::min(cnt[ds], h->hist_cap) * h->n_per_sys_dev[ds];
         }
-        const int64_t chunk = std::min<int64_t>(total, HISTORY_CHUNK);
-        if (h->hist_out_records < (size_t)chunk) {
-            if (h->d_hist_out) (void)hipFree(h->d_hist_out);
-            h->d_hist_out = nullptr;
-            h->hist_out_records = 0;
-            HIP_TRY(hipMalloc((void **)&h->d_hist_out, (size_t)chunk * sizeof(pos_history_record)));
-            h->hist_out_records = (size_t)chunk;
-        }
+        const int64_t chunk = (int64_t)h->hist_out_records;
         if ((rc = upload(h, h->d_hist_start, start))) return rc;
         for (int64_t first = 0; first < total; first += chunk) {
             const int64_t last = std::min<int64_t>(total, first + chunk);
@@ -2368,7 +2368,6 @@ void pos_destroy(pos_ens *h) {
     adjoint_release(h);
     for (void *p : h->allocs) (void)hipFree(p);
     if (h->pinned) (void)hipHostFree(h->pinned);
-    if (h->d_hist_out) (void)hipFree(h->d_hist_out);
     for (hipEvent_t e : h->op_ev)
         if (e) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamDestroy(h->stream);

@@ -100,3 +100,21 @@ def test_drained_records_in_input_order(oracle, systems, steps, chunk_edge):
             np.testing.assert_array_equal(rec["velocity"][b0:b0 + n[s]], ref["velocity"][o])
     assert len(first) == counts.sum()
     assert np.all(more["system"] % 3 != 2) and len(more) > 0
+
+
+def test_draining_takes_no_device_memory():
+    """The memory to pack records in comes with the record buffer, so a drain
+    succeeds however full the device is by then."""
+    import torch
+    from posidonius_amd.ensemble import Ensemble
+    torch.cuda.init()
+    spec = gen.config2(3000, seed=31, n_min=7, n_max=7)
+    spec.system["historic_snapshot_period"][:] = 0.9 * spec.system["time_step"]
+    with Ensemble(spec) as ens:
+        ens.enable_history(16)
+        assert 16 * spec.n_bodies > 1 << 18        # more than one stretch of 168-byte records
+        ens.step(14)
+        ens.get_state(("current_time",))
+        before = torch.cuda.mem_get_info()[0]
+        assert len(ens.drain_history()) == 14 * spec.n_bodies
+        assert before - torch.cuda.mem_get_info()[0] < 20 << 20
