@@ -107,8 +107,9 @@ def _host_index(spec: EnsembleSpec) -> np.ndarray:
 
 def _equal(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether two tensors hold the same values, False where that cannot be
-    asked for (while tracing, or of a transformed tensor)."""
-    if torch.compiler.is_compiling():
+    asked for (while tracing, whose result serves other values too, or of a
+    transformed tensor)."""
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
         return False
     try:
         return torch.equal(a, b)

@@ -21,3 +21,19 @@ def test_early_end_is_the_last_iterate(n, ecc, iterations):
     assert torch.equal(got.view(torch.int64), E.view(torch.int64))
     stacked = torch.func.vmap(lambda m: _eccentric_anomaly(e, m, iterations))(torch.stack([M, M]))
     assert torch.equal(stacked[1], E)
+
+
+def test_a_trace_holds_every_iteration():
+    """A traced call serves other inputs than it was traced with: where the
+    iteration ends for those must not be in the trace."""
+    from posidonius_amd import differentiable, generators as gen
+    spec = gen.config2(200, seed=3, n_min=3, n_max=9)
+    a = torch.tensor(spec.elements["a"])
+
+    def state(a, e):
+        return differentiable.state_from_elements(spec, a, e)
+
+    traced = torch.jit.trace(state, (a, torch.full_like(a, 0.01)), check_trace=False)
+    e = torch.full_like(a, 0.9999)
+    for got, want in zip(traced(a, e), state(a, e)):
+        assert torch.equal(got, want)
