@@ -173,36 +173,30 @@ struct WaveLds {
     __device__ __forceinline__ double k2_of(const DevEnsemble &, int lane, int) const { return k2[lane]; }
 };
 
-// Every kernel that uses the exchange area runs one wavefront per workgroup
-// (__launch_bounds__(64)), so the lanes that publish and the lanes that read
-// a value are in the same wavefront.  The LDS executes the operations of one
-// wavefront in the order they are issued, so a read issued after a write sees
-// it: ordering the two at wavefront scope is enough, which costs no wait
-// (a workgroup-scope barrier would wait for every outstanding LDS write).
-#ifndef POS_WSYNC_WORKGROUP
-#define POS_WSYNC_WORKGROUP 0
-#endif
+// Orders the exchanges between the lanes of one wavefront.  The LDS executes
+// the operations of a wavefront in the order they are issued, so a read issued
+// after a write sees it: ordering the two at wavefront scope is enough, which
+// costs no wait (a workgroup-scope barrier would wait for every outstanding LDS
+// write).  It is no barrier: the wavefronts of a team call it in code of their own
+// role, on rows that no other one touches at the time.
 __device__ __forceinline__ void wsync() {
-#if POS_WSYNC_WORKGROUP
-    __syncthreads();
-#else
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-#endif
 }
 
-// The lane group of `lane` in wave `wave`: its device system, first lane and
-// this lane's index in it.  A lane past the wave's groups gets gvalid =
-// false, the wave's first system and its own lane as group start (so that
-// every LDS index it forms stays inside the wave's columns).
-// Meeting point of the wavefronts of a team.
+// Meeting point of the wavefronts of a team; it orders rows that one writes and
+// others read.
 __device__ __forceinline__ void team_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// The lane group of `lane` in wave `wave`: its device system, first lane and
+// this lane's index in it.  A lane past the wave's groups gets gvalid =
+// false, the wave's first system and its own lane as group start (so that
+// every LDS index it forms stays inside the wave's columns).
 struct LaneGroup {
     int sys, gbase, k;
     bool gvalid;
