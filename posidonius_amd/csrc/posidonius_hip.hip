@@ -82,11 +82,11 @@ __device__ inline void load_lane(const DevEnsemble &E, WaveLds &lds, Lane &B, in
         if ((f & F_RF) && (roles & POS_ROLE_FLAT_ORBITING)) f |= F_RF_ROLE;
         if ((f & F_GR) && (roles & POS_ROLE_GR_ORBITING)) f |= F_GR_ROLE;
     }
-    if constexpr ((V & VAR_FAST) != 0) {   // the launch holds only systems of the fixed effect set
+    if constexpr ((V & VAR_FAST) != 0) {   // the fixed effect set's operators, whatever their coordinates
         const bool orb = valid && k != B.host;   // every other body has every orbiting role there
         f = (valid ? F_VALID : 0u) | ((valid && k == B.host) ? F_HOST : 0u) | F_TIDES | F_RF | F_GR | F_SPIN |
             (orb ? (F_TIDES_ROLE | F_RF_ROLE | F_GR_ROLE) : 0u);
-        B.coord = (V & VAR_JACOBI) ? POS_COORD_JACOBI : POS_COORD_DEMOCRATIC_HELIOCENTRIC;
+        B.coord = POS_COORD_DEMOCRATIC_HELIOCENTRIC;
     }
     B.flags = f;
     B.dt = E.dt[s];
@@ -1428,9 +1428,8 @@ int launch_effects(pos_ens *h, double *d_a, double *d_l) {
             case 4: hipLaunchKernelGGL(effects_kernel<4>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
             case 5: hipLaunchKernelGGL(effects_kernel<5>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
             case 6: hipLaunchKernelGGL(effects_kernel<6>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
-            case 8: case 40:   // the effects do not depend on the coordinates
+            case 8: case 24: case 40:   // the effects do not depend on the coordinates
                 hipLaunchKernelGGL(effects_kernel<8>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
-            case 24: hipLaunchKernelGGL(effects_kernel<24>, g, dim3(64), 0, h->stream, h->E, d_a, d_l, w0, w1); break;
             default: return fail(POS_E_INVALID, "internal error: unknown kernel variant");
         }
         HIP_TRY(hipGetLastError());

@@ -129,7 +129,7 @@ def _eccentric_anomaly(e, M, iterations):
     for k in range(1, iterations + 1):
         E2, E1 = E1, E
         E = E - (E - e * torch.sin(E) - M) / (1.0 - e * torch.cos(E))
-        if k % 8 == 0 and k >= 2 and _equal(E, E2):
+        if k % 8 == 0 and _equal(E, E2):
             return E if (iterations - k) % 2 == 0 else E1
     return E
 
