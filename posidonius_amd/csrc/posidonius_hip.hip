@@ -539,8 +539,10 @@ struct pos_ens {
     double *d_op_a = nullptr, *d_op_l = nullptr;   // operator outputs, [3][n_bodies]
     uint32_t *d_op_st = nullptr;                    // operator status, [n_systems]
     double *d_unperm = nullptr;                     // per-body field in caller order, [n_bodies][3]
-    int *d_body_perm = nullptr;                     // body_perm on the device
-    int *d_body_inv = nullptr, *d_sys_inv = nullptr;   // device index of each caller body / system
+    // on the device, one after the other: body_perm, the device index of each
+    // caller body, that of each caller system
+    int *d_body_perm = nullptr, *d_body_inv = nullptr, *d_sys_inv = nullptr;
+    std::vector<int> index_tables;
     char *pinned = nullptr;                         // small read-backs land here
     size_t pinned_bytes = 0;
     int steps_per_launch = 1;
@@ -627,10 +629,17 @@ template <class T> int download(pos_ens *h, std::vector<T> &dst, const T *src, s
 int body_staging(pos_ens *h) {
     int rc;
     if (!h->d_unperm) {
-        const int nb = h->n_bodies;
-        if ((rc = dalloc(h, &h->d_unperm, 3 * (size_t)nb)) || (rc = dalloc(h, &h->d_body_perm, nb)) ||
-            (rc = upload(h, h->d_body_perm, h->body_perm)))
+        const int nb = h->n_bodies, ns = h->n_systems;
+        std::vector<int> &t = h->index_tables;
+        t = h->body_perm;
+        t.resize(2 * (size_t)nb + ns);
+        for (int db = 0; db < nb; ++db) t[nb + h->body_perm[db]] = db;
+        for (int ds = 0; ds < ns; ++ds) t[2 * (size_t)nb + h->sys_perm[ds]] = ds;
+        if ((rc = dalloc(h, &h->d_unperm, 3 * (size_t)nb)) || (rc = dalloc(h, &h->d_body_perm, t.size())) ||
+            (rc = upload(h, h->d_body_perm, t)))
             return rc;
+        h->d_body_inv = h->d_body_perm + nb;
+        h->d_sys_inv = h->d_body_inv + nb;
     }
     return POS_OK;
 }
@@ -1677,15 +1686,6 @@ int32_t pos_create(const pos_ensemble_desc *d, const pos_options *opts, pos_ens 
     {
         double *scratch_ptr = nullptr;
         if ((rc = noalloc_scratch(h->device, &scratch_ptr)) || (rc = body_staging(h))) { pos_destroy(h); return rc; }
-        std::vector<int> body_inv(nb), sys_inv(ns);
-        for (int db = 0; db < nb; ++db) body_inv[h->body_perm[db]] = db;
-        for (int ds = 0; ds < ns; ++ds) sys_inv[h->sys_perm[ds]] = ds;
-        if ((rc = dalloc(h, &h->d_body_inv, nb)) || (rc = dalloc(h, &h->d_sys_inv, ns)) ||
-            (rc = upload(h, h->d_body_inv, body_inv)) || (rc = upload(h, h->d_sys_inv, sys_inv))) {
-            pos_destroy(h);
-            return rc;
-        }
-        if (hipStreamSynchronize(h->stream) != hipSuccess) { pos_destroy(h); return fail(POS_E_HIP, "synchronize failed"); }
     }
     h->eff_dev = eff;
     h->roles_dev = roles;
