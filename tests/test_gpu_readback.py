@@ -118,3 +118,19 @@ def test_draining_takes_no_device_memory():
         before = torch.cuda.mem_get_info()[0]
         assert len(ens.drain_history()) == 14 * spec.n_bodies
         assert before - torch.cuda.mem_get_info()[0] < 20 << 20
+
+
+def test_fields_that_do_not_fit_are_read_one_by_one():
+    """Four fields of three doubles fill the packed buffer up to less than the
+    smallest field: every other one, per system and per body, integers and rows,
+    takes the path that also serves where no pinned memory can be had."""
+    from posidonius_amd.ensemble import Ensemble
+    spec = gen.config2(9500, seed=12, n_min=2, n_max=3)
+    spec = spec.subset(range(int(np.searchsorted(spec.body_offset, LIMIT // 96, side="right")) - 1))
+    left = LIMIT - 96 * spec.n_bodies
+    assert 0 <= left < 4 * spec.n_systems
+    with Ensemble(spec, group_size=-2) as ens:
+        ens.step(2)
+        whole = ens.get_state()
+        for k, a in whole.items():
+            np.testing.assert_array_equal(a, ens.get_state((k,))[k], err_msg=k)
