@@ -7,8 +7,8 @@
 // writes the coefficients of every product of a stretch of steps;
 // sweep_stretch walks the stretch backwards and only multiplies.  In place of
 // 40 us a step (one wavefront a SIMD at most, 11,000 vector instructions in
-// one chain) the preparation, spread over the chip, takes 4.6 us and the sweep
-// 5.4 us, bound by the latency of its 20 exchanges through LDS; both at once 7.4
+// one chain) the preparation, spread over the chip, takes 4.8 us and the sweep
+// 6.5 us, bound by the latency of its 20 exchanges through LDS; both at once 7.4
 // us (1,024 systems of four bodies).  An ensemble that fills the chip is bound by
 // its instructions, not by their chain, and would be by the coefficients'
 // traffic (3 KB a body and step each way): there adjoint_segment_kernel, which

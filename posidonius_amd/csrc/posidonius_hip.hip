@@ -302,8 +302,9 @@ __global__ __launch_bounds__(64) void adjoint_segment_kernel(AdjArgs Ar) {
 // each), and the coefficients of the next one by the others, one wavefront per set
 // of systems, step and part of the step.  Either may be empty.  One launch of
 // both keeps the few long wavefronts of the sweep from waiting for SIMDs that the
-// many of the preparation hold: 1,024 systems of four bodies, 10 steps: 79 us,
-// against 58 and 49 us one after the other and 97 in two streams.  ALT, EVO: see
+// many of the preparation hold: 1,024 systems of four bodies, 11 steps: 81 us,
+// where the preparation alone takes 52 and the sweep 6.5 a step; in two streams
+// the sweep took 1.7 times as long beside the preparation.  ALT, EVO: see
 // adjoint_segment_kernel.
 template <int NM, bool ALT, bool EVO>
 __global__ __launch_bounds__(64) void adjoint_stretch_kernel(AdjArgs Ar, Stretch sweep, Stretch prepare) {
@@ -672,7 +673,9 @@ struct ReadRequest {
 // field by field against packed: 0.7 KiB 143 / 25 us, 0.5 MiB 166 / 52,
 // 2 MiB 240 / 135, 4 MiB 425 / 305, 8 MiB 755 / 615. The limit keeps a handle's
 // first call cheap: pinned memory costs about 0.7 ms per MiB unless the runtime
-// has a freed block of the size.
+// has a freed block of the size. The six fields of 5,000 systems (2 MiB), first
+// call of the process 314 us field by field and 1,185 packed, of a later handle
+// 288 and 253; of 1,000 systems 398 and 389, then 181 and 89.
 constexpr size_t SMALL_READ_BYTES = 2 << 20;
 
 // Records packed at once when draining historic snapshots (40 MiB).
@@ -1148,6 +1151,8 @@ template <int V> void launch_steps_variant(pos_ens *h, int grid, int n_steps, in
 // 1 / 2 / 4: 23.4 / 16.2 / 15.1 us at 250 entries, 26.0 / 21.0 / 18.9 at 500,
 // 25.9 / 21.5 / 30.1 at 600, 27.0 / 24.1 / 36.0 at 1,000 and
 // 35.4 / 34.6 / 45.4, then 37.4 / 42.6 / 52.4 at 1,150 and 1,500.
+// The same limits serve the largest systems: of 16 bodies 26 us at 250 entries
+// (teams of 4), 32 at 500, 35 at 520 and 41 at 1,000 (of 2), 55 at 1,040 (of 1).
 int team_size(const pos_ens *h, int waves) {
     return waves <= 2 * h->n_cus ? 4 : waves <= 4 * h->n_cus ? 2 : 1;
 }
@@ -1210,11 +1215,14 @@ void adjoint_sets(const pos_ens *h, std::vector<int> &first, std::vector<int> &c
 }
 
 // The prepared sweep's workspace, if this ensemble is one it serves better: up to
-// one set of systems per CU.  The adjoint of 32 steps in one kernel and
-// prepared, us a step: 128 sets of systems of four bodies 48.1 and 23.1, 256
-// sets 51.1 and 38.9, 384 sets 56.4 and 63.3; of 2 to 12 bodies 118 sets 74.8 and
-// 36.2, 243 sets 79.9 and 66.9, 487 sets 90.5 and 137; of two bodies 128 sets
-// 42.1 and 26.4, 256 sets 44.4 and 46.5; of 16 bodies 256 sets 93.8 and 50.7.
+// one set of systems per CU.  A whole pos_adjoint of 32 steps in one kernel and
+// prepared, us a step: 128 sets of systems of two bodies 43.2 and 25.4, 256 sets
+// 44.3 and 44.6, 384 sets 48.0 and 75.2; of four bodies 46.9 and 22.4, 51.2 and
+// 39.1, 54.9 and 63.7; of eight 60.5 and 23.7, 64.7 and 42.7, 69.6 and 69.2; of
+// 16 87.0 and 28.1, 92.2 and 48.8, 97.1 and 80.0; of 2 to 12 bodies 148 sets 72.8
+// and 31.0, 305 sets 77.2 and 58.6, 616 sets 85.4 and 120.  The line is drawn
+// where the smallest systems are even; large ones would gain up to 1.5 times as
+// many sets.
 // The two sweeps' gradients differ in their last digits, so nothing but the
 // ensemble (and the handle's option) decides.  The workspace (two halves, one
 // swept while the other is filled) is bounded, a segment is swept by stretches of
@@ -1323,8 +1331,8 @@ int launch_record(pos_ens *h, const DevEnsemble &E, int len, const TapeRef &tape
 }
 
 // The tapes of a whole run are kept up to this: 1,024 systems of four bodies and
-// 256 steps (162 MB) take 3.7 ms to record and 3.0 to differentiate, against 4.5
-// and 5.1 with every segment run a second time.
+// 256 steps (162 MB) take 3.7 ms to record and 2.1 to differentiate, against 3.6
+// and 3.6 with the last two segments' tapes only.
 constexpr size_t KEPT_TAPE_BYTES = (size_t)1 << 30;
 size_t kept_tape_bytes(const pos_options &o) {
     const int mib = o.reserved[POS_OPT_ADJOINT_TAPE_MIB];

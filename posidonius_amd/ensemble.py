@@ -147,8 +147,9 @@ class Ensemble:
 
     # -- discrete adjoint -----------------------------------------------------
     def adjoint_record(self, n_steps: int, segment_steps: int = 0):
-        """Advance n_steps like ``step`` and keep a checkpoint every
-        ``segment_steps`` steps (0 = 1000) for ``adjoint``."""
+        """Advance n_steps like ``step`` in segments of ``segment_steps`` steps
+        (0 = 1000), keeping their step tapes, or of a long run checkpoints, for
+        ``adjoint``."""
         abi.check(self._lib.pos_adjoint_record(self._h, C.c_int64(int(n_steps)), int(segment_steps)))
 
     def adjoint(self, position=None, velocity=None, angular_momentum=None) -> Dict[str, np.ndarray]:
