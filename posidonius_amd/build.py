@@ -12,14 +12,18 @@
 * ``-mllvm -amdgpu-sched-strategy=iterative-maxocc``: the machine scheduler
   variant that measured fastest for the step kernel (3.15e8 vs 3.01e8
   system-steps/s with the default strategy on the 65,536-system ensemble).
-  Scheduling reorders instructions only; results are bitwise unchanged.
+  Scheduling reorders instructions only; results are bitwise unchanged;
+* ``-save-temps=obj``: the device listing is kept for `partial_spills`.
 """
 from __future__ import annotations
 
+import glob
 import os
+import re
 import shutil
 import subprocess
 import sys
+import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 SRC = os.path.join(HERE, "csrc", "posidonius_hip.hip")
@@ -37,18 +41,65 @@ def hipcc() -> str:
     raise RuntimeError("hipcc not found")
 
 
+def partial_spills(listing: str) -> list[str]:
+    """Vector registers saved or copied where a divergent branch has joined but
+    its lanes are still switched off, as "kernel label: instruction".
+
+    The register allocator of ROCm 7.2 can put a spill at the top of a join
+    block, before the ``s_or_b64 exec, exec`` that restores the lanes that
+    skipped the branch: those lanes never store the value and later reload what
+    the slot held.  (It did for the number of the lane's system at
+    ``act && (...)`` in whfast_fixed_kernel with one wavefront a set: a system
+    stopped before the launch stored its time over another's, or out of range.)
+    Nothing in the source is wrong then, so the listing is looked through: a
+    label that an ``s_cbranch_execz`` jumps to, then vector instructions before
+    the restore.  A region that two branches leave early may also end so, but
+    after arithmetic of its own, which a join has none of.
+    """
+    found = []
+    for m in re.finditer(r"^(_Z\w+):.*?$(.*?)^\.Lfunc_end", listing, re.M | re.S):
+        joins = set(re.findall(r"s_cbranch_execz (\.LBB\w+)", m[2]))
+        label, early = None, []
+        for line in m[2].splitlines():
+            code = line.split(";")[0].strip()
+            if q := re.match(r"(\.LBB\w+):", line):
+                label, early = (q[1] if q[1] in joins else None), []
+            elif not label or not code:
+                continue
+            elif re.match(r"s_or_b64 exec, exec", code):
+                found += [f"{m[1]} {label}: {e}" for e in early]
+                label = None
+            elif re.match(r"s_c?branch|s_endpgm|s_\w+ exec\b|s_\w+_saveexec", code):
+                label = None
+            elif re.match(r"scratch_|v_accvgpr_|v_mov_b(32|64)\w* [va]\S+, [va]", code):
+                early.append(line.strip())
+            elif re.match(r"v_(?!readlane|writelane|readfirstlane)|global_|flat_|ds_|buffer_", code):
+                label = None
+    return found
+
+
 def build_library(verbose: bool = False, extra_flags=None) -> str:
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-O3", "-std=c++17", "-fPIC", "-shared",
            "-ffp-contract=off", "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
            "-mllvm", "-amdgpu-sched-strategy=iterative-maxocc",
            "-Wall", "-Wno-unused-function",
-           "-I", os.path.join(os.path.dirname(HERE), "include"),
-           SRC, "-o", OUT + ".tmp"]
+           "-I", os.path.join(os.path.dirname(HERE), "include"), "-save-temps=obj", SRC]
     if extra_flags:
         cmd[1:1] = list(extra_flags)
-    if verbose:
-        print(" ".join(cmd), flush=True)
-    subprocess.run(cmd, check=True)
+    with tempfile.TemporaryDirectory() as temps:
+        built = os.path.join(temps, os.path.basename(OUT))
+        cmd += ["-o", built]
+        if verbose:
+            print(" ".join(cmd), flush=True)
+        subprocess.run(cmd, check=True)
+        listings = glob.glob(os.path.join(temps, f"*{ARCH}*.s"))
+        if not listings:
+            raise RuntimeError("no device listing in " + temps)
+        for path in listings:
+            with open(path) as f:
+                if found := partial_spills(f.read()):
+                    raise RuntimeError("registers spilled under a partial mask:\n" + "\n".join(found))
+        shutil.copy(built, OUT + ".tmp")
     os.replace(OUT + ".tmp", OUT)
     return OUT
 

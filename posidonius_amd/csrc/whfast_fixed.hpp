@@ -1260,11 +1260,14 @@ __device__ __forceinline__ void fixed_run(const DevEnsemble &E, FixedLds<M, (V &
     // start of the step; whether the system takes the step is known to their
     // owner only after the barrier, a stopped system keeps those of its last
     // evaluation), and which systems go on and record a snapshot
-    // (whfast.rs:239-256).
+    // (whfast.rs:239-256).  `snap` takes no branch: with `&&` the compiler saved
+    // B.sys inside the branch, for the lanes of systems that go on alone, and
+    // fixed_store then wrote a stopped system's time over another's (build.py's
+    // partial_spills).
     auto publish = [&](bool velocities) {
         if constexpr (W::OWN_V) {
             act = !(B.status & STOPPED);
-            snap = act && (B.last_hist < 0. || B.last_hist + B.hist_period <= B.t);
+            snap = act & ((B.last_hist < 0.) | (B.last_hist + B.hist_period <= B.t));
             if constexpr (M > 1) {
                 const unsigned long long live = __ballot(act), taken = __ballot(snap);
                 if (lane == 0) { lds.team.live = live; lds.team.snap = taken; }

@@ -83,3 +83,31 @@ def test_adjoint_does_not_depend_on_the_team_size(per_cu, more):
     for a, b in zip(out[0], out[1]):
         for k in b:
             np.testing.assert_array_equal(a[k][:few.n_bodies], b[k], err_msg=k)
+
+
+@pytest.mark.parametrize("coords,gr", [(abi.COORD_DEMOCRATIC_HELIOCENTRIC, abi.GR_KIDDER1995),
+                                       (abi.COORD_WHDS, abi.GR_KIDDER1995),
+                                       (abi.COORD_DEMOCRATIC_HELIOCENTRIC, abi.GR_NEWHALL1983)],
+                         ids=["kidder", "whds", "newhall"])
+@pytest.mark.parametrize("per_cu", [0, 2, 4])
+def test_a_team_serves_set_after_set(per_cu, coords, gr):
+    """With fewer workgroups than sets of systems, a team takes one set after
+    another, some of systems that had stopped before the launch, in the same LDS
+    and scratch memory: the bits of a workgroup per set."""
+    from posidonius_amd.ensemble import Ensemble
+    spec = ensemble(edge(per_cu, 20), coords, 73)
+    spec.system["gr_implementation"][:] = gr
+    out = []
+    for grid in (0, 7):
+        with Ensemble(spec, mapping="packed", group_size=64, steps_per_launch=4, persistent_grid=grid) as ens:
+            ens.enable_history(16)
+            ens.step(9)
+            part = [ens.get_state(), ens.drain_history()]
+            if gr == abi.GR_KIDDER1995:
+                ens.adjoint_record(5, 2)
+                w = np.ones((spec.n_bodies, 3))
+                part += [ens.adjoint(position=w, velocity=w, angular_momentum=w), ens.get_state()]
+            out.append(part)
+    for a, b in zip(*out):
+        for k in (a if isinstance(a, dict) else a.dtype.names):
+            np.testing.assert_array_equal(a[k], b[k], err_msg=k)
