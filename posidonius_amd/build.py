@@ -92,7 +92,7 @@ def build_library(verbose: bool = False, extra_flags=None) -> str:
         if verbose:
             print(" ".join(cmd), flush=True)
         subprocess.run(cmd, check=True)
-        listings = glob.glob(os.path.join(temps, f"*{ARCH}*.s"))
+        listings = glob.glob(os.path.join(temps, "*amdgcn*.s"))
         if not listings:
             raise RuntimeError("no device listing in " + temps)
         for path in listings:
